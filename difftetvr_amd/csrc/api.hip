@@ -220,6 +220,7 @@ struct dtv_view {
     bool sub_tiles = false;         // the last render binned tiles larger than 8x8
     bool queued = false;            // the last render took its tiles from a work queue (the adjoint does too)
     bool cost_ordered = true;       // the last render launched its tiles heaviest first
+    int edge = 8;                   // pixels per side a wave of the last render took (8: a tile, less: a part of one)
     int64_t planned_cap = 0;  // > 0: planned (synchronisation-free) rendering with this record capacity
     // state of the last render
     bool rendered = false;
@@ -295,6 +296,19 @@ bool make_uniforms(const dtv_camera& camera, const dtv_render_params& params, Vi
     U.depth_axis[2] = -camera.view[10];
     U.linear_depth = params.segment_length == DTV_SEGMENT_LINEAR_DEPTH ? 1 : 0;
     return true;
+}
+
+// Pixels per side that a wave of the tile renderer takes, by the number of 8x8 tiles: the GPU's 1,024 SIMDs hold
+// three such waves each, and below that the deepest tile's wave decides the time.  Measured on a step (forward,
+// loss, adjoint) of cube grids with waves of 8x8 / 4x4 / 2x2 pixels, us: 96 tiles 745 / 342 / 247, 256 tiles
+// 1315 / 549 / 379, 625 tiles 2361 / 962 / 842, 1,024 tiles 1193 / 599 / 625, 2,304 tiles 1718 / 1071 / 1367,
+// 4,096 tiles 2264 / 1862 / 2760, 5,000 tiles 3750 / 3054 / 3797, 9,216 tiles 2660 / 3232 / 5478.  (A batch's
+// records cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)
+int wave_edge(const dtv_render_params& prm, int64_t tiles) {
+    if (prm.renderer != DTV_RENDERER_TILE || prm.tile_launch != DTV_TILE_LAUNCH_GRID ||
+        (prm.tile_size != 0 && prm.tile_size != 8) || (prm.segments_per_pass != 0 && prm.segments_per_pass != 128))
+        return 8;
+    return tiles <= 768 ? 2 : tiles <= 5120 ? 4 : 8;
 }
 
 // Binning, sort and forward render of a batch (one host synchronisation, after the record count).
@@ -483,7 +497,8 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     DTV_HIP(view->ranges.ensure(sizeof(uint2) * tiles));
     DTV_HIP(view->tile_frags.ensure(sizeof(uint32_t) * subtiles));
     DTV_HIP(view->tile_order.ensure(2 * sizeof(uint32_t) * subtiles));
-    view->cost_ordered = params->tile_order == 0;
+    const int edge = wave_edge(*params, tiles);
+    view->cost_ordered = params->tile_order == 0 && edge == 8;
     // forward launch order: tiles by record count, heaviest first
     const uint32_t* fwd_order = view->cost_ordered ? view->tile_order.as<uint32_t>() : nullptr;
     view->mark(DTV_STAGE_RANGES, 0, s);
@@ -519,7 +534,8 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     else
         launch_render_forward(dI, n, subtiles, fwd_order, view->sorted_recs(), view->ranges.as<uint2>(),
                               view->pixel_state(), kinds, s, spp, tile != 8,
-                              params->tile_launch == DTV_TILE_LAUNCH_QUEUE ? view->tile_queue() : nullptr);
+                              params->tile_launch == DTV_TILE_LAUNCH_QUEUE ? view->tile_queue() : nullptr, edge);
+    view->edge = edge;
     view->mark(DTV_STAGE_FORWARD, 1, s);
     DTV_HIP(hipGetLastError());
     view->colour_kinds = kinds;
@@ -651,7 +667,7 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         launch_render_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n,
                               view->total_subtiles, adj_order, view->sorted_recs(), view->ranges.as<uint2>(), ps,
                               use_abs_grad ? 1 : 0, adjoint_mode, view->colour_kinds, s, view->sub_tiles,
-                              view->queued ? view->tile_queue() : nullptr);
+                              view->queued ? view->tile_queue() : nullptr, view->edge);
     }
     for (const Fold& fo : folds) launch_fold_vertex_grads(fo.acc, fo.V, fo.grad_pos, fo.grad_col, s);
     view->mark(DTV_STAGE_ADJOINT, 1, s);
@@ -832,7 +848,8 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
     uint32_t* counts = reinterpret_cast<uint32_t*>(base + o_counts);
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + o_hist);
     uint2* ranges = reinterpret_cast<uint2*>(base + o_ranges);
-    uint32_t* order = params->tile_order == 0 ? reinterpret_cast<uint32_t*>(base + o_order) : nullptr;
+    const int edge = wave_edge(*params, tiles);
+    uint32_t* order = params->tile_order == 0 && edge == 8 ? reinterpret_cast<uint32_t*>(base + o_order) : nullptr;
     uint4* recs = reinterpret_cast<uint4*>(base + o_recs);
     // the item reaches the device as a kernel argument: no host staging
     hipLaunchKernelGGL(k_store_item, dim3(1), dim3(1), 0, s, B, dI);
@@ -858,7 +875,7 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
     ps.ckpt_n = nullptr;
     ps.counters = nullptr;
     ps.tile_frags = reinterpret_cast<uint32_t*>(base + o_tfrags);
-    launch_render_forward(dI, 1, tiles, order, recs, ranges, ps, colour_kind(m), s);
+    launch_render_forward(dI, 1, tiles, order, recs, ranges, ps, colour_kind(m), s, 128, false, nullptr, edge);
     if (out_overflow) hipLaunchKernelGGL(k_copy_flag, dim3(1), dim3(1), 0, s, overflow, out_overflow);
     DTV_HIP(hipGetLastError());
     return DTV_OK;

@@ -89,13 +89,16 @@ constexpr uint32_t kColoursPerVertex = 1, kColoursPerCell = 2;
 // sub: the batch bins tiles larger than 8x8 (the kernels then test coverage per 8x8 sub-tile).
 // queue: NULL launches one workgroup per tile; else a persistent grid (the workgroups the GPU holds at once)
 // takes the tiles in launch order from this device counter, which each launch zeroes first.
+// edge: 8, or 4 or 2 for (8 / edge)^2 waves per tile, each rendering edge x edge pixels (128 fragments per round,
+// 8x8 binning tiles, no queue; order is not used).
 void launch_render_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
                            const uint4* recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
-                           hipStream_t s, int round = 128, bool sub = false, uint32_t* queue = nullptr);
+                           hipStream_t s, int round = 128, bool sub = false, uint32_t* queue = nullptr,
+                           int edge = 8);
 void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                            const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps, int use_abs,
                            int mode, uint32_t colour_kinds, hipStream_t s, bool sub = false,
-                           uint32_t* queue = nullptr);
+                           uint32_t* queue = nullptr, int edge = 8);
 // Adds the tile renderer adjoint's interleaved accumulator rows acc [V][8] into grad_pos [V][3] and, unless
 // NULL, grad_col [V][4].
 void launch_fold_vertex_grads(const float* acc, int64_t V, float* grad_pos, float* grad_col, hipStream_t s);

@@ -31,6 +31,12 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
     return v;
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, d, 64));
+    return v;
+}
+
 // Sum across the wave, result valid in every lane.  DPP row operations within 16-lane rows, then
 // row broadcasts; all lanes must be active.
 __device__ __forceinline__ float wave_sum(float v) {

@@ -59,12 +59,15 @@ __device__ __forceinline__ float3_ lane_ray(float3_ mine, int pl) {
 // kCell: renders the items with per-cell colours (BatchItem::cell_col), else those with per-vertex colours; a
 // batch that holds both is rendered by one launch of each, every tile by the one matching its item.
 // kRound: fragments shaded per round (64, 128 or 256: segments per pass).  kSub: binning tiles larger than 8x8
-// (the workgroup's 8x8 sub-tile tests its own coverage).
-template <bool kCell, int kRound, bool kSub>
+// (the workgroup's 8x8 sub-tile tests its own coverage).  kEdge < 8: this wave renders part `part` of the tile
+// (PartOfTile).
+template <bool kCell, int kRound, bool kSub, int kEdge = kTileEdge>
 __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items, int nitems,
                                              const uint4* __restrict__ recs, const uint2* __restrict__ ranges,
                                              const PixelState& ps_all, uint32_t gsub, RecordLds& L,
-                                             FragListLds<kRound>& F) {
+                                             FragListLds<kRound>& F, uint32_t part = 0u) {
+    constexpr bool kPart = kEdge < kTileEdge;
+    static_assert(!(kPart && kSub), "parts of 8x8 binning tiles only");
     const BatchItem& B = items[item_of_sub(items, nitems, gsub)];
     if ((B.cell_col != nullptr) != kCell) return;
     const ViewUniforms& U = B.U;
@@ -76,12 +79,14 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
     const uint32_t gtile = st.gtile;
     const int lane = threadIdx.x;
     const uint64_t lt = lanemask_lt();
-    const int lx = lane & 7, ly = lane >> 3;
-    const int x = st.x0 + lx, y = st.y0 + ly;
+    const PartOfTile<kEdge> pt(part);
+    const int lx = lane % kEdge, ly = lane / kEdge;
+    const int x = st.x0 + pt.x0 + lx, y = st.y0 + pt.y0 + ly;
     // binning tiles larger than 8x8: coverage is tested here, from face triangles stashed in the fragment
     // list's space (free while a batch is staged)
     int32_t* stash = kSub ? reinterpret_cast<int32_t*>(F.entry) : nullptr;
-    const bool valid = x < U.width && y < U.height;
+    const bool valid = lane < pt.kPixels && x < U.width && y < U.height;
+    if (kPart && ballot(valid) == 0ull) return;
     const float3_ ro = f3(U.camPos[0], U.camPos[1], U.camPos[2]);
     {
         const float3_ rd = ray_direction(U, x, y);
@@ -98,28 +103,58 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
     uint32_t n = 0, last = rg.x, nck = 0, nlast = 0;
     bool done = !valid;
     // Two-stage prefetch: while a batch is shaded, the next batch's vertex data and the record words of the
-    // batch after it are in flight.
+    // batch after it are in flight (of a part: the candidates of the batch after that, too).
     RecordIn cur, nxt;
     RecordData cd;
-    if (lane < kBatch && rg.x + lane < rg.y) {
-        cur = load_record(recs, rg.x + lane);
-        fetch_record_data<kCell>(pos, col, cur, cd);
-    }
-    if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = load_record(recs, rg.x + kBatch + lane);
-    for (uint32_t base = rg.x; base < rg.y; base += kBatch) {
-        const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
-        if (lane < cnt) store_record<kSub>(U, cur, cd, L, lane, stash);
-        if (lane < kBatch && base + kBatch + lane < rg.y) {
-            cur = nxt;
+    PartFeed<kEdge, false> feed{recs, rg.x, rg.y, pt.origin, {}};
+    // a part's batch: the stream indices of its records (the entries of a part fill at most half the list)
+    static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kMaxFrags / 2, "no room for a part's indices");
+    uint32_t* const part_idx = reinterpret_cast<uint32_t*>(F.entry + kMaxFrags / 2);
+    uint32_t* const pend = part_idx + kBatch;
+    uint32_t cur_idx = 0u, nxt_idx = 0u;
+    int ncur = 0, nnxt = 0;
+    if constexpr (kPart) {
+        feed.load(lane);
+        ncur = feed.next(pend, lane, cur, cur_idx);
+        feed.load(lane);
+        if (lane < ncur) fetch_record_data<kCell>(pos, col, cur, cd);
+        nnxt = feed.next(pend, lane, nxt, nxt_idx);
+        feed.load(lane);
+    } else {
+        if (lane < kBatch && rg.x + lane < rg.y) {
+            cur = load_record(recs, rg.x + lane);
             fetch_record_data<kCell>(pos, col, cur, cd);
         }
-        if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = load_record(recs, base + 2 * kBatch + lane);
-        __syncthreads();
-        if constexpr (kSub) {
-            subtile_masks(L, stash, cnt, x, y, valid, lane);
+        if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = load_record(recs, rg.x + kBatch + lane);
+    }
+    for (uint32_t base = rg.x; kPart ? ncur > 0 : base < rg.y; base += kBatch) {
+        const int cnt = kPart ? ncur : (int)min((uint32_t)kBatch, rg.y - base);
+        if (lane < cnt) store_record<kSub>(U, cur, cd, L, lane, stash);
+        uint32_t mask;
+        if constexpr (kPart) {
+            if (lane < cnt) part_idx[lane] = cur_idx;
+            mask = pt.coverage(cur.rec, cnt, lane);
+            if (done) mask = 0u;
+            cur = nxt;
+            cur_idx = nxt_idx;
+            ncur = nnxt;
+            if (lane < ncur) fetch_record_data<kCell>(pos, col, cur, cd);
+            nnxt = feed.next(pend, lane, nxt, nxt_idx);
+            feed.load(lane);
             __syncthreads();
+        } else {
+            if (lane < kBatch && base + kBatch + lane < rg.y) {
+                cur = nxt;
+                fetch_record_data<kCell>(pos, col, cur, cd);
+            }
+            if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = load_record(recs, base + 2 * kBatch + lane);
+            __syncthreads();
+            if constexpr (kSub) {
+                subtile_masks(L, stash, cnt, x, y, valid, lane);
+                __syncthreads();
+            }
+            mask = done ? 0u : lane_coverage(L, cnt, lane);
         }
-        const uint32_t mask = done ? 0u : lane_coverage(L, cnt, lane);
         // the records' coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
         const uint32_t total = build_fragment_list(F.entry, rank_mask, mask, false, lane);
@@ -165,7 +200,7 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
                 }
                 C.w = Tout;
                 n++;
-                last = base + (F.entry[e] & 31) + 1;
+                last = (kPart ? part_idx[F.entry[e] & 31] : base + (F.entry[e] & 31)) + 1;
                 // periodic checkpoints bound the rounding the adjoint's chain of divisions accumulates; the last
                 // slot is kept for the underflow rule above
                 if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kTinyT && (int)nck < U.max_ckpt - 1) {
@@ -188,9 +223,11 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
         ps.last_rec[pix] = last;
         ps.num_ckpt[pix] = nck;
     }
-    // the tile's composited fragments: the adjoint's launch order ranks tiles by them
-    const uint32_t tile_total = wave_inclusive_scan(n);
-    if (lane == 63) ps.tile_frags[gsub] = tile_total;
+    // the tile's composited fragments: the adjoint's launch order ranks tiles by them (parts are not ranked)
+    if constexpr (!kPart) {
+        const uint32_t tile_total = wave_inclusive_scan(n);
+        if (lane == 63) ps.tile_frags[gsub] = tile_total;
+    }
 }
 
 // Next entry of the launch order for a persistent workgroup: one claim per tile from the launch's queue
@@ -224,18 +261,33 @@ __global__ __launch_bounds__(64) void k_render_forward(const BatchItem* __restri
     }
 }
 
+// (8 / kEdge)^2 workgroups per tile, one per part, in image order.
+template <bool kCell, int kEdge>
+__global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __restrict__ items, int nitems,
+                                                              const uint4* __restrict__ recs,
+                                                              const uint2* __restrict__ ranges, PixelState ps_all) {
+    __shared__ RecordLds L;
+    __shared__ FragListLds<kRoundDefault> F;
+    constexpr uint32_t kParts = PartOfTile<kEdge>::kParts;
+    forward_tile<kCell, kRoundDefault, false, kEdge>(items, nitems, recs, ranges, ps_all, blockIdx.x / kParts, L, F,
+                                                     blockIdx.x % kParts);
+}
+
 // kRef = false: exact derivative of the forward.  kRef = true: the reference's adjoint as written
 // (AdjointIntersectRasterization.glsl:111-362): per pixel from the blended output image, back to front, the
 // 'over' operator is inverted per sub-segment 3, 2, 1 (sub-segment 0 is skipped) with no checkpoints, and
 // each fragment's parameter gradients follow frag_backward_reference.
-// kCell: the items with per-cell colours (exact adjoint only), kSub: binning tiles larger than 8x8, as
-// k_render_forward.
-template <bool kRef, bool kCell, bool kSub>
+// kCell: the items with per-cell colours (exact adjoint only), kSub: binning tiles larger than 8x8, kEdge < 8: a
+// part of the tile, as k_render_forward.
+template <bool kRef, bool kCell, bool kSub, int kEdge = kTileEdge>
 __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items,
                                              const AdjointTarget* __restrict__ targets, int nitems,
                                              const uint4* __restrict__ recs, const uint2* __restrict__ ranges,
                                              const PixelState& ps_all, int use_abs, uint32_t gsub, RecordLds& L,
-                                             AdjFragLds& A, float4 (&s_seg)[kRef ? 3 : 1][kRoundAdj]) {
+                                             AdjFragLds& A, float4 (&s_seg)[kRef ? 3 : 1][kRoundAdj],
+                                             uint32_t part = 0u) {
+    constexpr bool kPart = kEdge < kTileEdge;
+    static_assert(!(kPart && kSub), "parts of 8x8 binning tiles only");
     const int item = item_of_sub(items, nitems, gsub);
     const BatchItem& B = items[item];
     if ((B.cell_col != nullptr) != kCell) return;
@@ -251,9 +303,10 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     const SubTile st = sub_tile(B, gsub);
     const uint32_t gtile = st.gtile;
     const int lane = threadIdx.x;
-    const int lx = lane & 7, ly = lane >> 3;
-    const int x = st.x0 + lx, y = st.y0 + ly;
-    const bool valid = x < U.width && y < U.height;
+    const PartOfTile<kEdge> pt(part);
+    const int lx = lane % kEdge, ly = lane / kEdge;
+    const int x = st.x0 + pt.x0 + lx, y = st.y0 + pt.y0 + ly;
+    const bool valid = lane < pt.kPixels && x < U.width && y < U.height;
     int32_t* stash = kSub ? reinterpret_cast<int32_t*>(A.entry) : nullptr;
     const float3_ ro = f3(U.camPos[0], U.camPos[1], U.camPos[2]);
     const float3_ my_rd = ray_direction(U, x, y);
@@ -300,24 +353,45 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     }
     bool done = !valid || n == 0;
     if (ballot(!done) == 0ull) return;
-    const uint32_t nrec = rg.y - rg.x;
-    const int nbatch = (int)((nrec + kBatch - 1) / kBatch);
-    // Batches run back to front.  The next batch's record words are loaded when the current batch starts and its
-    // vertex data just before the current batch's gradient atomics, so that staging it never waits on memory.
+    // Batches run back to front, from the last record that any of the wave's pixels composited (early ray
+    // termination leaves the records behind it out).  The next batch's record words are loaded when the current
+    // batch starts and its vertex data just before the current batch's gradient atomics, so that staging it never
+    // waits on memory.
+    const uint32_t behind = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u32(valid ? last : 0u));
+    const int nbatch = (int)((behind - rg.x + kBatch - 1) / kBatch);
     RecordIn nxt;
     RecordData nd;
-    {
+    PartFeed<kEdge, true> feed{recs, rg.x, behind, pt.origin, {}};
+    static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kAdjFrags / 2, "no room for a part's indices");
+    uint32_t* const part_idx = reinterpret_cast<uint32_t*>(A.entry + kAdjFrags / 2);  // as in the forward
+    uint32_t* const pend = part_idx + kBatch;
+    uint32_t nxt_idx = 0u;
+    int nnxt = 0;
+    if constexpr (kPart) {
+        feed.load(lane);
+        nnxt = feed.next(pend, lane, nxt, nxt_idx);
+        if (lane < nnxt) fetch_record_data<kCell>(pos, col, nxt, nd);
+    } else {
         const uint32_t b0 = rg.x + (uint32_t)(nbatch - 1) * kBatch;
         if (lane < kBatch && b0 + lane < rg.y) {
             nxt = load_record(recs, b0 + lane);
             fetch_record_data<kCell>(pos, col, nxt, nd);
         }
     }
-    for (int bi = nbatch - 1; bi >= 0; bi--) {
-        const uint32_t base = rg.x + (uint32_t)bi * kBatch;
-        const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
+    for (int bi = nbatch - 1; kPart ? nnxt > 0 : bi >= 0; bi--) {
+        const uint32_t base = kPart ? 0u : rg.x + (uint32_t)bi * kBatch;
+        const int cnt = kPart ? nnxt : (int)min((uint32_t)kBatch, rg.y - base);
         if (lane < cnt) store_record<kSub>(U, nxt, nd, L, lane, stash);
-        if (bi > 0 && lane < kBatch) nxt = load_record(recs, base - kBatch + lane);
+        uint32_t cover = 0u;
+        if constexpr (kPart) {
+            if (lane < cnt) part_idx[lane] = nxt_idx;
+            cover = pt.coverage(nxt.rec, cnt, lane);
+            feed.load(lane);
+            nnxt = feed.next(pend, lane, nxt, nxt_idx);
+        } else if (bi > 0 && lane < kBatch) {
+            nxt = load_record(recs, base - kBatch + lane);
+        }
+        const bool more = kPart ? nnxt > 0 : bi > 0;
         // lanes j and j + 32 own record j's 28 values (first / second half of 14) for this batch
         float acc[14];
 #pragma unroll
@@ -328,12 +402,19 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             __syncthreads();
         }
         // records at or after `last` were not composited in the forward (early ray termination)
-        const uint32_t nlive = last > base ? min((uint32_t)cnt, last - base) : 0u;
-        const uint32_t live = nlive >= 32u ? 0xFFFFFFFFu : ((1u << nlive) - 1u);
-        const uint32_t mask_all = done ? 0u : (lane_coverage(L, cnt, lane) & live);
+        uint32_t mask_all;
+        if constexpr (kPart) {  // slots back to front
+            uint32_t dead = 0u;
+            while (!done && dead < (uint32_t)cnt && part_idx[dead] >= last) dead++;
+            mask_all = done || dead >= 32u ? 0u : cover & (0xFFFFFFFFu << dead);
+        } else {
+            const uint32_t nlive = last > base ? min((uint32_t)cnt, last - base) : 0u;
+            const uint32_t live = nlive >= 32u ? 0xFFFFFFFFu : ((1u << nlive) - 1u);
+            mask_all = done ? 0u : (lane_coverage(L, cnt, lane) & live);
+        }
         // parts (back to front): all 32 records, or records 16-31 then 0-15 when the list exceeds kAdjFrags
         int nparts = 1;
-        {
+        if constexpr (!kPart) {
             const uint32_t inc = wave_inclusive_scan((uint32_t)__popc(mask_all));
             if ((uint32_t)__builtin_amdgcn_readlane((int)inc, 63) > (uint32_t)kAdjFrags) nparts = 2;
         }
@@ -341,7 +422,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
         const uint32_t pmask = nparts == 1 ? 0xFFFFFFFFu : (part == 0 ? 0xFFFF0000u : 0x0000FFFFu);
         const uint32_t mask = done ? 0u : (mask_all & pmask);
         uint32_t total;
-        const uint32_t off = build_fragment_list_by_pixel(A.entry, mask, true, lane, total);
+        const uint32_t off = build_fragment_list_by_pixel(A.entry, mask, !kPart, lane, total);
         const uint32_t mine_end = off + (uint32_t)__popc(mask);
         __syncthreads();
         for (uint32_t r0 = 0; r0 < total; r0 += kRoundAdj) {
@@ -614,8 +695,8 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             if (owner[1]) list[n0 + popc64(own1 & lanemask_lt())] = s1;
             __syncthreads();
             // The next batch's vertex data is requested before the atomics, so staging it does not wait for them.
-            // Only lanes 0..31 hold that batch's record words.
-            if (bi > 0 && lane < kBatch) fetch_record_data<kCell>(pos, col, nxt, nd);
+            // Only lanes 0..31 hold that batch's record words (of a part: lanes 0 to its count).
+            if (more && lane < (kPart ? nnxt : kBatch)) fetch_record_data<kCell>(pos, col, nxt, nd);
             uint32_t issued = 0;
             {
                 const int c = lane & 7;
@@ -678,6 +759,21 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint(const Batch
             __syncthreads();
         }
     }
+}
+
+template <bool kRef, bool kCell, int kEdge>
+__global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint_parts(const BatchItem* __restrict__ items,
+                                                                           const AdjointTarget* __restrict__ targets,
+                                                                           int nitems,
+                                                                           const uint4* __restrict__ recs,
+                                                                           const uint2* __restrict__ ranges,
+                                                                           PixelState ps_all, int use_abs) {
+    __shared__ RecordLds L;
+    __shared__ AdjFragLds A;
+    __shared__ float4 s_seg[kRef ? 3 : 1][kRoundAdj];
+    constexpr uint32_t kParts = PartOfTile<kEdge>::kParts;
+    adjoint_tile<kRef, kCell, false, kEdge>(items, targets, nitems, recs, ranges, ps_all, use_abs,
+                                            blockIdx.x / kParts, L, A, s_seg, blockIdx.x % kParts);
 }
 
 // Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.
@@ -788,10 +884,22 @@ static void launch_forward_kind(const BatchItem* items, int nitems, int64_t ntil
         launch_forward_round<kCell, kSub, kRoundDefault>(items, nitems, ntiles, order, recs, ranges, ps, queue, s);
 }
 
+template <int kEdge>
+static void launch_forward_parts(const BatchItem* items, int nitems, int64_t ntiles, const uint4* recs,
+                                 const uint2* ranges, PixelState ps, uint32_t colour_kinds, hipStream_t s) {
+    const dim3 grid((unsigned)(ntiles * PartOfTile<kEdge>::kParts));
+    if (colour_kinds & kColoursPerVertex)
+        hipLaunchKernelGGL((k_render_forward_parts<false, kEdge>), grid, dim3(64), 0, s, items, nitems, recs, ranges, ps);
+    if (colour_kinds & kColoursPerCell)
+        hipLaunchKernelGGL((k_render_forward_parts<true, kEdge>), grid, dim3(64), 0, s, items, nitems, recs, ranges, ps);
+}
+
 void launch_render_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
                            const uint4* recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
-                           hipStream_t s, int round, bool sub, uint32_t* queue) {
+                           hipStream_t s, int round, bool sub, uint32_t* queue, int edge) {
     if (ntiles <= 0) return;
+    if (edge == 4) return launch_forward_parts<4>(items, nitems, ntiles, recs, ranges, ps, colour_kinds, s);
+    if (edge == 2) return launch_forward_parts<2>(items, nitems, ntiles, recs, ranges, ps, colour_kinds, s);
     if (colour_kinds & kColoursPerVertex) {
         if (sub)
             launch_forward_kind<false, true>(items, nitems, ntiles, order, recs, ranges, ps, round, queue, s);
@@ -831,10 +939,32 @@ static void launch_adjoint_sub(const BatchItem* items, const AdjointTarget* targ
                                                queue, s);
 }
 
+template <int kEdge>
+static void launch_adjoint_parts(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
+                                 const uint4* recs, const uint2* ranges, PixelState ps, int use_abs, int mode,
+                                 uint32_t colour_kinds, hipStream_t s) {
+    const dim3 grid((unsigned)(ntiles * PartOfTile<kEdge>::kParts));
+    if ((colour_kinds & kColoursPerVertex) && mode == 1)
+        hipLaunchKernelGGL((k_render_adjoint_parts<true, false, kEdge>), grid, dim3(64), 0, s, items, targets, nitems,
+                           recs, ranges, ps, use_abs);
+    if ((colour_kinds & kColoursPerVertex) && mode != 1)
+        hipLaunchKernelGGL((k_render_adjoint_parts<false, false, kEdge>), grid, dim3(64), 0, s, items, targets,
+                           nitems, recs, ranges, ps, use_abs);
+    if (colour_kinds & kColoursPerCell)
+        hipLaunchKernelGGL((k_render_adjoint_parts<false, true, kEdge>), grid, dim3(64), 0, s, items, targets, nitems,
+                           recs, ranges, ps, use_abs);
+}
+
 void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                            const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps, int use_abs,
-                           int mode, uint32_t colour_kinds, hipStream_t s, bool sub, uint32_t* queue) {
+                           int mode, uint32_t colour_kinds, hipStream_t s, bool sub, uint32_t* queue, int edge) {
     if (ntiles <= 0) return;
+    if (edge == 4)
+        return launch_adjoint_parts<4>(items, targets, nitems, ntiles, recs, ranges, ps, use_abs, mode, colour_kinds,
+                                       s);
+    if (edge == 2)
+        return launch_adjoint_parts<2>(items, targets, nitems, ntiles, recs, ranges, ps, use_abs, mode, colour_kinds,
+                                       s);
     if (sub)
         launch_adjoint_sub<true>(items, targets, nitems, ntiles, order, recs, ranges, ps, use_abs, mode,
                                  colour_kinds, queue, s);

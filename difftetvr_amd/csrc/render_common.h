@@ -182,6 +182,101 @@ __device__ __forceinline__ uint32_t lane_coverage(const RecordLds& L, int cnt, i
     return m;
 }
 
+// Waves of a part of a tile.  With fewer 8x8 tiles than the GPU has SIMDs, a wave per tile leaves most of the chip
+// idle while the deepest tile's wave runs alone.  A tile is then rendered by (8 / kEdge)^2 waves of kEdge x kEdge
+// pixels each.  A wave's batches hold only the records that cover its own pixels, picked from the tile's stream
+// by their coverage masks, 128 candidates at a time.
+template <int kEdge>
+struct PartOfTile {
+    static constexpr int kAcross = 8 / kEdge, kParts = kAcross * kAcross, kPixels = kEdge * kEdge;
+    uint32_t origin;  // bit of the part's first pixel in a tile's coverage mask
+    int x0, y0;       // its position within the tile
+    __device__ __forceinline__ explicit PartOfTile(uint32_t part) {
+        x0 = (int)(part % kAcross) * kEdge;
+        y0 = (int)(part / kAcross) * kEdge;
+        origin = (uint32_t)(y0 * kTileEdge + x0);
+    }
+    // The pixels' bits of a coverage mask shifted down by origin.
+    static constexpr uint64_t pixel_bits() {
+        uint64_t m = 0;
+        for (int y = 0; y < kEdge; y++) m |= ((1ull << kEdge) - 1ull) << (kTileEdge * y);
+        return m;
+    }
+    // 32-bit mask of the batch's records (bit j: record j) that cover this lane's pixel; rec: lane j's record.
+    __device__ __forceinline__ uint32_t coverage(uint4 rec, int cnt, int lane) const {
+        const uint64_t m = lane < cnt ? (((uint64_t)rec.z << 32) | rec.y) >> origin : 0ull;
+        uint32_t mine = 0u;
+#pragma unroll
+        for (int p = 0; p < kPixels; p++) {
+            const uint32_t b = (uint32_t)ballot((m >> (kTileEdge * (p / kEdge) + p % kEdge)) & 1ull);
+            mine = lane == p ? b : mine;
+        }
+        return mine;
+    }
+};
+
+// The records of stream [begin, end) that cover a part's pixels, in stream order or (kReverse) against it.
+template <int kEdge, bool kReverse>
+struct PartFeed {
+    const uint4* __restrict__ recs;
+    uint32_t begin, end;  // the records not yet passed
+    uint32_t origin;
+    uint2 cand[2];        // coverage masks of this lane's candidates
+    __device__ __forceinline__ uint32_t index(int k, int lane) const {
+        return kReverse ? end - 1u - (uint32_t)(64 * k + lane) : begin + (uint32_t)(64 * k + lane);
+    }
+    __device__ __forceinline__ bool within(int k, int lane) const { return (uint32_t)(64 * k + lane) < end - begin; }
+    // Requests the next 128 candidates' masks.
+    __device__ __forceinline__ void load(int lane) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            cand[k] = make_uint2(0u, 0u);
+            if (within(k, lane)) {
+                const uint4* r = recs + 2 * (int64_t)index(k, lane) + 1;
+                cand[k] = make_uint2(r->y, r->z);
+            }
+        }
+    }
+    // The next batch, from the candidates load requested: lane j < the returned count gets record j and its index.
+    // pend: 32 words of LDS.
+    __device__ __forceinline__ int next(uint32_t* pend, int lane, RecordIn& r, uint32_t& idx) {
+        const uint64_t lt = lanemask_lt();
+        int cnt = 0;
+        while (end != begin) {
+            bool full = false;
+            uint32_t passed = 0;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                if (full) continue;
+                const uint64_t m = (((uint64_t)cand[k].y << 32) | cand[k].x) >> origin;
+                const bool hit = within(k, lane) && (m & PartOfTile<kEdge>::pixel_bits()) != 0ull;
+                const uint64_t hits = ballot(hit);
+                const int rank = cnt + popc64(hits & lt);
+                const bool take = hit && rank < kBatch;
+                if (take) pend[rank] = index(k, lane);
+                const int n = popc64(hits);
+                if (cnt + n >= kBatch) {
+                    full = true;
+                    passed = (uint32_t)(64 * k + 64 - __builtin_clzll(ballot(take)));
+                    cnt = kBatch;
+                } else {
+                    cnt += n;
+                    passed = min((uint32_t)(64 * (k + 1)), end - begin);
+                }
+            }
+            if (kReverse) end -= passed; else begin += passed;
+            if (full) break;
+            load(lane);
+        }
+        __syncthreads();
+        if (lane < cnt) {
+            idx = pend[lane];
+            r = load_record(recs, idx);
+        }
+        return cnt;
+    }
+};
+
 __device__ __forceinline__ float3_ lds_p(const RecordLds& L, int v, int j) {
     return f3(L.p[3 * v][j], L.p[3 * v + 1][j], L.p[3 * v + 2][j]);
 }
