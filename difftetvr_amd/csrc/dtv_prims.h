@@ -69,13 +69,56 @@ __device__ __forceinline__ void dpp_halve(const float (&in)[N], float (&out)[(N 
         out[k] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), CTRL, 0xF, 0xF, true));
     }
 }
+
+// The levels of row-lane bits 3 (row mirror) and 2 (half-row mirror): the lanes that keep x, and those that keep
+// y, are whole banks of four lanes there, so two masked additions do without the selects.  s_nop 1: a DPP operand
+// must not have been written by the two preceding VALU instructions, which the compiler cannot see in here.
+#define DTV_DPP_PAIR(NAME, MODE, LO, HI)                                                                           \
+    __device__ __forceinline__ float NAME(float x, float y) {                                                      \
+        float r;                                                                                                   \
+        asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 " MODE " row_mask:0xf bank_mask:" LO                     \
+                     "\n\tv_add_f32_dpp %0, %2, %2 " MODE " row_mask:0xf bank_mask:" HI                            \
+                     : "=&v"(r)                                                                                    \
+                     : "v"(x), "v"(y));                                                                            \
+        return r;                                                                                                  \
+    }                                                                                                              \
+    __device__ __forceinline__ void NAME##4(const float* in, float* out) {                                         \
+        asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %4, %4 " MODE " row_mask:0xf bank_mask:" LO                     \
+                     "\n\tv_add_f32_dpp %0, %5, %5 " MODE " row_mask:0xf bank_mask:" HI                            \
+                     "\n\tv_add_f32_dpp %1, %6, %6 " MODE " row_mask:0xf bank_mask:" LO                            \
+                     "\n\tv_add_f32_dpp %1, %7, %7 " MODE " row_mask:0xf bank_mask:" HI                            \
+                     "\n\tv_add_f32_dpp %2, %8, %8 " MODE " row_mask:0xf bank_mask:" LO                            \
+                     "\n\tv_add_f32_dpp %2, %9, %9 " MODE " row_mask:0xf bank_mask:" HI                            \
+                     "\n\tv_add_f32_dpp %3, %10, %10 " MODE " row_mask:0xf bank_mask:" LO                          \
+                     "\n\tv_add_f32_dpp %3, %11, %11 " MODE " row_mask:0xf bank_mask:" HI                          \
+                     : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3])                                  \
+                     : "v"(in[0]), "v"(in[1]), "v"(in[2]), "v"(in[3]), "v"(in[4]), "v"(in[5]), "v"(in[6]),         \
+                       "v"(in[7]));                                                                                \
+    }
+DTV_DPP_PAIR(dpp_row_mirror, "row_mirror", "0x3", "0xc")
+DTV_DPP_PAIR(dpp_half_mirror, "row_half_mirror", "0x5", "0xa")
+#undef DTV_DPP_PAIR
+
+template <int BIT, int N>
+__device__ __forceinline__ void dpp_halve_banks(const float (&in)[N], float (&out)[(N + 1) / 2]) {
+    constexpr int kFours = N / 8;
+#pragma unroll
+    for (int f = 0; f < kFours; f++) {
+        if constexpr (BIT == 3) dpp_row_mirror4(in + 8 * f, out + 4 * f); else dpp_half_mirror4(in + 8 * f, out + 4 * f);
+    }
+#pragma unroll
+    for (int k = 4 * kFours; k < (N + 1) / 2; k++) {
+        const float x = in[2 * k], y = in[2 * k + 1 < N ? 2 * k + 1 : 2 * k];
+        if constexpr (BIT == 3) out[k] = dpp_row_mirror(x, y); else out[k] = dpp_half_mirror(x, y);
+    }
+}
 }  // namespace detail
 
 // Reduce-scatter of N <= 32 per-lane values within each row of 16 lanes (each row reduces its own values):
 // lane L returns in out[k] the row's sum of value 16 k + row_scatter_index(L) (meaningful when below N).  Each
 // level pairs the values and halves them across one row-lane bit (3 and 2 by the DPP row mirror and half-row
-// mirror, 1 and 0 by quad permutations): about 3 VALU instructions per pair and level, where a full row sum of
-// every value costs about 8 each.  All lanes must be active.
+// mirror, 1 and 0 by quad permutations): 2 VALU instructions per pair on the first two levels and 3 on the others,
+// where a full row sum of every value costs about 8 each.  All lanes must be active.
 __device__ __forceinline__ int row_scatter_index(int lane) {
     return ((lane >> 3) & 1) | ((lane >> 1) & 2) | ((lane << 1) & 4) | ((lane << 3) & 8);
 }
@@ -86,8 +129,8 @@ __device__ __forceinline__ void row_reduce_scatter(const float (&v)[N], float (&
     constexpr int N1 = (N + 1) / 2, N2 = (N1 + 1) / 2, N3 = (N2 + 1) / 2;
     const int lane = lane_id();
     float a[N1], b[N2], c[N3];
-    detail::dpp_halve<0x140, 3>(v, a, lane);    // row_mirror: lane i <-> 15 - i
-    detail::dpp_halve<0x141, 2>(a, b, lane);    // row_half_mirror: lane i <-> 7 - i
+    detail::dpp_halve_banks<3>(v, a);           // row_mirror: lane i <-> 15 - i
+    detail::dpp_halve_banks<2>(a, b);           // row_half_mirror: lane i <-> 7 - i
     detail::dpp_halve<0x4E, 1>(b, c, lane);     // quad_perm [2,3,0,1]: lane i <-> i ^ 2
     detail::dpp_halve<0xB1, 0>(c, out, lane);   // quad_perm [1,0,3,2]: lane i <-> i ^ 1
 }
@@ -139,6 +182,10 @@ __device__ __forceinline__ uint64_t status_load64(const uint64_t* p) {
 __device__ __forceinline__ void atomic_add_f32(float* p, float v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// Waits for every load issued so far (vmcnt 0, the other counters unconstrained): loads and atomics share one
+// in-order counter, so values that are in registers before a group of atomics is issued need not wait for those.
+__device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // p in LDS.
 __device__ __forceinline__ void lds_add_f32(float* p, float v) {

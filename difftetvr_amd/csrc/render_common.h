@@ -633,6 +633,39 @@ __device__ __forceinline__ PixelState item_pixel_state(const PixelState& all, co
     return ps;
 }
 
+// A pixel's stored checkpoints, walked back to front: the next one's fragment count and transmittance (n1, t1; n1 =
+// 0xFFFFFFFF: none left), and those of the one before it, requested a checkpoint ahead: the step that passes a
+// checkpoint then waits for no load.
+struct CheckpointCursor {
+    uint32_t n1 = 0xFFFFFFFFu, n2 = 0xFFFFFFFFu;
+    float t1 = 1.0f, t2 = 1.0f;
+    int left = 0;  // checkpoints before (n2, t2)
+    __device__ __forceinline__ void request(int64_t P, const PixelState& ps, int pix) {
+        n2 = 0xFFFFFFFFu;
+        left--;
+        if (left >= 0) {
+            n2 = ps.ckpt_n[(int64_t)left * P + pix];
+            t2 = ps.ckpt_t[(int64_t)left * P + pix];
+        }
+    }
+    __device__ __forceinline__ void start(int count, int64_t P, const PixelState& ps, int pix) {
+        left = count;
+        request(P, ps, pix);
+        n1 = n2;
+        t1 = t2;
+        request(P, ps, pix);
+    }
+    // With n fragments still to undo: the transmittance behind them from a checkpoint taken there.
+    __device__ __forceinline__ void restore(uint32_t n, float& T, int64_t P, const PixelState& ps, int pix) {
+        if (n1 == n) {
+            T = t1;
+            n1 = n2;
+            t1 = t2;
+            request(P, ps, pix);
+        }
+    }
+};
+
 // ---------------------------------------------------------------------------------------------------------
 // Exact adjoint of one fragment given dL/dF.  Writes per-local-vertex gradients gp[v][xyz], gc[v][rgba].
 // Position gradient of face vertex j:  mu_j(P) * Q, Q = s*dLdt*N/(N.d) - [G^T dC - N (dC.G d)/(N.d)] with G the
