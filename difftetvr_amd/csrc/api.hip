@@ -2,6 +2,7 @@
 // pipeline, and the optimiser entry points.  Host C++; all device work is enqueued on the caller's stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -185,7 +186,6 @@ int setup_noalloc_scratch(int device) {
     return DTV_OK;
 }
 
-__global__ void k_store_item(BatchItem item, BatchItem* __restrict__ dst) { *dst = item; }
 __global__ void k_copy_flag(const uint32_t* __restrict__ src, int32_t* __restrict__ dst) { *dst = (int32_t)*src; }
 
 }  // namespace
@@ -208,10 +208,8 @@ struct dtv_view {
     int pinned_targets_cap = 0;
     hipEvent_t targets_copied = nullptr;   // the last upload out of pinnedTargets
     bool targets_pending = false;
-    BinStats* pinnedStats = nullptr;
-    DevBuf dItems, dTargets, counts, offsets, scan_status, small, block_stats, keys, vals, keys2, vals2,
-        recs, hist,
-        lookback, ranges;
+    ViewScratch* pinnedStats = nullptr;
+    DevBuf dItems, dTargets, bin_status, small, keys, vals, keys2, vals2, recs, hist, lookback, ranges;
     DevBuf ray_color, frag_count, last_rec, num_ckpt, ckpt_t, ckpt_n;
     DevBuf tile_frags, tile_order;  // per tile: forward's fragments; launch orders of the forward and adjoint
     DevBuf pt_info, pt_vert, pt_col, tri_grad;  // Projection renderer: per-tet triangles, per-corner gradients
@@ -237,8 +235,22 @@ struct dtv_view {
         if (which == 1) ev_recorded[stage] = true;
     }
     int nitems() const { return (int)items.size(); }
-    const uint4* sorted_recs() const { return recs.as<uint4>(); }
-    uint32_t* tile_queue() const { return reinterpret_cast<uint32_t*>(small.as<char>() + 384); }
+    ViewScratch* scratch() const { return small.as<ViewScratch>(); }
+    RecordStream stream() const { return {recs.as<uint4>(), &scratch()->route}; }
+    uint32_t* tile_queue() const { return &scratch()->queue; }
+    // Records the record and sort buffers hold (rec_bytes each in recs).
+    int64_t record_room(size_t rec_bytes) const {
+        const size_t n = std::min({keys.cap / 8, keys2.cap / 8, vals.cap / 4, vals2.cap / 4, recs.cap / rec_bytes});
+        return (int64_t)std::min<size_t>(n, (size_t)1 << 30);
+    }
+    hipError_t ensure_records(int64_t n, size_t rec_bytes) {
+        const size_t k = (size_t)(n > 0 ? n : 1);
+        for (DevBuf* b : {&keys, &keys2})
+            if (hipError_t e = b->ensure(8 * k); e != hipSuccess) return e;
+        for (DevBuf* b : {&vals, &vals2})
+            if (hipError_t e = b->ensure(4 * k); e != hipSuccess) return e;
+        return recs.ensure(rec_bytes * k);
+    }
     PixelState pixel_state() const {
         PixelState ps;
         ps.ray_color = ray_color.as<float4>();
@@ -340,7 +352,7 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     params = &prm;
     std::vector<BatchItem> items((size_t)n);
     std::vector<int64_t> item_V((size_t)n);
-    int64_t blocks = 0, tiles = 0, subtiles = 0, pixels = 0;
+    int64_t blocks = 0, tiles = 0, subtiles = 0, pixels = 0, tets = 0;
     uint32_t kinds = 0;
     for (int i = 0; i < n; i++) {
         const dtv_render_item& it = in[i];
@@ -371,7 +383,8 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
         B.sub0 = (uint32_t)subtiles;
         B.pixel0 = pixels;
         item_V[(size_t)i] = m.num_vertices;
-        blocks += count_pairs_blocks(m.num_cells);
+        blocks += bin_blocks(m.num_cells);
+        tets += m.num_cells;
         tiles += (int64_t)B.U.tiles_x * B.U.tiles_y;
         subtiles += (int64_t)B.U.sub_x * B.U.sub_y;
         pixels += (int64_t)B.U.width * B.U.height;
@@ -380,121 +393,118 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     }
     DTV_HIP(hipSetDevice(view->ctx->device));
     view->rendered = false;
-    // The items reach the device through pinned staging.  Under stream capture the upload becomes a graph node
-    // that reads the staging at every replay; otherwise the previous render's upload must have left the staging
-    // before it is overwritten (in planned mode nothing else waits for the device between renders).
-    if (!view->items_copied) DTV_HIP(hipEventCreateWithFlags(&view->items_copied, hipEventDisableTiming));
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     DTV_HIP(hipStreamIsCapturing(s, &capture));
     const bool capturing = capture != hipStreamCaptureStatusNone;
-    if (view->items_pending && !capturing) DTV_HIP(hipEventSynchronize(view->items_copied));
-    view->items_pending = false;
-    if (view->pinned_items_cap < n) {
-        if (view->pinnedItems) DTV_HIP(hipHostFree(view->pinnedItems));
-        view->pinnedItems = nullptr;
-        view->pinned_items_cap = 0;
-        DTV_HIP(hipHostMalloc((void**)&view->pinnedItems, sizeof(BatchItem) * (size_t)n, hipHostMallocDefault));
-        view->pinned_items_cap = n;
-    }
-    std::memcpy(view->pinnedItems, items.data(), sizeof(BatchItem) * (size_t)n);
     DTV_HIP(view->dItems.ensure(sizeof(BatchItem) * (size_t)n));
-    DTV_HIP(hipMemcpyAsync(view->dItems.p, view->pinnedItems, sizeof(BatchItem) * (size_t)n, hipMemcpyHostToDevice,
-                           s));
-    if (!capturing) {
-        DTV_HIP(hipEventRecord(view->items_copied, s));
-        view->items_pending = true;
-    }
     const BatchItem* dI = view->dItems.as<BatchItem>();
+    // One item reaches the device as a kernel argument, several through pinned staging.  Under stream capture the
+    // upload becomes a graph node that reads the staging at every replay; otherwise the previous render's upload
+    // must have left the staging before it is overwritten (in planned mode nothing else waits for the device
+    // between renders).
+    if (n > 1) {
+        if (!view->items_copied) DTV_HIP(hipEventCreateWithFlags(&view->items_copied, hipEventDisableTiming));
+        if (view->items_pending && !capturing) DTV_HIP(hipEventSynchronize(view->items_copied));
+        view->items_pending = false;
+        if (view->pinned_items_cap < n) {
+            if (view->pinnedItems) DTV_HIP(hipHostFree(view->pinnedItems));
+            view->pinnedItems = nullptr;
+            view->pinned_items_cap = 0;
+            DTV_HIP(hipHostMalloc((void**)&view->pinnedItems, sizeof(BatchItem) * (size_t)n, hipHostMallocDefault));
+            view->pinned_items_cap = n;
+        }
+        std::memcpy(view->pinnedItems, items.data(), sizeof(BatchItem) * (size_t)n);
+        DTV_HIP(hipMemcpyAsync(view->dItems.p, view->pinnedItems, sizeof(BatchItem) * (size_t)n,
+                               hipMemcpyHostToDevice, s));
+        if (!capturing) {
+            DTV_HIP(hipEventRecord(view->items_copied, s));
+            view->items_pending = true;
+        }
+    }
 
-    // 1. count (tile, face) records per tet, 2. scan
+    // 1. bin: (tile, face) records in (tet, face, tile) order
     const int64_t nslots = 256 * (blocks > 0 ? blocks : 1);
-    DTV_HIP(view->counts.ensure(sizeof(uint32_t) * nslots));
-    DTV_HIP(view->offsets.ensure(sizeof(uint32_t) * nslots));
-    DTV_HIP(view->scan_status.ensure(sizeof(uint64_t) * (scan_partitions(nslots) + 1)));
-    // stats 0, scan counter 64, total 128, overflow 192, atomics 256, sort route 320 (48 B), tile queue 384
-    DTV_HIP(view->small.ensure(448));
-    BinStats* dstats = view->small.as<BinStats>();
-    uint32_t* scan_counter = reinterpret_cast<uint32_t*>(view->small.as<char>() + 64);
-    uint64_t* scan_total = reinterpret_cast<uint64_t*>(view->small.as<char>() + 128);
-    DTV_HIP(view->block_stats.ensure(sizeof(uint32_t) * 4 * (blocks + 1)));
+    const size_t rec_bytes = proj ? sizeof(uint4) : 2 * sizeof(uint4);
+    DTV_HIP(view->bin_status.ensure(sizeof(uint64_t) * (size_t)bin_status_words(blocks)));
+    DTV_HIP(view->small.ensure(sizeof(ViewScratch)));
+    DTV_HIP(view->hist.ensure(sizeof(uint32_t) * (8 * 256 + 8)));
+    DTV_HIP(view->ranges.ensure(sizeof(uint2) * tiles));
     if (proj) {
         DTV_HIP(view->pt_info.ensure(sizeof(uint32_t) * nslots));
         DTV_HIP(view->pt_vert.ensure(sizeof(float4) * 5 * nslots));
         DTV_HIP(view->pt_col.ensure(sizeof(float4) * 5 * nslots));
     }
-    view->mark(DTV_STAGE_COUNT_PAIRS, 0, s);
-    if (proj)
-        launch_pt_count(dI, n, blocks, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
-                        view->pt_col.as<float4>(), view->counts.as<uint32_t>(), view->block_stats.as<uint32_t>(), s);
-    else
-        launch_count_pairs(dI, n, blocks, view->counts.as<uint32_t>(), view->block_stats.as<uint32_t>(), s);
-    view->mark(DTV_STAGE_COUNT_PAIRS, 1, s);
-    view->mark(DTV_STAGE_SCAN, 0, s);
-    scan_exclusive_u32(view->counts.as<uint32_t>(), view->offsets.as<uint32_t>(), 256 * blocks,
-                       view->scan_status.as<uint64_t>(), scan_counter, scan_total, s);
-    launch_reduce_bin_stats(view->block_stats.as<uint32_t>(), blocks, scan_total, dstats, s);
-    view->mark(DTV_STAGE_SCAN, 1, s);
-    DTV_HIP(hipGetLastError());
-    // The record count: read back after one synchronisation, or, in planned mode, a fixed capacity with the
-    // count left in device memory (scan_total) for the kernels to read.
+    ViewScratch* scratch = view->scratch();
+    uint32_t* hist = view->hist.as<uint32_t>();
+    // The record count: read back after one synchronisation (the records are then in place unless the buffers
+    // turn out too small, as in a view's first render, which bins again into larger ones), or, in planned mode, a
+    // fixed capacity with the count left in device memory for the kernels to read.
     const bool planned = view->planned_cap > 0;
-    BinStats st{};
-    int64_t K;
+    const bool small = bin_small(tets, pixels);
+    if (planned) DTV_HIP(view->ensure_records(view->planned_cap, rec_bytes));
+    auto bin = [&](int64_t cap) {
+        ClearList clear;
+        clear.add(view->bin_status.p, 2 * bin_status_words(blocks));
+        clear.add(scratch, (int64_t)(offsetof(ViewScratch, cleared) / 4));
+        clear.add(hist, 8 * 256 + 8);
+        clear.add(view->ranges.p, 2 * tiles);
+        launch_clear(clear, n == 1 ? &items[0] : nullptr, n == 1 ? view->dItems.as<BatchItem>() : nullptr, nullptr, 0,
+                     nullptr, s);
+        const BinOut out{view->bin_status.as<uint64_t>(), scratch, view->keys.as<uint64_t>(), view->recs.as<uint4>(),
+                         (uint64_t)cap};
+        if (proj)
+            launch_pt_bin(dI, n, blocks, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
+                          view->pt_col.as<float4>(), small, out, s);
+        else
+            launch_bin(dI, n, blocks, small, out, s);
+    };
+    view->mark(DTV_STAGE_COUNT_PAIRS, 0, s);
+    int64_t K = planned ? view->planned_cap : view->record_room(rec_bytes);
+    bin(K);
+    uint32_t dmin = 0;
+    int dbits = 0;
     if (!planned) {
-        DTV_HIP(hipMemcpyAsync(view->pinnedStats, dstats, sizeof(BinStats), hipMemcpyDeviceToHost, s));
+        DTV_HIP(hipMemcpyAsync(view->pinnedStats, scratch, offsetof(ViewScratch, ticket), hipMemcpyDeviceToHost, s));
         DTV_HIP(hipStreamSynchronize(s));
-        st = *view->pinnedStats;
-        if (st.total_pairs >= (1ull << 30))
+        const ViewScratch& st = *view->pinnedStats;
+        if (st.total >= (1ull << 30))
             return fail(DTV_ERR_OUT_OF_MEMORY, f + ": more than 2^30 (tile, face) records");
-        K = (int64_t)st.total_pairs;
+        if ((int64_t)st.total > K) {
+            DTV_HIP(view->ensure_records((int64_t)st.total, rec_bytes));
+            bin((int64_t)st.total);
+        }
+        K = (int64_t)st.total;
         view->num_pairs = K;
-        view->num_tris = st.num_tris;
+        view->num_tris = 0;
+        uint32_t not_min = 0, dmax = 0;
+        for (const BinSlot& b : st.slots) {
+            view->num_tris += b.tris;
+            not_min = std::max(not_min, b.not_min);
+            dmax = std::max(dmax, b.max);
+        }
+        dmin = ~not_min;
+        if (dmax > dmin) dbits = sort_bits(dmax - dmin);
     } else {
-        K = view->planned_cap;
         view->num_pairs = -1;
         view->num_tris = -1;
     }
-    const uint64_t* n_dev = planned ? scan_total : nullptr;
-    uint32_t* overflow = reinterpret_cast<uint32_t*>(view->small.as<char>() + 192);
-    fill_u32(overflow, 0u, 1, s);
+    view->mark(DTV_STAGE_COUNT_PAIRS, 1, s);
+    for (int stage : {DTV_STAGE_SCAN, DTV_STAGE_EMIT}) {  // part of the binning pass
+        view->mark(stage, 0, s);
+        view->mark(stage, 1, s);
+    }
+    DTV_HIP(hipGetLastError());
+    const uint64_t* n_dev = planned ? &scratch->total : nullptr;
 
-    // 3. emit, 4. sort, 5. tile ranges
-    DTV_HIP(view->keys.ensure(sizeof(uint64_t) * (K > 0 ? K : 1)));
-    DTV_HIP(view->vals.ensure(sizeof(uint32_t) * (K > 0 ? K : 1)));
-    DTV_HIP(view->keys2.ensure(sizeof(uint64_t) * (K > 0 ? K : 1)));
-    DTV_HIP(view->vals2.ensure(sizeof(uint32_t) * (K > 0 ? K : 1)));
-    DTV_HIP(view->recs.ensure(2 * sizeof(uint4) * (K > 0 ? K : 1)));
-    view->mark(DTV_STAGE_EMIT, 0, s);
-    if (proj)
-        launch_pt_emit(dI, n, blocks, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
-                       view->offsets.as<uint32_t>(), view->counts.as<uint32_t>(), view->keys.as<uint64_t>(),
-                       view->vals.as<uint32_t>(), K, overflow, s);
-    else
-        launch_emit_pairs(dI, n, blocks, view->offsets.as<uint32_t>(), view->counts.as<uint32_t>(),
-                          view->keys.as<uint64_t>(), view->vals.as<uint32_t>(), K, overflow, s);
-    view->mark(DTV_STAGE_EMIT, 1, s);
-    uint32_t mask = 0;
-    // planned: a pass per depth digit (which of them vary is not known on the host; constant ones exit at once)
-    const uint32_t varying = planned ? 0xFFFFFFFFu : (st.key_and ^ st.key_or);
-    for (int p = 0; p < 4; p++)
-        if ((varying >> (8 * p)) & 255u) mask |= 1u << p;
-    int tile_bits = 0;
-    while ((1ll << tile_bits) < tiles) tile_bits++;
-    for (int p = 0; 8 * p < tile_bits; p++) mask |= 1u << (4 + p);
-    int npass = 0;
-    for (int p = 0; p < 8; p++) npass += (mask >> p) & 1;
-    DTV_HIP(view->hist.ensure(sizeof(uint32_t) * 8 * 256 + 64));
-    DTV_HIP(view->lookback.ensure(sizeof(uint32_t) * 256 * (size_t)(npass > 0 ? npass : 1) *
-                                  (size_t)(sort_partitions(K) + 1)));
-    // planned: a depth digit all keys share costs one launch that exits at once (the sort routes on the device)
-    SortRoute* route = reinterpret_cast<SortRoute*>(view->small.as<char>() + 320);
+    // 2. sort the records by (tile, depth)
+    int tbits = 0;
+    while ((1ll << tbits) < tiles) tbits++;
+    const SortInput sort_in{view->keys.as<uint64_t>(), view->keys2.as<uint64_t>(), view->vals.as<uint32_t>(),
+                       view->vals2.as<uint32_t>(), K, n_dev, planned ? scratch->slots : nullptr, dmin, dbits, tbits};
+    DTV_HIP(view->lookback.ensure(sizeof(uint32_t) * (size_t)sort_lookback_words(K, sort_max_passes(tbits))));
     view->mark(DTV_STAGE_SORT, 0, s);
-    view->sort_passes = radix_sort_pairs(view->keys.as<uint64_t>(), view->vals.as<uint32_t>(),
-                                         view->keys2.as<uint64_t>(), view->vals2.as<uint32_t>(), K, n_dev, mask,
-                                         view->hist.as<uint32_t>(), view->lookback.as<uint32_t>(),
-                                         view->hist.as<uint32_t>() + 8 * 256, route, s);
+    view->sort_passes = sort_records(sort_in, hist, hist + 8 * 256, view->lookback.as<uint32_t>(), &scratch->route, s);
     view->mark(DTV_STAGE_SORT, 1, s);
-    DTV_HIP(view->ranges.ensure(sizeof(uint2) * tiles));
     DTV_HIP(view->tile_frags.ensure(sizeof(uint32_t) * subtiles));
     DTV_HIP(view->tile_order.ensure(2 * sizeof(uint32_t) * subtiles));
     const int edge = wave_edge(*params, tiles);
@@ -502,7 +512,8 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     // forward launch order: tiles by record count, heaviest first
     const uint32_t* fwd_order = view->cost_ordered ? view->tile_order.as<uint32_t>() : nullptr;
     view->mark(DTV_STAGE_RANGES, 0, s);
-    launch_tile_ranges(route, K, n_dev, tiles, view->ranges.as<uint2>(), s);
+    launch_tile_ranges(&scratch->route, K, n_dev, view->ranges.as<uint2>(), edge < 8 ? view->recs.as<uint4>() : nullptr,
+                       s);
     if (fwd_order) {
         if (tile == 8) {
             launch_tile_order(view->ranges.as<uint2>(), nullptr, tiles, view->tile_order.as<uint32_t>(), s);
@@ -512,14 +523,9 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
             launch_tile_order(nullptr, cost, subtiles, view->tile_order.as<uint32_t>(), s);
         }
     }
-    if (proj)
-        launch_pt_gather(dI, n, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(), route, K, n_dev,
-                         view->recs.as<uint4>(), s);
-    else
-        launch_gather_records(dI, n, route, K, n_dev, view->recs.as<uint4>(), s);
     view->mark(DTV_STAGE_RANGES, 1, s);
 
-    // 6. render
+    // 3. render
     DTV_HIP(view->ray_color.ensure(sizeof(float4) * pixels));
     DTV_HIP(view->frag_count.ensure(sizeof(uint32_t) * pixels));
     DTV_HIP(view->last_rec.ensure(sizeof(uint32_t) * pixels));
@@ -528,11 +534,10 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     DTV_HIP(view->ckpt_n.ensure(sizeof(uint32_t) * pixels * kMaxCheckpoints));
     view->mark(DTV_STAGE_FORWARD, 0, s);
     if (proj)
-        launch_pt_forward(dI, n, tiles, fwd_order, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
-                          view->pt_col.as<float4>(), view->sorted_recs(), view->ranges.as<uint2>(),
-                          view->pixel_state(), s);
+        launch_pt_forward(dI, n, tiles, fwd_order, view->pt_vert.as<float4>(), view->pt_col.as<float4>(),
+                          view->stream(), view->ranges.as<uint2>(), view->pixel_state(), s);
     else
-        launch_render_forward(dI, n, subtiles, fwd_order, view->sorted_recs(), view->ranges.as<uint2>(),
+        launch_render_forward(dI, n, subtiles, fwd_order, view->stream(), view->ranges.as<uint2>(),
                               view->pixel_state(), kinds, s, spp, tile != 8,
                               params->tile_launch == DTV_TILE_LAUNCH_QUEUE ? view->tile_queue() : nullptr, edge);
     view->edge = edge;
@@ -577,21 +582,28 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         if (!aligned16(tg[i].dimage)) return fail(DTV_ERR_INVALID_ARGUMENT, f + ": dimage must be 16-byte aligned");
     }
     DTV_HIP(hipSetDevice(view->ctx->device));
-    if (!view->targets_copied) DTV_HIP(hipEventCreateWithFlags(&view->targets_copied, hipEventDisableTiming));
-    // Under stream capture the upload becomes a graph node that reads the staging at every replay (nothing may
-    // wait on the device then); otherwise the staging of the previous call must have been consumed first.
+    // Few targets reach the device as kernel arguments, more through pinned staging.  Under stream capture the upload
+    // becomes a graph node that reads the staging at every replay (nothing may wait on the device then); otherwise
+    // the staging of the previous call must have been consumed first.
+    const bool staged = n > kClearTargets;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     DTV_HIP(hipStreamIsCapturing(s, &capture));
     const bool capturing = capture != hipStreamCaptureStatusNone;
-    if (view->targets_pending && !capturing) DTV_HIP(hipEventSynchronize(view->targets_copied));
-    view->targets_pending = false;
-    if (view->pinned_targets_cap < n) {
-        if (view->pinnedTargets) DTV_HIP(hipHostFree(view->pinnedTargets));
-        view->pinnedTargets = nullptr;
-        view->pinned_targets_cap = 0;
-        DTV_HIP(hipHostMalloc((void**)&view->pinnedTargets, sizeof(AdjointTarget) * (size_t)n, hipHostMallocDefault));
-        view->pinned_targets_cap = n;
+    if (staged) {
+        if (!view->targets_copied) DTV_HIP(hipEventCreateWithFlags(&view->targets_copied, hipEventDisableTiming));
+        if (view->targets_pending && !capturing) DTV_HIP(hipEventSynchronize(view->targets_copied));
+        view->targets_pending = false;
+        if (view->pinned_targets_cap < n) {
+            if (view->pinnedTargets) DTV_HIP(hipHostFree(view->pinnedTargets));
+            view->pinnedTargets = nullptr;
+            view->pinned_targets_cap = 0;
+            DTV_HIP(hipHostMalloc((void**)&view->pinnedTargets, sizeof(AdjointTarget) * (size_t)n,
+                                  hipHostMallocDefault));
+            view->pinned_targets_cap = n;
+        }
     }
+    std::vector<AdjointTarget> targets(tg, tg + n);
+    ClearList clear;
     // Each distinct gradient target (the items of one mesh share theirs) accumulates its vertex gradients in
     // zeroed interleaved rows (8 floats per vertex), folded into its gradients after the adjoint.
     struct Fold {
@@ -601,7 +613,6 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         float* grad_col;
     };
     std::vector<Fold> folds;
-    std::memcpy(view->pinnedTargets, tg, sizeof(AdjointTarget) * (size_t)n);
     {
         std::unordered_map<const float*, int> first;  // grad_pos -> first item
         std::vector<int64_t> row0((size_t)n, -1);
@@ -632,22 +643,27 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
             r += fo.V;
         }
         for (int i = 0; i < n; i++)
-            view->pinnedTargets[i].acc = row0[(size_t)i] >= 0 ? base + 8 * row0[(size_t)i] : nullptr;
-        if (rows > 0) fill_u32(reinterpret_cast<uint32_t*>(base), 0u, 8 * rows, s);
+            targets[(size_t)i].acc = row0[(size_t)i] >= 0 ? base + 8 * row0[(size_t)i] : nullptr;
+        clear.add(base, 8 * rows);
     }
     DTV_HIP(view->dTargets.ensure(sizeof(AdjointTarget) * (size_t)n));
-    DTV_HIP(hipMemcpyAsync(view->dTargets.p, view->pinnedTargets, sizeof(AdjointTarget) * (size_t)n,
-                           hipMemcpyHostToDevice, s));
-    if (!capturing) {
-        DTV_HIP(hipEventRecord(view->targets_copied, s));
-        view->targets_pending = true;
+    if (staged) {
+        std::memcpy(view->pinnedTargets, targets.data(), sizeof(AdjointTarget) * (size_t)n);
+        DTV_HIP(hipMemcpyAsync(view->dTargets.p, view->pinnedTargets, sizeof(AdjointTarget) * (size_t)n,
+                               hipMemcpyHostToDevice, s));
+        if (!capturing) {
+            DTV_HIP(hipEventRecord(view->targets_copied, s));
+            view->targets_pending = true;
+        }
     }
     PixelState ps = view->pixel_state();
     view->atomics_counted = view->timing;
     if (view->timing) {  // count the gradient atomics along with the stage timers
-        ps.counters = reinterpret_cast<unsigned long long*>(view->small.as<char>() + 256);
-        fill_u32(reinterpret_cast<uint32_t*>(ps.counters), 0u, 2, s);
+        ps.counters = &view->scratch()->atomics;
+        clear.add(ps.counters, 2);
     }
+    launch_clear(clear, nullptr, nullptr, targets.data(), staged ? 0 : n,
+                 staged ? nullptr : view->dTargets.as<AdjointTarget>(), s);
     // adjoint launch order: tiles by the forward's composited fragments, heaviest first
     const uint32_t* adj_order = nullptr;
     if (view->cost_ordered) {
@@ -661,11 +677,11 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         DTV_HIP(view->tri_grad.ensure(sizeof(float) * (size_t)(tg_floats > 0 ? tg_floats : 1)));
         launch_pt_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n, view->total_tiles,
                           view->total_blocks, adj_order, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
-                          view->pt_col.as<float4>(), view->sorted_recs(), view->ranges.as<uint2>(), ps,
+                          view->pt_col.as<float4>(), view->stream(), view->ranges.as<uint2>(), ps,
                           view->tri_grad.as<float>(), tg_floats, use_abs_grad ? 1 : 0, s);
     } else {
         launch_render_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n,
-                              view->total_subtiles, adj_order, view->sorted_recs(), view->ranges.as<uint2>(), ps,
+                              view->total_subtiles, adj_order, view->stream(), view->ranges.as<uint2>(), ps,
                               use_abs_grad ? 1 : 0, adjoint_mode, view->colour_kinds, s, view->sub_tiles,
                               view->queued ? view->tile_queue() : nullptr, view->edge);
     }
@@ -721,7 +737,7 @@ int dtv_view_create(dtv_ctx* ctx, dtv_view** out_view) {
     DTV_HIP(hipSetDevice(ctx->device));
     dtv_view* v = new dtv_view();
     v->ctx = ctx;
-    hipError_t e = hipHostMalloc((void**)&v->pinnedStats, sizeof(BinStats) + 16, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc((void**)&v->pinnedStats, sizeof(ViewScratch), hipHostMallocDefault);
     if (e != hipSuccess) {
         delete v;
         return fail(DTV_ERR_HIP, std::string("dtv_view_create: hipHostMalloc: ") + hipGetErrorString(e));
@@ -734,9 +750,8 @@ int dtv_view_destroy(dtv_view* v) {
     if (!v) return DTV_OK;
     (void)hipSetDevice(v->ctx->device);
     (void)hipDeviceSynchronize();
-    DevBuf* bufs[] = {&v->dItems, &v->dTargets, &v->counts, &v->offsets, &v->scan_status, &v->small, &v->block_stats, &v->keys,
-                      &v->vals, &v->keys2,
-                      &v->vals2, &v->recs, &v->hist, &v->lookback, &v->ranges, &v->ray_color, &v->frag_count, &v->last_rec,
+    DevBuf* bufs[] = {&v->dItems, &v->dTargets, &v->bin_status, &v->small, &v->keys, &v->vals, &v->keys2, &v->vals2,
+                      &v->recs, &v->hist, &v->lookback, &v->ranges, &v->ray_color, &v->frag_count, &v->last_rec,
                       &v->num_ckpt, &v->ckpt_t, &v->ckpt_n, &v->tile_frags, &v->tile_order, &v->pt_info,
                       &v->pt_vert, &v->pt_col, &v->tri_grad, &v->vacc};
     for (DevBuf* b : bufs) b->release();
@@ -810,15 +825,10 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
     B.tile0 = 0;
     B.sub0 = 0;
     B.pixel0 = 0;
-    const int64_t blocks = count_pairs_blocks(m.num_cells);
-    const int64_t nslots = 256 * (blocks > 0 ? blocks : 1);
+    const int64_t blocks = bin_blocks(m.num_cells);
     const int64_t K = kNaMaxRecords;
-    int tile_bits = 0;
-    while ((1ll << tile_bits) < tiles) tile_bits++;
-    uint32_t mask = 0xFu;  // every depth digit: which of them vary is known only on the device
-    for (int p = 0; 8 * p < tile_bits; p++) mask |= 1u << (4 + p);
-    int npass = 0;
-    for (int p = 0; p < 8; p++) npass += (mask >> p) & 1;
+    int tbits = 0;
+    while ((1ll << tbits) < tiles) tbits++;
     // carve the scratch (256-byte aligned pieces)
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -826,11 +836,11 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
         off += (bytes + 255) & ~(size_t)255;
         return o;
     };
-    const size_t o_item = take(sizeof(BatchItem)), o_small = take(384), o_counts = take(4 * (size_t)nslots),
-                 o_offsets = take(4 * (size_t)nslots), o_status = take(8 * (size_t)(scan_partitions(nslots) + 1)),
-                 o_bstats = take(16 * (size_t)(blocks + 1)), o_keys = take(8 * (size_t)K), o_keys2 = take(8 * (size_t)K),
+    const size_t o_item = take(sizeof(BatchItem)), o_small = take(sizeof(ViewScratch)),
+                 o_status = take(8 * (size_t)bin_status_words(blocks)), o_keys = take(8 * (size_t)K), o_keys2 = take(8 * (size_t)K),
                  o_vals = take(4 * (size_t)K), o_vals2 = take(4 * (size_t)K), o_recs = take(32 * (size_t)K),
-                 o_hist = take(4 * 8 * 256 + 64), o_lookback = take(4 * 256 * (size_t)npass * (sort_partitions(K) + 1)),
+                 o_hist = take(4 * (8 * 256 + 8)),
+                 o_lookback = take(4 * (size_t)sort_lookback_words(K, sort_max_passes(tbits))),
                  o_ranges = take(8 * (size_t)tiles), o_tfrags = take(4 * (size_t)tiles), o_order = take(4 * (size_t)tiles),
                  o_color = take(16 * (size_t)P), o_count = take(4 * (size_t)P), o_last = take(4 * (size_t)P),
                  o_nck = take(4 * (size_t)P);
@@ -840,32 +850,27 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
     if (!base) return fail(DTV_ERR_HIP, f + ": scratch not set up on this device");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     BatchItem* dI = reinterpret_cast<BatchItem*>(base + o_item);
-    char* small = base + o_small;
-    uint32_t* scan_counter = reinterpret_cast<uint32_t*>(small + 64);
-    uint64_t* scan_total = reinterpret_cast<uint64_t*>(small + 128);
-    uint32_t* overflow = reinterpret_cast<uint32_t*>(small + 192);
-    SortRoute* route = reinterpret_cast<SortRoute*>(small + 320);
-    uint32_t* counts = reinterpret_cast<uint32_t*>(base + o_counts);
+    ViewScratch* scratch = reinterpret_cast<ViewScratch*>(base + o_small);
+    uint32_t* overflow = &scratch->overflow;
     uint32_t* hist = reinterpret_cast<uint32_t*>(base + o_hist);
     uint2* ranges = reinterpret_cast<uint2*>(base + o_ranges);
     const int edge = wave_edge(*params, tiles);
     uint32_t* order = params->tile_order == 0 && edge == 8 ? reinterpret_cast<uint32_t*>(base + o_order) : nullptr;
-    uint4* recs = reinterpret_cast<uint4*>(base + o_recs);
-    // the item reaches the device as a kernel argument: no host staging
-    hipLaunchKernelGGL(k_store_item, dim3(1), dim3(1), 0, s, B, dI);
-    launch_count_pairs(dI, 1, blocks, counts, reinterpret_cast<uint32_t*>(base + o_bstats), s);
-    scan_exclusive_u32(counts, reinterpret_cast<uint32_t*>(base + o_offsets), 256 * blocks,
-                       reinterpret_cast<uint64_t*>(base + o_status), scan_counter, scan_total, s);
-    fill_u32(overflow, 0u, 1, s);
-    launch_emit_pairs(dI, 1, blocks, reinterpret_cast<uint32_t*>(base + o_offsets), counts,
-                      reinterpret_cast<uint64_t*>(base + o_keys), reinterpret_cast<uint32_t*>(base + o_vals), K,
-                      overflow, s);
-    radix_sort_pairs(reinterpret_cast<uint64_t*>(base + o_keys), reinterpret_cast<uint32_t*>(base + o_vals),
-                     reinterpret_cast<uint64_t*>(base + o_keys2), reinterpret_cast<uint32_t*>(base + o_vals2), K,
-                     scan_total, mask, hist, reinterpret_cast<uint32_t*>(base + o_lookback), hist + 8 * 256, route, s);
-    launch_tile_ranges(route, K, scan_total, tiles, ranges, s);
+    const RecordStream recs{reinterpret_cast<uint4*>(base + o_recs), &scratch->route};
+    ClearList clear;
+    clear.add(base + o_status, 2 * bin_status_words(blocks));
+    clear.add(scratch, (int64_t)(offsetof(ViewScratch, cleared) / 4));
+    clear.add(hist, 8 * 256 + 8);
+    clear.add(ranges, 2 * tiles);
+    launch_clear(clear, &B, dI, nullptr, 0, nullptr, s);  // the item reaches the device as a kernel argument
+    const BinOut out{reinterpret_cast<uint64_t*>(base + o_status), scratch, reinterpret_cast<uint64_t*>(base + o_keys),
+                     reinterpret_cast<uint4*>(base + o_recs), (uint64_t)K};
+    launch_bin(dI, 1, blocks, bin_small(m.num_cells, P), out, s);
+    const SortInput in{out.keys, reinterpret_cast<uint64_t*>(base + o_keys2), reinterpret_cast<uint32_t*>(base + o_vals),
+                       reinterpret_cast<uint32_t*>(base + o_vals2), K, &scratch->total, scratch->slots, 0u, 0, tbits};
+    sort_records(in, hist, hist + 8 * 256, reinterpret_cast<uint32_t*>(base + o_lookback), &scratch->route, s);
+    launch_tile_ranges(&scratch->route, K, &scratch->total, ranges, edge < 8 ? recs.recs : nullptr, s);
     if (order) launch_tile_order(ranges, nullptr, tiles, order, s);
-    launch_gather_records(dI, 1, route, K, scan_total, recs, s);
     PixelState ps;
     ps.ray_color = reinterpret_cast<float4*>(base + o_color);
     ps.frag_count = reinterpret_cast<uint32_t*>(base + o_count);
@@ -1031,7 +1036,7 @@ int dtv_view_export_fragments(dtv_view* view, const dtv_mesh* mesh, int32_t max_
         return fail(DTV_ERR_INVALID_ARGUMENT, "dtv_view_export_fragments: mesh differs from the rendered one");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     DTV_HIP(hipSetDevice(view->ctx->device));
-    launch_export_fragments(view->dItems.as<BatchItem>(), view->nitems(), view->total_subtiles, view->sorted_recs(),
+    launch_export_fragments(view->dItems.as<BatchItem>(), view->nitems(), view->total_subtiles, view->stream(),
                             view->ranges.as<uint2>(), view->pixel_state(), max_per_pixel, out_ids, s);
     DTV_HIP(hipGetLastError());
     return DTV_OK;
@@ -1049,12 +1054,12 @@ int dtv_view_records_overflowed(dtv_view* view, int32_t* out_overflowed, int64_t
     if (!view->rendered) return fail(DTV_ERR_NOT_RENDERED, "dtv_view_records_overflowed: view has not been rendered");
     DTV_HIP(hipSetDevice(view->ctx->device));
     DTV_HIP(hipDeviceSynchronize());
-    uint64_t total = 0;
-    DTV_HIP(hipMemcpy(&total, view->small.as<char>() + 128, sizeof(total), hipMemcpyDeviceToHost));
-    BinStats st{};
+    ViewScratch st;
     DTV_HIP(hipMemcpy(&st, view->small.p, sizeof(st), hipMemcpyDeviceToHost));
+    const uint64_t total = st.total;
     view->num_pairs = (int64_t)total;
-    view->num_tris = st.num_tris;
+    view->num_tris = 0;
+    for (const BinSlot& b : st.slots) view->num_tris += b.tris;
     const int64_t cap = view->planned_cap > 0 ? view->planned_cap : (int64_t)total;
     *out_overflowed = (int64_t)total > cap ? 1 : 0;
     if (out_records) *out_records = (int64_t)total;
@@ -1081,7 +1086,7 @@ int dtv_view_get_stats(dtv_view* view, dtv_view_stats* out) {
         DTV_HIP(hipSetDevice(view->ctx->device));
         DTV_HIP(hipDeviceSynchronize());
         unsigned long long c = 0;
-        DTV_HIP(hipMemcpy(&c, view->small.as<char>() + 256, sizeof(c), hipMemcpyDeviceToHost));
+        DTV_HIP(hipMemcpy(&c, &view->scratch()->atomics, sizeof(c), hipMemcpyDeviceToHost));
         out->num_gradient_atomics = (int64_t)c;
     }
     return DTV_OK;

@@ -2,142 +2,65 @@
 //
 // Replaces GenerateTrianglesIntersect.glsl:74-132 (per-tet projection + front faces, one atomic append each),
 // ComputeTriangleDepths.glsl:72-110 (centroid-depth keys) and the rasteriser's fragment generation.  Each front
-// face becomes one (tile, face) record per 8x8 screen tile of its pixel-centre bounding box that the face's edge
-// functions do not exclude (tile_may_cover), keyed by (tile << 32 | depth-key bits).  Counting and emission are
-// two passes over the tets separated by a device-wide scan, so records are written in (tet, face, tile) order
-// and the stable sort keeps that order for equal depth keys.  The sort moves face ids; k_gather_records then
-// lays the sorted records out for the tile renderer as {face id, exact 64-bit coverage mask of the tile}
-// (one thread per record, so the per-pixel edge tests are spread evenly over the GPU).
-#include "dtv_kernels.h"
-#include "dtv_prims.h"
-#include "raster.h"
+// face becomes one (tile, face) record per 8x8 screen tile with a pixel centre it covers, keyed by
+// (tile << 32 | depth-key bits), with the exact 64-bit coverage mask of the tile (bin_block.h).  Records are
+// written in (tet, face, tile) order and the stable sort keeps that order for equal depth keys.  The sort moves
+// record indices; the tile renderers read the records through them.
+#include "bin_block.h"
 
 namespace dtv {
 
-// One thread per tet slot of the batch's block grid; counts[slot] = records of the tet (all its faces).
-__global__ __launch_bounds__(256) void k_count_pairs(const BatchItem* __restrict__ items, int nitems,
-                                                      uint32_t* __restrict__ counts, uint4* __restrict__ block_stats) {
-    const BatchItem& B = items[item_of_block(items, nitems, blockIdx.x)];
+// One workgroup per kTets tets of the batch's block grid.
+template <int kTets>
+__global__ __launch_bounds__(kBinBlock) void k_bin(const BatchItem* __restrict__ items, int nitems, BinOut out) {
+    __shared__ BinLds<kTets> L;
+    const uint32_t part = bin_ticket(L, out.scratch);
+    const BatchItem& B = items[item_of_block(items, nitems, part / (kBinUnit / kTets))];
     const ViewUniforms& U = B.U;
-    const int64_t tet = (int64_t)(blockIdx.x - B.block0) * 256 + threadIdx.x;
-    uint32_t c = 0, ntri = 0, kand = 0xFFFFFFFFu, kor = 0u;
-    if (tet < B.T) {
-        ProjectedTet PT;
-        project_tet(U, B.cells, B.pos, tet, PT);
-        if (!PT.culled) {
-#pragma unroll
-            for (int f = 0; f < 4; f++) {
-                if (!(PT.visible & (1u << f))) continue;
-                ntri++;
-                const FaceBins b = face_bins(U, PT, f);
-                const uint32_t cf = face_record_count(b);
-                c += cf;
-                if (cf) {
-                    uint32_t k = face_key(PT, f);
-                    kand &= k;
-                    kor |= k;
-                }
-            }
-        }
-    }
-    counts[(int64_t)blockIdx.x * 256 + threadIdx.x] = c;
-    // Per-block partials (no global atomics: one address hit by every wave serialises at the memory side).
-    __shared__ uint4 s_part[4];
-    const uint32_t wtri = wave_sum_u32(ntri);
-    const uint32_t wand = wave_and_u32(kand);
-    const uint32_t wor = wave_or_u32(kor);
-    if (lane_id() == 0) s_part[threadIdx.x / 64] = make_uint4(wtri, wand, wor, 0u);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint4 r = s_part[0];
-        for (int w = 1; w < (int)(blockDim.x / 64); w++) {
-            r.x += s_part[w].x;
-            r.y &= s_part[w].y;
-            r.z |= s_part[w].z;
-        }
-        block_stats[blockIdx.x] = r;
-    }
-}
-
-// Reduces the per-block partials of k_count_pairs; the record total comes from the scan.
-__global__ __launch_bounds__(256) void k_reduce_bin_stats(const uint4* __restrict__ block_stats, int64_t nblocks,
-                                                           const uint64_t* __restrict__ scan_total,
-                                                           BinStats* __restrict__ stats) {
-    __shared__ uint4 s_part[4];
-    uint32_t ntri = 0, kand = 0xFFFFFFFFu, kor = 0u;
-    for (int64_t i = threadIdx.x; i < nblocks; i += blockDim.x) {
-        const uint4 b = block_stats[i];
-        ntri += b.x;
-        kand &= b.y;
-        kor |= b.z;
-    }
-    const uint32_t wtri = wave_sum_u32(ntri), wand = wave_and_u32(kand), wor = wave_or_u32(kor);
-    if (lane_id() == 0) s_part[threadIdx.x / 64] = make_uint4(wtri, wand, wor, 0u);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint4 r = s_part[0];
-        for (int w = 1; w < 4; w++) {
-            r.x += s_part[w].x;
-            r.y &= s_part[w].y;
-            r.z |= s_part[w].z;
-        }
-        stats->total_pairs = *scan_total;
-        stats->num_tris = r.x;
-        stats->key_and = r.y;
-        stats->key_or = r.z;
-    }
-}
-
-// Same grid as k_count_pairs: writes the tet's records at offsets[slot], faces in order, tiles row-major.
-// keys/vals are the sort input, vals = the record's face id tet * 4 + face (the stable sort keeps equal keys in
-// emit order, so the payload need not encode it).
-// Records at index >= cap (the capacity of keys/vals) are not written; *overflow is then set to 1.
-__global__ __launch_bounds__(256) void k_emit_pairs(const BatchItem* __restrict__ items, int nitems,
-                                                     const uint32_t* __restrict__ offsets,
-                                                     const uint32_t* __restrict__ counts,
-                                                     uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                     uint64_t cap, uint32_t* __restrict__ overflow) {
-    const BatchItem& B = items[item_of_block(items, nitems, blockIdx.x)];
-    const ViewUniforms& U = B.U;
-    const int64_t tet = (int64_t)(blockIdx.x - B.block0) * 256 + threadIdx.x;
-    if (tet >= B.T) return;
-    const int64_t slot = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    uint32_t left = counts[slot];
-    if (left == 0) return;
-    uint32_t o = offsets[slot];
+    const int64_t tet = (int64_t)part * kTets - (int64_t)B.block0 * kBinUnit + threadIdx.x;
     ProjectedTet PT;
-    project_tet(U, B.cells, B.pos, tet, PT);
+    PT.culled = true;
+    PT.visible = 0;
+    if (threadIdx.x < kTets && tet < B.T) project_tet(U, B.cells, B.pos, tet, PT);
+    const uint32_t visible = PT.culled ? 0u : PT.visible;
+    uint32_t nfaces;
+    uint32_t e = block_exclusive_scan<kBinBlock>((uint32_t)__popc(visible), L.tmp, nfaces);
+    uint32_t kmin = 0xFFFFFFFFu, kmax = 0u;
+    if (visible)
+#pragma unroll
+        for (int v = 0; v < 4; v++) bin_vertex(U, L, v, PT.ndc[v][0], PT.ndc[v][1]);
 #pragma unroll
     for (int f = 0; f < 4; f++) {
-        if (!(PT.visible & (1u << f)) || left == 0) continue;
-        const FaceBins b = face_bins(U, PT, f);
-        const uint64_t k = (uint64_t)face_key(PT, f);
-        const uint32_t id = (uint32_t)(tet * 4 + f);
-        const bool test = test_tiles(b);
-        // Bounded by the stored count: the pass recomputes the same records, but never writes past its slots.
-        for (int ty = b.ty0; ty <= b.ty1 && left > 0; ty++)
-            for (int tx = b.tx0; tx <= b.tx1 && left > 0; tx++) {
-                if (test && !tile_may_cover(b.S, tx, ty, b.shift)) continue;
-                if (o < cap) {
-                    keys[o] = ((uint64_t)(B.tile0 + (uint32_t)(ty * U.tiles_x + tx)) << 32) | k;
-                    vals[o] = id;
-                } else {
-                    *overflow = 1u;
-                }
-                o++;
-                left--;
-            }
+        if (!(visible & (1u << f))) continue;
+        const uint32_t k = face_key(PT, f);
+        if (bin_entry(U, L, e, (uint32_t)f, kFaceTable[f][0], kFaceTable[f][1], kFaceTable[f][2], k, 0u)) {
+            kmin = min(kmin, k);
+            kmax = max(kmax, k);
+        }
+        e++;
     }
+    bin_stats(out.scratch, part, (uint32_t)__popc(visible), kmin, kmax);
+    bin_emit<true>(B, L, nfaces, part, gridDim.x, out);
 }
 
-__global__ void k_tile_ranges(const SortRoute* __restrict__ route, int64_t n_cap, const uint64_t* __restrict__ n_dev,
-                              uint2* __restrict__ ranges) {
-    const uint64_t* __restrict__ keys = route->keys_out;
+// ranges[t] = the sorted records of tile t; masks (kMasks): their coverage masks in sorted order.
+template <bool kMasks>
+__global__ __launch_bounds__(256) void k_tile_ranges(const SortRoute* __restrict__ route, int64_t n_cap,
+                                                     const uint64_t* __restrict__ n_dev, uint2* __restrict__ ranges,
+                                                     const uint4* __restrict__ recs) {
+    const uint32_t* __restrict__ keys = route->keys;
+    const uint32_t* __restrict__ vals = route->vals;
+    uint2* __restrict__ masks = route->masks;
+    const uint32_t shift = route->tile_shift;
     const int64_t n = run_count(n_cap, n_dev);
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t t = (uint32_t)(keys[i] >> 32);
-        if (i == 0 || (uint32_t)(keys[i - 1] >> 32) != t) ranges[t].x = (uint32_t)i;
-        if (i == n - 1 || (uint32_t)(keys[i + 1] >> 32) != t) ranges[t].y = (uint32_t)(i + 1);
+        const uint32_t t = keys[i] >> shift;
+        if (i == 0 || keys[i - 1] >> shift != t) ranges[t].x = (uint32_t)i;
+        if (i == n - 1 || keys[i + 1] >> shift != t) ranges[t].y = (uint32_t)(i + 1);
+        if constexpr (kMasks) {
+            const uint4 r = recs[2 * (int64_t)vals[i] + 1];
+            masks[i] = make_uint2(r.y, r.z);
+        }
     }
 }
 
@@ -152,21 +75,23 @@ __device__ __forceinline__ uint32_t cost_bucket(uint32_t c) {
     return 8u * (uint32_t)e + m;
 }
 
-// The lanes of the wave whose bucket equals this lane's (eq, live lanes only) and this lane's rank among them.
-// Every lane of the wave must take part.
-__device__ __forceinline__ void bucket_match(bool live, uint32_t b, uint64_t& eq, uint32_t& rank) {
-    eq = ballot(live);
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const uint64_t bk = ballot(((b >> k) & 1u) != 0u);
-        eq &= ((b >> k) & 1u) ? bk : ~bk;
-    }
-    rank = (uint32_t)popc64(eq & lanemask_lt());
-}
-
 // Tiles per thread per step: their costs are loaded together, so the loads overlap (one step per pass up to
 // 16K tiles, a 1024x1024 view).
 constexpr int kOrderPer = 16;
+
+// Adds one to counter[b] for every live lane and returns the count before it.  Tiles without cost share one bucket
+// and are many, so their lanes are added together (LDS atomics on one address serialise); the others spread over
+// the buckets.  Every lane of the wave must take part.
+__device__ __forceinline__ uint32_t bucket_add(uint32_t* counter, bool live, uint32_t b) {
+    const bool empty = live && b == 0u;
+    const uint64_t m = ballot(empty);
+    const uint32_t below = (uint32_t)popc64(m & lanemask_lt());
+    uint32_t at = 0u;
+    if (live && (!empty || below == 0u)) at = atomicAdd(&counter[b], empty ? (uint32_t)popc64(m) : 1u);
+    const int leader = m != 0ull ? __builtin_ctzll(m) : 0;
+    const uint32_t at0 = (uint32_t)__shfl((int)at, leader, 64);
+    return empty ? at0 + below : at;
+}
 
 __device__ __forceinline__ void load_buckets(const uint2* __restrict__ ranges, const uint32_t* __restrict__ cost,
                                              uint32_t i0, uint32_t n, uint32_t b[kOrderPer]) {
@@ -194,11 +119,8 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint2* __restrict__ r
         load_buckets(ranges, cost, i0, n, b);
 #pragma unroll
         for (int q = 0; q < kOrderPer; q++) {
-            const bool live = i0 + 1024u * q + t < n;
-            uint64_t eq;
-            uint32_t rank;
-            bucket_match(live, b[q], eq, rank);
-            if (live && rank == 0u) atomicAdd(&count[b[q]], (uint32_t)popc64(eq));
+            if (i0 + 1024u * q >= n) break;  // uniform
+            (void)bucket_add(count, i0 + 1024u * q + t < n, b[q]);
         }
     }
     __syncthreads();
@@ -218,53 +140,17 @@ __global__ __launch_bounds__(1024) void k_tile_order(const uint2* __restrict__ r
         }
     }
     __syncthreads();
-    const int lane = (int)(t & 63u);
     for (uint32_t i0 = 0; i0 < n; i0 += 1024u * kOrderPer) {
         uint32_t b[kOrderPer];
         load_buckets(ranges, cost, i0, n, b);
 #pragma unroll
         for (int q = 0; q < kOrderPer; q++) {
+            if (i0 + 1024u * q >= n) break;  // uniform
             const uint32_t i = i0 + 1024u * q + t;
-            const bool live = i < n;
-            uint64_t eq;
-            uint32_t rank;
-            bucket_match(live, b[q], eq, rank);
-            uint32_t base = 0u;
-            if (live && rank == 0u) base = atomicAdd(&start[b[q]], (uint32_t)popc64(eq));
-            const int leader = eq != 0ull ? __ffsll((unsigned long long)eq) - 1 : lane;
-            base = __shfl(base, leader, 64);
-            if (live) order[base + rank] = i;
+            const uint32_t at = bucket_add(start, i < n, b[q]);
+            if (i < n) order[at] = i;
         }
     }
-}
-
-// Sorted record i = out[2i], out[2i + 1] = {the tet's 4 vertex indices}, {face id, coverage mask low, high, 0}:
-// the face sorted_ids[i] is projected again (the same arithmetic as binning) and its exact coverage of the
-// record's tile computed.  Carrying the vertex indices saves the renderer one dependent load per record.
-__global__ __launch_bounds__(256) void k_gather_records(const BatchItem* __restrict__ items, int nitems,
-                                                         const SortRoute* __restrict__ route, int64_t n_cap,
-                                                         const uint64_t* __restrict__ n_dev,
-                                                         uint4* __restrict__ out) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= run_count(n_cap, n_dev)) return;
-    const uint64_t* __restrict__ sorted_keys = route->keys_out;
-    const uint32_t* __restrict__ sorted_ids = route->vals_out;
-    const uint32_t id = sorted_ids[i];
-    const uint32_t gtile = (uint32_t)(sorted_keys[i] >> 32);
-    const BatchItem& B = items[item_of_tile(items, nitems, gtile)];
-    const ViewUniforms& U = B.U;
-    const int tile = (int)(gtile - B.tile0);
-    const int64_t tet = id >> 2;
-    const int4 vid = *reinterpret_cast<const int4*>(B.cells + 4 * tet);
-    ProjectedTet PT;
-    project_face(U, vid, B.pos, (int)(id & 3), PT);  // the tet passed culling when its records were emitted
-    ScreenTri S;
-    face_screen(U, PT, id & 3, S);
-    // larger binning tiles: each 8x8 sub-tile's renderer tests its own pixels (no mask here)
-    const uint64_t m =
-        U.tile_shift == 3 ? tile_coverage(S, tile % U.tiles_x, tile / U.tiles_x, U.width, U.height) : 0ull;
-    out[2 * i] = make_uint4((uint32_t)vid.x, (uint32_t)vid.y, (uint32_t)vid.z, (uint32_t)vid.w);
-    out[2 * i + 1] = make_uint4(id, (uint32_t)m, (uint32_t)(m >> 32), 0u);
 }
 
 // cost[g] = records of the binning tile that holds 8x8 sub-tile g (the forward's launch order for binning tiles
@@ -289,49 +175,40 @@ void launch_subtile_cost(const BatchItem* items, int nitems, int64_t nsub, const
                        ranges, cost);
 }
 
-int64_t count_pairs_blocks(int64_t T) { return T > 0 ? (T + 255) / 256 : 0; }
+int64_t bin_blocks(int64_t T) { return T > 0 ? (T + kBinUnit - 1) / kBinUnit : 0; }
+int64_t bin_status_words(int64_t nblocks) { return 4 * nblocks + 1; }
 
-void launch_count_pairs(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* counts, uint32_t* block_stats,
+// A workgroup of 64 tets keeps all threads busy where a tet has many candidate tiles, and makes more workgroups of a
+// small mesh; of fine meshes it makes too many (a ticket costs about 14 ns).  Measured, 64 / 256 tets, us: 24,576
+// tets at 256^2 43 / 62, ball of 132K tets at 768^2 131 / 201, 196K tets at 1024^2 162 / 242, 1.57M at 2048^2 829 /
+// 1143; 196K at 507x389 103 / 76, 400K-tet ball at 512^2 159 / 151, 1.57M at 1024^2 515 / 402, 16 such views at
+// 512^2 5429 / 3033.
+bool bin_small(int64_t tets, int64_t pixels) { return tets <= 65536 || 4 * pixels >= 5 * tets; }
+
+void launch_bin(const BatchItem* items, int nitems, int64_t nblocks, bool small, const BinOut& out, hipStream_t s) {
+    if (nblocks <= 0) return;
+    if (small)
+        hipLaunchKernelGGL(k_bin<64>, dim3((unsigned)(4 * nblocks)), dim3(kBinBlock), 0, s, items, nitems, out);
+    else
+        hipLaunchKernelGGL(k_bin<256>, dim3((unsigned)nblocks), dim3(kBinBlock), 0, s, items, nitems, out);
+}
+
+void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, uint2* ranges, const uint4* recs,
                         hipStream_t s) {
-    if (nblocks <= 0) return;
-    hipLaunchKernelGGL(k_count_pairs, dim3((unsigned)nblocks), dim3(256), 0, s, items, nitems, counts,
-                       reinterpret_cast<uint4*>(block_stats));
-}
-
-void launch_reduce_bin_stats(const uint32_t* block_stats, int64_t nblocks, const uint64_t* scan_total,
-                             BinStats* stats, hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce_bin_stats, dim3(1), dim3(256), 0, s, reinterpret_cast<const uint4*>(block_stats),
-                       nblocks, scan_total, stats);
-}
-
-void launch_emit_pairs(const BatchItem* items, int nitems, int64_t nblocks, const uint32_t* offsets,
-                       const uint32_t* counts, uint64_t* keys, uint32_t* vals, int64_t cap, uint32_t* overflow,
-                       hipStream_t s) {
-    if (nblocks <= 0) return;
-    hipLaunchKernelGGL(k_emit_pairs, dim3((unsigned)nblocks), dim3(256), 0, s, items, nitems, offsets, counts, keys,
-                       vals, (uint64_t)cap, overflow);
-}
-
-void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, int64_t num_tiles,
-                        uint2* ranges, hipStream_t s) {
-    fill_u32(reinterpret_cast<uint32_t*>(ranges), 0u, 2 * num_tiles, s);
     if (n <= 0) return;
     int64_t blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(k_tile_ranges, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges);
+    if (recs != nullptr)
+        hipLaunchKernelGGL(k_tile_ranges<true>, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges, recs);
+    else
+        hipLaunchKernelGGL(k_tile_ranges<false>, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges,
+                           recs);
 }
 
 void launch_tile_order(const uint2* ranges, const uint32_t* cost, int64_t num_tiles, uint32_t* order,
                        hipStream_t s) {
     if (num_tiles <= 0) return;
     hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, ranges, cost, (uint32_t)num_tiles, order);
-}
-
-void launch_gather_records(const BatchItem* items, int nitems, const SortRoute* route, int64_t n,
-                           const uint64_t* n_dev, uint4* out, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_gather_records, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, items, nitems, route,
-                       n, n_dev, out);
 }
 
 }  // namespace dtv

@@ -11,53 +11,86 @@ namespace dtv {
 
 // sort.hip
 void fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s);
-int64_t scan_partitions(int64_t n);
-void scan_exclusive_u32(const uint32_t* in, uint32_t* out, int64_t n, uint64_t* status, uint32_t* counter,
-                        uint64_t* total, hipStream_t s);
-int64_t sort_partitions(int64_t n);
-// Where the sorted pairs end up, decided on the device: a selected digit that every key shares is skipped
-// (its pass exits at once), so the ping-pong parity is known only there.  pass_src[i]: 0 = pass i reads the
-// first buffers, 1 = the alternates, 2 = skipped.
-struct SortRoute {
-    uint32_t pass_src[8];
-    const uint64_t* keys_out;
-    const uint32_t* vals_out;
+// Zeroes up to kClearRegions word ranges in one launch; a non-NULL item_dst also receives *item, and a non-NULL
+// targets_dst the ntargets (<= kClearTargets) targets, all carried as kernel arguments (no host staging).
+constexpr int kClearRegions = 6, kClearTargets = 8;
+struct ClearList {
+    uint32_t* p[kClearRegions];
+    int64_t n[kClearRegions];  // words
+    int count = 0;
+    void add(void* ptr, int64_t words) {
+        p[count] = static_cast<uint32_t*>(ptr);
+        n[count++] = words;
+    }
 };
-// n_dev (may be NULL): the element count in device memory, clamped to n (the capacity the launches are sized
-// for); NULL sorts exactly n.  route (device) receives the result buffers; returns the passes launched.
-int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, int64_t n,
-                     const uint64_t* n_dev, uint32_t digit_mask, uint32_t* hist, uint32_t* lookback,
-                     uint32_t* counters, SortRoute* route, hipStream_t s);
+void launch_clear(const ClearList& regions, const BatchItem* item, BatchItem* item_dst, const AdjointTarget* targets,
+                  int ntargets, AdjointTarget* targets_dst, hipStream_t s);
 
-// binning.hip
-struct BinStats {
-    uint64_t total_pairs;   // sum of (tile, face) records
-    uint32_t num_tris;      // visible faces
-    uint32_t key_and;       // AND of depth keys of all faces that produce records
-    uint32_t key_or;        // OR of the same keys
+// What one render keeps in a small device buffer.  The words up to `cleared` are zeroed before binning.
+constexpr int kBinSlots = 64;
+struct BinSlot {
+    uint32_t tris;     // visible faces (Projection: triangles)
+    uint32_t not_min;  // complement of the smallest depth key
+    uint32_t max;      // largest depth key
     uint32_t pad;
 };
-int64_t count_pairs_blocks(int64_t T);
-// Grid of nblocks 256-tet blocks over all items (item i owns blocks [block0_i, block0_{i+1})).  counts[256 * nblocks]
-// gets the (tile, face) record count of every tet slot (0 for padding); block_stats the per-block partials.
-void launch_count_pairs(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* counts, uint32_t* block_stats,
+// Where the sort left its result (written by its histogram kernel).
+struct SortRoute {
+    const uint32_t* keys;  // sorted compact keys; tile = key >> tile_shift
+    const uint32_t* vals;  // sorted record indices
+    uint2* masks;          // room for one coverage mask per sorted record
+    uint32_t tile_shift;
+};
+struct ViewScratch {
+    BinSlot slots[kBinSlots];
+    uint64_t total;     // records, written or not
+    uint32_t ticket;
+    uint32_t overflow;  // a record lay beyond the capacity
+    uint32_t cleared;   // (marks the end of the zeroed words)
+    uint32_t queue;     // tile work queue
+    unsigned long long atomics;
+    SortRoute route;
+};
+
+// The records' sort: by tile, then depth key, equal keys in record order.
+struct SortInput {
+    uint64_t* keys;  // [cap] tile << 32 | depth key; overwritten
+    uint64_t* keys2; // [cap]
+    uint32_t* vals;  // [cap]
+    uint32_t* vals2; // [cap]
+    int64_t cap;             // records the launches are sized for
+    const uint64_t* n_dev;   // actual count in device memory, clamped to cap; NULL: cap
+    const BinSlot* slots;    // the depth keys' range in device memory, or NULL: dmin and dbits below
+    uint32_t dmin;           // smallest depth key
+    int dbits;               // bits of the largest depth key minus dmin
+    int tbits;               // bits of a tile number
+};
+int sort_bits(uint32_t range);       // bits of an unsigned number
+int sort_max_passes(int tbits);      // passes at most
+int64_t sort_lookback_words(int64_t cap, int passes);
+// hist: [8 * 256] words and counters: [8] words, zeroed by the caller; lookback: sort_lookback_words.  Returns the
+// passes launched.
+int sort_records(const SortInput& in, uint32_t* hist, uint32_t* counters, uint32_t* lookback, SortRoute* route,
+                 hipStream_t s);
+
+// binning.hip
+int64_t bin_blocks(int64_t T);  // 256-tet blocks
+int64_t bin_status_words(int64_t nblocks);  // look-back words (64 bits) of a launch
+bool bin_small(int64_t tets, int64_t pixels);  // whether workgroups of 64 tets are faster than ones of 256
+struct BinOut {
+    uint64_t* status;      // [bin_status_words(blocks)] look-back words, zeroed
+    ViewScratch* scratch;
+    uint64_t* keys;        // [cap] tile << 32 | depth key
+    uint4* recs;           // [cap] records: two uint4 each (Projection: one)
+    uint64_t cap;
+};
+// Bins the tets of all items (item i owns blocks [block0_i, block0_{i+1}) of 256 tets): scratch->total records, of
+// which those below cap are written, in (tet, face, tile) order.
+void launch_bin(const BatchItem* items, int nitems, int64_t nblocks, bool small, const BinOut& out, hipStream_t s);
+// ranges[t] (zeroed): the sorted records of tile t.  recs (may be NULL): the unsorted records of the tile renderer,
+// whose coverage masks then go to route->masks in sorted order.
+void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, uint2* ranges, const uint4* recs,
                         hipStream_t s);
-// stats.total_pairs = *scan_total; the other fields reduce the per-block partials of launch_count_pairs.
-void launch_reduce_bin_stats(const uint32_t* block_stats, int64_t nblocks, const uint64_t* scan_total,
-                             BinStats* stats, hipStream_t s);
-// keys/vals: sort input, vals = face id (tet * 4 + face) of the record.
-// Writes only records below cap (the buffers' capacity) and sets *overflow = 1 if any record lies beyond.
-void launch_emit_pairs(const BatchItem* items, int nitems, int64_t nblocks, const uint32_t* offsets,
-                       const uint32_t* counts, uint64_t* keys, uint32_t* vals, int64_t cap, uint32_t* overflow,
-                       hipStream_t s);
-// n: capacity the launch is sized for; n_dev (may be NULL): actual count in device memory (see run_count).
-// The sorted keys and face ids are route->keys_out / vals_out (device pointers, set by the sort).
-void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, int64_t num_tiles,
-                        uint2* ranges, hipStream_t s);
-// out[2i], out[2i + 1] = {tet vertex indices}, {face id, 8x8 coverage mask low, high, 0} of sorted record i: the
-// tile renderer's record stream.
-void launch_gather_records(const BatchItem* items, int nitems, const SortRoute* route, int64_t n,
-                           const uint64_t* n_dev, uint4* out, hipStream_t s);
 // cost[g] = record count of the binning tile holding 8x8 sub-tile g, for g < nsub.
 void launch_subtile_cost(const BatchItem* items, int nitems, int64_t nsub, const uint2* ranges, uint32_t* cost,
                          hipStream_t s);
@@ -68,6 +101,11 @@ void launch_tile_order(const uint2* ranges, const uint32_t* cost, int64_t num_ti
                        hipStream_t s);
 
 // render.hip
+// The records in binning order (two uint4 each; Projection one) and the sort's result.
+struct RecordStream {
+    const uint4* recs;
+    const SortRoute* route;
+};
 // Per-pixel state of a rendered batch, concatenated over its items (P = all pixels of the batch); item i's
 // checkpoint planes start at max_ckpt * pixel0_i.
 struct PixelState {
@@ -89,39 +127,35 @@ constexpr uint32_t kColoursPerVertex = 1, kColoursPerCell = 2;
 // sub: the batch bins tiles larger than 8x8 (the kernels then test coverage per 8x8 sub-tile).
 // queue: NULL launches one workgroup per tile; else a persistent grid (the workgroups the GPU holds at once)
 // takes the tiles in launch order from this device counter, which each launch zeroes first.
+// recs: the records in binning order; the sorted order is route->vals.
 // edge: 8, or 4 or 2 for (8 / edge)^2 waves per tile, each rendering edge x edge pixels (128 fragments per round,
 // 8x8 binning tiles, no queue; order is not used).
 void launch_render_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                           const uint4* recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
+                           RecordStream recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
                            hipStream_t s, int round = 128, bool sub = false, uint32_t* queue = nullptr,
                            int edge = 8);
 void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
-                           const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps, int use_abs,
+                           const uint32_t* order, RecordStream recs, const uint2* ranges, PixelState ps, int use_abs,
                            int mode, uint32_t colour_kinds, hipStream_t s, bool sub = false,
                            uint32_t* queue = nullptr, int edge = 8);
 // Adds the tile renderer adjoint's interleaved accumulator rows acc [V][8] into grad_pos [V][3] and, unless
 // NULL, grad_col [V][4].
 void launch_fold_vertex_grads(const float* acc, int64_t V, float* grad_pos, float* grad_col, hipStream_t s);
-void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, const uint4* recs,
+void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
                              const uint2* ranges, PixelState ps, int max_per_pixel, int32_t* out_ids, hipStream_t s);
 
 // proj.hip: the Projection renderer.  Per-tet buffers are indexed by the tet's slot in the batch's block grid
 // (block0 * 256 + tet): pt_info [slots], pt_vert / pt_col [5 * slots] (the five vertices' NDC xyz + thickness,
-// colour); tri_grad [21 * 4 * slots] (the adjoint's per-triangle-corner sums).  Records: recs[2i + 1] =
-// {triangle slot id (tet * 4 + k, item-local tet), coverage mask low, high, 0}.
-void launch_pt_count(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* pt_info, float4* pt_vert,
-                     float4* pt_col, uint32_t* counts, uint32_t* block_stats, hipStream_t s);
-void launch_pt_emit(const BatchItem* items, int nitems, int64_t nblocks, const uint32_t* pt_info,
-                    const float4* pt_vert, const uint32_t* offsets, const uint32_t* counts, uint64_t* keys,
-                    uint32_t* vals, int64_t cap, uint32_t* overflow, hipStream_t s);
-void launch_pt_gather(const BatchItem* items, int nitems, const uint32_t* pt_info, const float4* pt_vert,
-                      const SortRoute* route, int64_t n, const uint64_t* n_dev, uint4* out, hipStream_t s);
+// colour); tri_grad [21 * 4 * slots] (the adjoint's per-triangle-corner sums).  Records: recs[i] =
+// {triangle slot id (tet * 4 + k, item-local tet), coverage mask low, high, corner slots}.
+void launch_pt_bin(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* pt_info, float4* pt_vert,
+                   float4* pt_col, bool small, const BinOut& out, hipStream_t s);
 void launch_pt_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                       const uint32_t* pt_info, const float4* pt_vert, const float4* pt_col, const uint4* recs,
-                       const uint2* ranges, PixelState ps, hipStream_t s);
+                       const float4* pt_vert, const float4* pt_col, RecordStream recs, const uint2* ranges,
+                       PixelState ps, hipStream_t s);
 void launch_pt_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                        int64_t nblocks, const uint32_t* order, const uint32_t* pt_info, const float4* pt_vert,
-                       const float4* pt_col, const uint4* recs, const uint2* ranges, PixelState ps, float* tri_grad,
+                       const float4* pt_col, RecordStream recs, const uint2* ranges, PixelState ps, float* tri_grad,
                        int64_t tri_grad_floats, int use_abs, hipStream_t s);
 
 // optim.hip

@@ -179,6 +179,30 @@ __device__ __forceinline__ uint64_t status_load64(const uint64_t* p) {
     return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Sum of the counts of the parts before `part` in a decoupled look-back, 64 parts at a time; publishes this part's.
+// One full wave calls it; status words (flag in bits 62-63) start at 0, and the parts before `part` are running.
+__device__ __forceinline__ uint64_t lookback_sum(uint64_t* status, uint32_t part, uint64_t count) {
+    constexpr uint64_t kAgg = 1ull << 62, kInc = 2ull << 62, kValue = (1ull << 62) - 1ull;
+    const int lane = lane_id();
+    if (lane == 0) status_store64(&status[part], (part == 0u ? kInc : kAgg) | count);
+    uint64_t before = 0;
+    for (int64_t p = (int64_t)part - 1; p >= 0;) {
+        const int64_t q = p - lane;
+        const uint64_t w = q >= 0 ? status_load64(&status[q]) : kInc;
+        const uint64_t inc = ballot((w & ~kValue) == kInc), none = ballot((w & ~kValue) == 0ull);
+        const int stop = inc != 0ull ? __builtin_ctzll(inc) : 63;  // the nearest part that knows its prefix
+        if (none & (~0ull >> (63 - stop))) continue;                // a part this side of it has not counted yet
+        uint64_t v = lane <= stop ? w & kValue : 0ull;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor((unsigned long long)v, d, 64);
+        before += v;
+        if (inc != 0ull) break;
+        p -= 64;
+    }
+    if (part != 0u && lane == 0) status_store64(&status[part], kInc | (before + count));
+    return before;
+}
+
 __device__ __forceinline__ void atomic_add_f32(float* p, float v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -14,7 +14,7 @@
 // thicknesses (reduce-scatters within rows of 16 lanes, summed per batch in LDS, then one atomic per value into
 // the triangle's slot).  A per-tet pass carries them back through the triangle construction to the vertex
 // positions and colours.
-#include "raster.h"
+#include "bin_block.h"
 #include "render_common.h"
 
 namespace dtv {
@@ -278,186 +278,62 @@ __device__ __forceinline__ void pt_load_tet(const BatchItem& B, int64_t tet, flo
     }
 }
 
-// Corners of triangle k from the tet's five vertices held in registers (selects: a run-time index would place
-// the array in scratch memory).
-__device__ __forceinline__ void pt_tri_corners(const float4 (&pv)[5], const PtDec& D, int k, float4 (&q)[3]) {
-    float x[5], y[5], z[5];
+// Element i of a register array (selects: a run-time index would place the array in scratch memory).
+__device__ __forceinline__ float sel5(const float (&v)[5], int i) {
+    float r = v[0];
 #pragma unroll
-    for (int i = 0; i < 5; i++) {
-        x[i] = pv[i].x;
-        y[i] = pv[i].y;
-        z[i] = pv[i].z;
-    }
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const int v = pt_corner(D, k, j);
-        float rx = x[0], ry = y[0], rz = z[0];
-#pragma unroll
-        for (int i = 1; i < 5; i++) {
-            rx = v == i ? x[i] : rx;
-            ry = v == i ? y[i] : ry;
-            rz = v == i ? z[i] : rz;
-        }
-        q[j] = make_float4(rx, ry, rz, 0.f);  // pt_screen reads x, y, z
-    }
+    for (int k = 1; k < 5; k++) r = i == k ? v[k] : r;
+    return r;
 }
 
-// Fixed-point screen triangle (oriented to positive area) and centroid key of the triangle with corners qc
-// (NDC x, y, z).
-__device__ __forceinline__ void pt_screen(const ViewUniforms& U, const float4 (&qc)[3], ScreenTri& S, uint32_t& key) {
-    const float hw = 0.5f * (float)U.width, hh = 0.5f * (float)U.height;
-    float z[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const float4 q = qc[j];
-        const float xf = q.x * hw + hw;
-        const float yf = q.y * hh + hh;
-        S.X[j] = (int32_t)rintf(xf * 256.0f);
-        S.Y[j] = (int32_t)rintf(yf * 256.0f);
-        z[j] = q.z;
-    }
-    key = __float_as_uint(((z[0] + z[1]) + z[2]) / 3.0f);
-    int64_t area = (int64_t)(S.X[1] - S.X[0]) * (S.Y[2] - S.Y[0]) - (int64_t)(S.Y[1] - S.Y[0]) * (S.X[2] - S.X[0]);
-    if (area < 0) {
-        const int32_t tx = S.X[1], ty = S.Y[1];
-        S.X[1] = S.X[2];
-        S.Y[1] = S.Y[2];
-        S.X[2] = tx;
-        S.Y[2] = ty;
-        area = -area;
-    }
-    S.area2 = area;
-}
-
-// One thread per tet slot: decisions, the five vertices, and the record count of its triangles.
-__global__ __launch_bounds__(256) void k_pt_count(const BatchItem* __restrict__ items, int nitems,
-                                                   uint32_t* __restrict__ pt_info, float4* __restrict__ pt_vert,
-                                                   float4* __restrict__ pt_col, uint32_t* __restrict__ counts,
-                                                   uint4* __restrict__ block_stats) {
-    const BatchItem& B = items[item_of_block(items, nitems, blockIdx.x)];
+// One workgroup per kTets tets, a thread per tet: decisions and the five vertices; then the block's (tile, triangle)
+// records (bin_block.h), {triangle id, coverage mask low, high, corner slots}; corner slots: the tet's vertex slot
+// (0-4) of triangle corner j in bits 3 j .. 3 j + 2.
+template <int kTets>
+__global__ __launch_bounds__(kBinBlock) void k_pt_bin(const BatchItem* __restrict__ items, int nitems,
+                                                      uint32_t* __restrict__ pt_info, float4* __restrict__ pt_vert,
+                                                      float4* __restrict__ pt_col, BinOut out) {
+    __shared__ BinLds<kTets> L;
+    const uint32_t part = bin_ticket(L, out.scratch);
+    const BatchItem& B = items[item_of_block(items, nitems, part / (kBinUnit / kTets))];
     const ViewUniforms& U = B.U;
-    const int64_t tet = (int64_t)(blockIdx.x - B.block0) * 256 + threadIdx.x;
-    uint32_t c = 0, ntri = 0, kand = 0xFFFFFFFFu, kor = 0u;
-    if (tet < B.T) {
+    const int64_t tet = (int64_t)part * kTets - (int64_t)B.block0 * kBinUnit + threadIdx.x;
+    PtDec D{};
+    float z[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    if (threadIdx.x < kTets && tet < B.T) {
         float P[4][3], C[4][4];
         int32_t vid[4];
         pt_load_tet(B, tet, P, C, vid);
-        const PtDec D = pt_decide(U, P);
-        const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;  // the tet's slot in the batch
+        D = pt_decide(U, P);
+        const int64_t g = (int64_t)part * kTets + threadIdx.x;  // the tet's slot in the batch
         pt_info[g] = pt_pack(D);
         if (D.ntri) {
             PtVerts V;
             pt_vertices(D, U, P, C, B.cell_col != nullptr, V);
-            float4 pv[5];
 #pragma unroll
             for (int v = 0; v < 5; v++) {
-                pv[v] = make_float4(V.ndc[v][0], V.ndc[v][1], V.ndc[v][2], V.dep[v]);
-                pt_vert[5 * g + v] = pv[v];
+                z[v] = V.ndc[v][2];
+                bin_vertex(U, L, v, V.ndc[v][0], V.ndc[v][1]);
+                pt_vert[5 * g + v] = make_float4(V.ndc[v][0], V.ndc[v][1], V.ndc[v][2], V.dep[v]);
                 pt_col[5 * g + v] = make_float4(V.col[v][0], V.col[v][1], V.col[v][2], V.col[v][3]);
             }
-            for (int k = 0; k < D.ntri; k++) {
-                ScreenTri S;
-                uint32_t key;
-                float4 q[3];
-                pt_tri_corners(pv, D, k, q);
-                pt_screen(U, q, S, key);
-                const uint32_t cf = face_record_count(screen_bins(U, S));
-                c += cf;
-                ntri++;
-                if (cf) {
-                    kand &= key;
-                    kor |= key;
-                }
-            }
         }
     }
-    counts[(int64_t)blockIdx.x * 256 + threadIdx.x] = c;
-    __shared__ uint4 s_part[4];
-    const uint32_t wtri = wave_sum_u32(ntri), wand = wave_and_u32(kand), wor = wave_or_u32(kor);
-    if (lane_id() == 0) s_part[threadIdx.x / 64] = make_uint4(wtri, wand, wor, 0u);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint4 r = s_part[0];
-        for (int w = 1; w < (int)(blockDim.x / 64); w++) {
-            r.x += s_part[w].x;
-            r.y &= s_part[w].y;
-            r.z |= s_part[w].z;
+    uint32_t ntri;
+    const uint32_t e = block_exclusive_scan<kBinBlock>((uint32_t)D.ntri, L.tmp, ntri);
+    uint32_t kmin = 0xFFFFFFFFu, kmax = 0u;
+    for (int k = 0; k < D.ntri; k++) {
+        const int a = pt_corner(D, k, 0), b = pt_corner(D, k, 1), c = pt_corner(D, k, 2);
+        // centroid key: NDC z of the three corners
+        const uint32_t key = __float_as_uint(((sel5(z, a) + sel5(z, b)) + sel5(z, c)) / 3.0f);
+        const uint32_t slots = (uint32_t)a | ((uint32_t)b << 3) | ((uint32_t)c << 6);
+        if (bin_entry(U, L, e + (uint32_t)k, (uint32_t)k, a, b, c, key, slots)) {
+            kmin = min(kmin, key);
+            kmax = max(kmax, key);
         }
-        block_stats[blockIdx.x] = r;
     }
-}
-
-// Same grid: the tet's records at offsets[slot], triangles in order, tiles row-major; vals = tet * 4 + k.
-__global__ __launch_bounds__(256) void k_pt_emit(const BatchItem* __restrict__ items, int nitems,
-                                                  const uint32_t* __restrict__ pt_info,
-                                                  const float4* __restrict__ pt_vert,
-                                                  const uint32_t* __restrict__ offsets,
-                                                  const uint32_t* __restrict__ counts, uint64_t* __restrict__ keys,
-                                                  uint32_t* __restrict__ vals, uint64_t cap,
-                                                  uint32_t* __restrict__ overflow) {
-    const BatchItem& B = items[item_of_block(items, nitems, blockIdx.x)];
-    const ViewUniforms& U = B.U;
-    const int64_t tet = (int64_t)(blockIdx.x - B.block0) * 256 + threadIdx.x;
-    if (tet >= B.T) return;
-    const int64_t slot = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    uint32_t left = counts[slot];
-    if (left == 0) return;
-    uint32_t o = offsets[slot];
-    const PtDec D = pt_unpack(pt_info[slot]);
-    float4 pv[5];
-#pragma unroll
-    for (int v = 0; v < 5; v++) pv[v] = pt_vert[5 * slot + v];
-    for (int k = 0; k < D.ntri && left > 0; k++) {
-        ScreenTri S;
-        uint32_t key;
-        float4 q[3];
-        pt_tri_corners(pv, D, k, q);
-        pt_screen(U, q, S, key);
-        const FaceBins b = screen_bins(U, S);
-        const bool test = test_tiles(b);
-        const uint32_t id = (uint32_t)(tet * 4 + k);
-        for (int ty = b.ty0; ty <= b.ty1 && left > 0; ty++)
-            for (int tx = b.tx0; tx <= b.tx1 && left > 0; tx++) {
-                if (test && !tile_may_cover(b.S, tx, ty, b.shift)) continue;
-                if (o < cap) {
-                    keys[o] = ((uint64_t)(B.tile0 + (uint32_t)(ty * U.tiles_x + tx)) << 32) | (uint64_t)key;
-                    vals[o] = id;
-                } else {
-                    *overflow = 1u;
-                }
-                o++;
-                left--;
-            }
-    }
-}
-
-// Sorted record i: out[2i + 1] = {triangle id, coverage mask low, high, corner slots} (out[2i] is not used);
-// corner slots: the tet's vertex slot (0-4) of triangle corner j in bits 3 j .. 3 j + 2.
-__global__ __launch_bounds__(256) void k_pt_gather(const BatchItem* __restrict__ items, int nitems,
-                                                    const uint32_t* __restrict__ pt_info,
-                                                    const float4* __restrict__ pt_vert,
-                                                    const SortRoute* __restrict__ route, int64_t n_cap,
-                                                    const uint64_t* __restrict__ n_dev, uint4* __restrict__ out) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= run_count(n_cap, n_dev)) return;
-    const uint32_t id = route->vals_out[i];
-    const uint32_t gtile = (uint32_t)(route->keys_out[i] >> 32);
-    const BatchItem& B = items[item_of_tile(items, nitems, gtile)];
-    const ViewUniforms& U = B.U;
-    const int tile = (int)(gtile - B.tile0);
-    const int64_t g = (int64_t)B.block0 * 256 + (id >> 2);
-    const PtDec D = pt_unpack(pt_info[g]);
-    ScreenTri S;
-    uint32_t key;
-    float4 q[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) q[j] = pt_vert[5 * g + pt_corner(D, (int)(id & 3), j)];
-    pt_screen(U, q, S, key);
-    const uint64_t m = tile_coverage(S, tile % U.tiles_x, tile / U.tiles_x, U.width, U.height);
-    const int k = (int)(id & 3);
-    const uint32_t slots = (uint32_t)pt_corner(D, k, 0) | ((uint32_t)pt_corner(D, k, 1) << 3) |
-                           ((uint32_t)pt_corner(D, k, 2) << 6);
-    out[2 * i + 1] = make_uint4(id, (uint32_t)m, (uint32_t)(m >> 32), slots);
+    bin_stats(out.scratch, part, (uint32_t)D.ntri, kmin, kmax);
+    bin_emit<false>(B, L, ntri, part, gridDim.x, out);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -551,7 +427,7 @@ struct PtFragLds {
 __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__ items, int nitems,
                                                     const uint32_t* __restrict__ order,
                                                     const float4* __restrict__ pt_vert,
-                                                    const float4* __restrict__ pt_col, const uint4* __restrict__ recs,
+                                                    const float4* __restrict__ pt_col, RecordStream stream,
                                                     const uint2* __restrict__ ranges, PixelState ps_all) {
     __shared__ PtRecLds L;
     __shared__ PtFragLds F;
@@ -572,15 +448,19 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
     const int64_t slot0 = (int64_t)B.block0 * 256;
     float4 C = make_float4(0.f, 0.f, 0.f, 1.0f);  // premultiplied RGB, transmittance
     uint32_t n = 0, nck = 0, nlast = 0, last = rg.x;
-    // Two-stage prefetch: while a batch is shaded, the next batch's corner data and the record words of the
-    // batch after it are in flight.
+    // Three-stage prefetch: while a batch is shaded, the next batch's corner data, the record words of the batch
+    // after it and the record indices of the one after that are in flight.
+    const uint4* __restrict__ recs = stream.recs;
+    const uint32_t* __restrict__ rec_of = stream.route->vals;
     uint4 cur = make_uint4(0u, 0u, 0u, 0u), nxt = cur;
+    uint32_t ahead = 0u;
     PtRecData cd;
+    if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = recs[rec_of[rg.x + kBatch + lane]];
     if (lane < kBatch && rg.x + lane < rg.y) {
-        cur = recs[2 * (int64_t)(rg.x + lane) + 1];
+        cur = recs[rec_of[rg.x + lane]];
         pt_fetch(pt_vert, pt_col, slot0, cur, cd);
     }
-    if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = recs[2 * (int64_t)(rg.x + kBatch + lane) + 1];
+    if (lane < kBatch && rg.x + 2 * kBatch + lane < rg.y) ahead = rec_of[rg.x + 2 * kBatch + lane];
     for (uint32_t base = rg.x; base < rg.y; base += kBatch) {
         const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
         if (lane < cnt) pt_store(slot0, cur, cd, L, lane);
@@ -588,7 +468,8 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
             cur = nxt;
             pt_fetch(pt_vert, pt_col, slot0, cur, cd);
         }
-        if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = recs[2 * (int64_t)(base + 2 * kBatch + lane) + 1];
+        if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = recs[ahead];
+        if (lane < kBatch && base + 3 * kBatch + lane < rg.y) ahead = rec_of[base + 3 * kBatch + lane];
         __syncthreads();
         uint32_t mask = 0u;
         if (valid)
@@ -675,7 +556,7 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
                                                     const AdjointTarget* __restrict__ targets, int nitems,
                                                     const uint32_t* __restrict__ order,
                                                     const float4* __restrict__ pt_vert,
-                                                    const float4* __restrict__ pt_col, const uint4* __restrict__ recs,
+                                                    const float4* __restrict__ pt_col, RecordStream stream,
                                                     const uint2* __restrict__ ranges, PixelState ps_all,
                                                     float* __restrict__ tri_grad, int use_abs) {
     __shared__ PtRecLds L;
@@ -721,17 +602,21 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
     const bool per_cell = B.cell_col != nullptr;
     const uint32_t nrec = rg.y - rg.x;
     const int nbatch = (int)((nrec + kBatch - 1) / kBatch);
-    // A batch's record words are loaded a batch ahead, its corner data while the batch before is being summed up.
+    // A batch's record words are loaded a batch ahead (their indices two), its corner data while the batch before is being summed up.
     // Both have arrived before that batch's atomics are issued: a load waits for every atomic issued before it.
     const int64_t slot0 = (int64_t)B.block0 * 256;
+    const uint4* __restrict__ recs = stream.recs;
+    const uint32_t* __restrict__ rec_of = stream.route->vals;
     uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t ahead = 0u;  // this lane's record of the next batch
     PtRecData R;
     {
         const uint32_t b0 = rg.x + (uint32_t)(nbatch - 1) * kBatch;
         if (lane < kBatch && b0 + lane < rg.y) {
-            rec = recs[2 * (int64_t)(b0 + lane) + 1];
+            rec = recs[rec_of[b0 + lane]];
             pt_fetch(pt_vert, pt_col, slot0, rec, R);
         }
+        if (nbatch > 1 && lane < kBatch) ahead = rec_of[b0 - kBatch + lane];
     }
     for (int bi = nbatch - 1; bi >= 0; bi--) {
         const uint32_t base = rg.x + (uint32_t)bi * kBatch;
@@ -749,7 +634,10 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
             const uint32_t m2 = (uint32_t)ballot(sub & 4u), m3 = (uint32_t)ballot(sub & 8u);
             gm = grp == 0 ? m0 : grp == 1 ? m1 : grp == 2 ? m2 : m3;
         }
-        if (bi > 0 && lane < kBatch) rec = recs[2 * (int64_t)(base - kBatch + lane) + 1];
+        if (bi > 0 && lane < kBatch) {
+            rec = recs[ahead];
+            if (bi > 1) ahead = rec_of[base - 2 * kBatch + lane];
+        }
         for (int e = lane; e < kBatch * 16; e += 64)
             reinterpret_cast<float4*>(&s_acc[0][0])[e] = make_float4(0.f, 0.f, 0.f, 0.f);  // all four copies
         __syncthreads();
@@ -1213,40 +1101,28 @@ __global__ __launch_bounds__(64) void k_pt_backprop(const BatchItem* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------------------------
-void launch_pt_count(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* pt_info, float4* pt_vert,
-                     float4* pt_col, uint32_t* counts, uint32_t* block_stats, hipStream_t s) {
+void launch_pt_bin(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* pt_info, float4* pt_vert,
+                   float4* pt_col, bool small, const BinOut& out, hipStream_t s) {
     if (nblocks <= 0) return;
-    hipLaunchKernelGGL(k_pt_count, dim3((unsigned)nblocks), dim3(256), 0, s, items, nitems, pt_info, pt_vert, pt_col,
-                       counts, reinterpret_cast<uint4*>(block_stats));
-}
-
-void launch_pt_emit(const BatchItem* items, int nitems, int64_t nblocks, const uint32_t* pt_info,
-                    const float4* pt_vert, const uint32_t* offsets, const uint32_t* counts, uint64_t* keys,
-                    uint32_t* vals, int64_t cap, uint32_t* overflow, hipStream_t s) {
-    if (nblocks <= 0) return;
-    hipLaunchKernelGGL(k_pt_emit, dim3((unsigned)nblocks), dim3(256), 0, s, items, nitems, pt_info, pt_vert, offsets,
-                       counts, keys, vals, (uint64_t)cap, overflow);
-}
-
-void launch_pt_gather(const BatchItem* items, int nitems, const uint32_t* pt_info, const float4* pt_vert,
-                      const SortRoute* route, int64_t n, const uint64_t* n_dev, uint4* out, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_pt_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, items, nitems, pt_info,
-                       pt_vert, route, n, n_dev, out);
+    if (small)
+        hipLaunchKernelGGL(k_pt_bin<64>, dim3((unsigned)(4 * nblocks)), dim3(kBinBlock), 0, s, items, nitems, pt_info,
+                           pt_vert, pt_col, out);
+    else
+        hipLaunchKernelGGL(k_pt_bin<256>, dim3((unsigned)nblocks), dim3(kBinBlock), 0, s, items, nitems, pt_info,
+                           pt_vert, pt_col, out);
 }
 
 void launch_pt_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                       const uint32_t* pt_info, const float4* pt_vert, const float4* pt_col, const uint4* recs,
-                       const uint2* ranges, PixelState ps, hipStream_t s) {
+                       const float4* pt_vert, const float4* pt_col, RecordStream recs, const uint2* ranges,
+                       PixelState ps, hipStream_t s) {
     if (ntiles <= 0) return;
-    (void)pt_info;  // the records carry their corners' vertex slots
     hipLaunchKernelGGL(k_pt_forward, dim3((unsigned)ntiles), dim3(64), 0, s, items, nitems, order, pt_vert, pt_col,
                        recs, ranges, ps);
 }
 
 void launch_pt_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                        int64_t nblocks, const uint32_t* order, const uint32_t* pt_info, const float4* pt_vert,
-                       const float4* pt_col, const uint4* recs, const uint2* ranges, PixelState ps, float* tri_grad,
+                       const float4* pt_col, RecordStream recs, const uint2* ranges, PixelState ps, float* tri_grad,
                        int64_t tri_grad_floats, int use_abs, hipStream_t s) {
     if (ntiles <= 0) return;
     fill_u32(reinterpret_cast<uint32_t*>(tri_grad), 0u, tri_grad_floats, s);

@@ -46,8 +46,8 @@ struct TileEdge {
     bool tie;
 };
 
-// (tx, ty): a tile of 1 << shift pixels (8 by default).
-__device__ __forceinline__ TileEdge tile_edge(const ScreenTri& S, int e, int tx, int ty, int shift = 3) {
+// (tx, ty): a tile of 1 << shift pixels.
+__device__ __forceinline__ TileEdge tile_edge(const ScreenTri& S, int e, int tx, int ty, int shift) {
     const int a = e, b = e == 2 ? 0 : e + 1;
     const long long dx = S.X[b] - S.X[a], dy = S.Y[b] - S.Y[a];
     const long long px0 = 256LL * ((long long)tx << shift) + 128, py0 = 256LL * ((long long)ty << shift) + 128;
@@ -58,10 +58,9 @@ __device__ __forceinline__ TileEdge tile_edge(const ScreenTri& S, int e, int tx,
     t.tie = dy < 0 || (dy == 0 && dx > 0);
     return t;
 }
-
 // False when some edge function is negative at every pixel centre of tile (tx, ty): a record of that tile
 // could not cover a pixel.  (The maximum of E over the tile's centre lattice sits at a corner.)
-__device__ __forceinline__ bool tile_may_cover(const ScreenTri& S, int tx, int ty, int shift = 3) {
+__device__ __forceinline__ bool tile_may_cover(const ScreenTri& S, int tx, int ty, int shift) {
     const long long n1 = (1 << shift) - 1;
 #pragma unroll
     for (int e = 0; e < 3; e++) {
@@ -91,70 +90,52 @@ __device__ __forceinline__ bool pixel_inside(const int32_t X[3], const int32_t Y
 // Faces whose bounding box spans more tiles than this keep every tile of it (bounded per-thread work).
 constexpr int kMaxTestedTiles = 64;
 
-__device__ __forceinline__ bool test_tiles(const FaceBins& b) {
-    return (b.tx1 - b.tx0 + 1) * (b.ty1 - b.ty0 + 1) <= kMaxTestedTiles;
-}
-
-__device__ __forceinline__ uint32_t face_record_count(const FaceBins& b) {
-    if (b.tx0 > b.tx1 || b.ty0 > b.ty1) return 0u;
-    if (!test_tiles(b)) return (uint32_t)((b.tx1 - b.tx0 + 1) * (b.ty1 - b.ty0 + 1));
-    uint32_t c = 0;
-    for (int ty = b.ty0; ty <= b.ty1; ty++)
-        for (int tx = b.tx0; tx <= b.tx1; tx++) c += tile_may_cover(b.S, tx, ty, b.shift) ? 1u : 0u;
-    return c;
-}
-
-// Exact coverage of tile (tx, ty): bit ly * 8 + lx is set when the centre of pixel (8 tx + lx, 8 ty + ly) is
-// inside the triangle; pixels outside the viewport are clear.  Edges whose extremes over the tile decide every
-// pixel at once are not evaluated per pixel.
+// Exact coverage of 8x8 tile (tx, ty): bit ly * 8 + lx is set when the centre of pixel (8 tx + lx, 8 ty + ly) is
+// inside the triangle; pixels outside the viewport are clear.
+//
+// Per edge E = 256 W + r with W = q + ly dx - lx dy, q = floor(C / 256), r = C mod 256 (C: E at the tile's first
+// pixel), so E > 0, or E == 0 on a tie edge  <=>  W >= wmin.  Screen coordinates span less than 2^26 (the guard band
+// of 16 viewports, 1/256 pixel), so ly dx - lx dy stays below 7 * 2^27 < 2^30 in magnitude and q may be clamped to
+// +-2^30, beyond which it decides every pixel: all of it is exact in 32 bits.  The three edges' signs are combined
+// per pixel and collected by one funnel shift, 5 instructions a pixel without branches.
 __device__ __forceinline__ uint64_t tile_coverage(const ScreenTri& S, int tx, int ty, int width, int height) {
-    const int nx = min(8, width - 8 * tx), ny = min(8, height - 8 * ty);
-    const uint64_t row = nx >= 8 ? 0xFFull : ((1ull << nx) - 1ull);
-    uint64_t m = 0;
-    for (int ly = 0; ly < ny; ly++) m |= row << (8 * ly);
-#pragma unroll 1
+    const int32_t px = 2048 * tx + 128, py = 2048 * ty + 128;
+    int32_t dx[3], dy[3], row[3];  // row: W - wmin at the last pixel of the row in hand
+#pragma unroll
     for (int e = 0; e < 3; e++) {
-        const TileEdge t = tile_edge(S, e, tx, ty);
-        const long long ex = 7 * t.sx, ey = 7 * t.sy;
-        const long long emax = t.C + (ex > 0 ? ex : 0) + (ey > 0 ? ey : 0);
-        const long long emin = t.C + (ex < 0 ? ex : 0) + (ey < 0 ? ey : 0);
-        if (emax < 0 || (emax == 0 && !t.tie)) return 0ull;
-        if (emin > 0 || (emin == 0 && t.tie)) continue;  // the edge admits every pixel of the tile
-        uint64_t em = 0;
-        // sx = -256 dy and sy = 256 dx, so E = 256 W + r with W = q + ly dx - lx dy, q = floor(C / 256),
-        // r = C mod 256: E > 0 or (E == 0 on a tie edge)  <=>  W >= wmin.  The edge crosses the tile, so
-        // emin <= 0 <= emax bounds |E| by 7 (|sx| + |sy|) and |W| by 7 (|dx| + |dy|) + 1 < 2^31 for screen
-        // coordinates below 2^26 (the guard band keeps them below 2^25.2): exact in 32-bit integers.
-        const long long dx = t.sy >> 8, dy = -(t.sx >> 8);
-        if (dx > -(1ll << 27) && dx < (1ll << 27) && dy > -(1ll << 27) && dy < (1ll << 27)) {
-            const int dxi = (int)dx, dyi = (int)dy;
-            const int r = (int)(t.C & 255);
-            const int wmin = (r > 0 || t.tie) ? 0 : 1;
-            const int q = (int)(t.C >> 8);
-            // only values at the tile's 64 pixel centres are formed (no step past the tile can overflow)
-#pragma unroll
-            for (int ly = 0; ly < 8; ly++) {
-                const int Wr = q + ly * dxi;
-                uint32_t rm = 0;
-#pragma unroll
-                for (int lx = 0; lx < 8; lx++) rm |= (uint32_t)(Wr - lx * dyi >= wmin) << lx;
-                em |= (uint64_t)rm << (8 * ly);
-            }
-        } else {
-            long long Er = t.C;
-#pragma unroll 1
-            for (int ly = 0; ly < 8; ly++) {
-                long long E = Er;
-                for (int lx = 0; lx < 8; lx++) {
-                    if (E > 0 || (E == 0 && t.tie)) em |= 1ull << (8 * ly + lx);
-                    E += t.sx;
-                }
-                Er += t.sy;
-            }
-        }
-        m &= em;
-        if (m == 0) return 0ull;
+        const int a = e, b = e == 2 ? 0 : e + 1;
+        dx[e] = S.X[b] - S.X[a];
+        dy[e] = S.Y[b] - S.Y[a];
+        const int64_t C = (int64_t)dx[e] * (int64_t)(py - S.Y[a]) - (int64_t)dy[e] * (int64_t)(px - S.X[a]);
+        const int32_t hi = (int32_t)(C >> 38);
+        int32_t q = (int32_t)(C >> 8);
+        q = hi > 0 ? (1 << 30) : hi < -1 ? -(1 << 30) : q;
+        const bool tie = dy[e] < 0 || (dy[e] == 0 && dx[e] > 0);
+        const int32_t wmin = ((uint32_t)C & 255u) != 0u || tie ? 0 : 1;
+        row[e] = (q - wmin) + 7 * (dx[e] - dy[e]);
     }
+    uint32_t out[2];
+#pragma unroll
+    for (int half = 1; half >= 0; half--) {
+        uint32_t m = 0u;  // sign bits, first pixel highest: set outside
+#pragma unroll
+        for (int ly = 3; ly >= 0; ly--) {
+            int32_t v[3] = {row[0], row[1], row[2]};
+#pragma unroll
+            for (int lx = 7; lx >= 0; lx--) {
+                m = __builtin_amdgcn_alignbit(m, (uint32_t)(v[0] | v[1] | v[2]), 31u);
+#pragma unroll
+                for (int e = 0; e < 3; e++) v[e] += dy[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 3; e++) row[e] -= dx[e];
+        }
+        out[half] = ~m;
+    }
+    const int nx = min(8, width - 8 * tx), ny = min(8, height - 8 * ty);
+    uint64_t m = ((uint64_t)out[1] << 32) | out[0];
+    if (nx < 8) m &= 0x0101010101010101ull * ((1ull << nx) - 1ull);
+    if (ny < 8) m &= (1ull << (8 * ny)) - 1ull;
     return m;
 }
 

@@ -63,7 +63,7 @@ __device__ __forceinline__ float3_ lane_ray(float3_ mine, int pl) {
 // (PartOfTile).
 template <bool kCell, int kRound, bool kSub, int kEdge = kTileEdge>
 __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items, int nitems,
-                                             const uint4* __restrict__ recs, const uint2* __restrict__ ranges,
+                                             RecordStream stream, const uint2* __restrict__ ranges,
                                              const PixelState& ps_all, uint32_t gsub, RecordLds& L,
                                              FragListLds<kRound>& F, uint32_t part = 0u) {
     constexpr bool kPart = kEdge < kTileEdge;
@@ -102,11 +102,14 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
     float4 C = make_float4(0.f, 0.f, 0.f, 1.0f);  // premultiplied RGB, transmittance
     uint32_t n = 0, last = rg.x, nck = 0, nlast = 0;
     bool done = !valid;
-    // Two-stage prefetch: while a batch is shaded, the next batch's vertex data and the record words of the
-    // batch after it are in flight (of a part: the candidates of the batch after that, too).
+    // Three-stage prefetch: while a batch is shaded, the next batch's vertex data, the record words of the batch
+    // after it and the record indices of the one after that (of a part: its candidates' masks) are in flight.
     RecordIn cur, nxt;
     RecordData cd;
-    PartFeed<kEdge, false> feed{recs, rg.x, rg.y, pt.origin, {}};
+    const uint4* __restrict__ recs = stream.recs;
+    const uint32_t* __restrict__ rec_of = stream.route->vals;
+    PartFeed<kEdge, false> feed{recs, rec_of, stream.route->masks, rg.x, rg.y, pt.origin, {}};
+    uint32_t ahead = 0u;  // this lane's record of the batch after nxt's
     // a part's batch: the stream indices of its records (the entries of a part fill at most half the list)
     static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kMaxFrags / 2, "no room for a part's indices");
     uint32_t* const part_idx = reinterpret_cast<uint32_t*>(F.entry + kMaxFrags / 2);
@@ -121,11 +124,12 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
         nnxt = feed.next(pend, lane, nxt, nxt_idx);
         feed.load(lane);
     } else {
+        if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = load_record(recs, rec_of[rg.x + kBatch + lane]);
         if (lane < kBatch && rg.x + lane < rg.y) {
-            cur = load_record(recs, rg.x + lane);
+            cur = load_record(recs, rec_of[rg.x + lane]);
             fetch_record_data<kCell>(pos, col, cur, cd);
         }
-        if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = load_record(recs, rg.x + kBatch + lane);
+        if (lane < kBatch && rg.x + 2 * kBatch + lane < rg.y) ahead = rec_of[rg.x + 2 * kBatch + lane];
     }
     for (uint32_t base = rg.x; kPart ? ncur > 0 : base < rg.y; base += kBatch) {
         const int cnt = kPart ? ncur : (int)min((uint32_t)kBatch, rg.y - base);
@@ -147,7 +151,8 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
                 cur = nxt;
                 fetch_record_data<kCell>(pos, col, cur, cd);
             }
-            if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = load_record(recs, base + 2 * kBatch + lane);
+            if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = load_record(recs, ahead);
+            if (lane < kBatch && base + 3 * kBatch + lane < rg.y) ahead = rec_of[base + 3 * kBatch + lane];
             __syncthreads();
             if constexpr (kSub) {
                 subtile_masks(L, stash, cnt, x, y, valid, lane);
@@ -245,16 +250,16 @@ __device__ __forceinline__ uint32_t claim_tile(uint32_t* __restrict__ queue) {
 template <bool kCell, int kRound, bool kSub, bool kQueue>
 __global__ __launch_bounds__(64) void k_render_forward(const BatchItem* __restrict__ items, int nitems,
                                                         const uint32_t* __restrict__ order,
-                                                        const uint4* __restrict__ recs,
+                                                        RecordStream stream,
                                                         const uint2* __restrict__ ranges, PixelState ps_all,
                                                         uint32_t* __restrict__ queue, uint32_t ntiles) {
     __shared__ RecordLds L;
     __shared__ FragListLds<kRound> F;
     if constexpr (!kQueue) {
-        forward_tile<kCell, kRound, kSub>(items, nitems, recs, ranges, ps_all, global_tile_of_block(order), L, F);
+        forward_tile<kCell, kRound, kSub>(items, nitems, stream, ranges, ps_all, global_tile_of_block(order), L, F);
     } else {
         for (uint32_t t = claim_tile(queue); t < ntiles; t = claim_tile(queue)) {
-            forward_tile<kCell, kRound, kSub>(items, nitems, recs, ranges, ps_all,
+            forward_tile<kCell, kRound, kSub>(items, nitems, stream, ranges, ps_all,
                                               order != nullptr ? order[t] : t, L, F);
             __syncthreads();
         }
@@ -264,12 +269,12 @@ __global__ __launch_bounds__(64) void k_render_forward(const BatchItem* __restri
 // (8 / kEdge)^2 workgroups per tile, one per part, in image order.
 template <bool kCell, int kEdge>
 __global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __restrict__ items, int nitems,
-                                                              const uint4* __restrict__ recs,
+                                                              RecordStream stream,
                                                               const uint2* __restrict__ ranges, PixelState ps_all) {
     __shared__ RecordLds L;
     __shared__ FragListLds<kRoundDefault> F;
     constexpr uint32_t kParts = PartOfTile<kEdge>::kParts;
-    forward_tile<kCell, kRoundDefault, false, kEdge>(items, nitems, recs, ranges, ps_all, blockIdx.x / kParts, L, F,
+    forward_tile<kCell, kRoundDefault, false, kEdge>(items, nitems, stream, ranges, ps_all, blockIdx.x / kParts, L, F,
                                                      blockIdx.x % kParts);
 }
 
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __
 template <bool kRef, bool kCell, bool kSub, int kEdge = kTileEdge>
 __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items,
                                              const AdjointTarget* __restrict__ targets, int nitems,
-                                             const uint4* __restrict__ recs, const uint2* __restrict__ ranges,
+                                             RecordStream stream, const uint2* __restrict__ ranges,
                                              const PixelState& ps_all, int use_abs, uint32_t gsub, RecordLds& L,
                                              AdjFragLds& A, float4 (&s_seg)[kRef ? 3 : 1][kRoundAdj],
                                              uint32_t part = 0u) {
@@ -356,12 +361,15 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     // Batches run back to front, from the last record that any of the wave's pixels composited (early ray
     // termination leaves the records behind it out).  The next batch's record words are loaded when the current
     // batch starts and its vertex data just before the current batch's gradient atomics, so that staging it never
-    // waits on memory.
+    // waits on memory (record indices one batch further ahead).
     const uint32_t behind = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u32(valid ? last : 0u));
     const int nbatch = (int)((behind - rg.x + kBatch - 1) / kBatch);
     RecordIn nxt;
     RecordData nd;
-    PartFeed<kEdge, true> feed{recs, rg.x, behind, pt.origin, {}};
+    const uint4* __restrict__ recs = stream.recs;
+    const uint32_t* __restrict__ rec_of = stream.route->vals;
+    PartFeed<kEdge, true> feed{recs, rec_of, stream.route->masks, rg.x, behind, pt.origin, {}};
+    uint32_t ahead = 0u;  // this lane's record of the next batch
     static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kAdjFrags / 2, "no room for a part's indices");
     uint32_t* const part_idx = reinterpret_cast<uint32_t*>(A.entry + kAdjFrags / 2);  // as in the forward
     uint32_t* const pend = part_idx + kBatch;
@@ -374,9 +382,10 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     } else {
         const uint32_t b0 = rg.x + (uint32_t)(nbatch - 1) * kBatch;
         if (lane < kBatch && b0 + lane < rg.y) {
-            nxt = load_record(recs, b0 + lane);
+            nxt = load_record(recs, rec_of[b0 + lane]);
             fetch_record_data<kCell>(pos, col, nxt, nd);
         }
+        if (nbatch > 1 && lane < kBatch) ahead = rec_of[b0 - kBatch + lane];
     }
     for (int bi = nbatch - 1; kPart ? nnxt > 0 : bi >= 0; bi--) {
         const uint32_t base = kPart ? 0u : rg.x + (uint32_t)bi * kBatch;
@@ -389,7 +398,8 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             feed.load(lane);
             nnxt = feed.next(pend, lane, nxt, nxt_idx);
         } else if (bi > 0 && lane < kBatch) {
-            nxt = load_record(recs, base - kBatch + lane);
+            nxt = load_record(recs, ahead);
+            if (bi > 1) ahead = rec_of[base - 2 * kBatch + lane];
         }
         const bool more = kPart ? nnxt > 0 : bi > 0;
         // lanes j and j + 32 own record j's 28 values (first / second half of 14) for this batch
@@ -742,7 +752,7 @@ template <bool kRef, bool kCell, bool kSub, bool kQueue>
 __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint(const BatchItem* __restrict__ items,
                                                         const AdjointTarget* __restrict__ targets, int nitems,
                                                         const uint32_t* __restrict__ order,
-                                                        const uint4* __restrict__ recs,
+                                                        RecordStream stream,
                                                         const uint2* __restrict__ ranges, PixelState ps_all,
                                                         int use_abs, uint32_t* __restrict__ queue,
                                                         uint32_t ntiles) {
@@ -750,11 +760,11 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint(const Batch
     __shared__ AdjFragLds A;
     __shared__ float4 s_seg[kRef ? 3 : 1][kRoundAdj];  // reference mode: sub-segment colours, then their adjoints
     if constexpr (!kQueue) {
-        adjoint_tile<kRef, kCell, kSub>(items, targets, nitems, recs, ranges, ps_all, use_abs,
+        adjoint_tile<kRef, kCell, kSub>(items, targets, nitems, stream, ranges, ps_all, use_abs,
                                         global_tile_of_block(order), L, A, s_seg);
     } else {
         for (uint32_t t = claim_tile(queue); t < ntiles; t = claim_tile(queue)) {
-            adjoint_tile<kRef, kCell, kSub>(items, targets, nitems, recs, ranges, ps_all, use_abs,
+            adjoint_tile<kRef, kCell, kSub>(items, targets, nitems, stream, ranges, ps_all, use_abs,
                                             order != nullptr ? order[t] : t, L, A, s_seg);
             __syncthreads();
         }
@@ -765,20 +775,20 @@ template <bool kRef, bool kCell, int kEdge>
 __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint_parts(const BatchItem* __restrict__ items,
                                                                            const AdjointTarget* __restrict__ targets,
                                                                            int nitems,
-                                                                           const uint4* __restrict__ recs,
+                                                                           RecordStream stream,
                                                                            const uint2* __restrict__ ranges,
                                                                            PixelState ps_all, int use_abs) {
     __shared__ RecordLds L;
     __shared__ AdjFragLds A;
     __shared__ float4 s_seg[kRef ? 3 : 1][kRoundAdj];
     constexpr uint32_t kParts = PartOfTile<kEdge>::kParts;
-    adjoint_tile<kRef, kCell, false, kEdge>(items, targets, nitems, recs, ranges, ps_all, use_abs,
+    adjoint_tile<kRef, kCell, false, kEdge>(items, targets, nitems, stream, ranges, ps_all, use_abs,
                                             blockIdx.x / kParts, L, A, s_seg, blockIdx.x % kParts);
 }
 
 // Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.
 __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __restrict__ items, int nitems,
-                                                          const uint4* __restrict__ recs,
+                                                          RecordStream stream,
                                                           const uint2* __restrict__ ranges, PixelState ps_all,
                                                           int max_per_pixel, int32_t* __restrict__ out_ids_all) {
     __shared__ RecordLds L;
@@ -787,6 +797,8 @@ __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __rest
     const BatchItem& B = items[item_of_sub(items, nitems, gsub)];
     const ViewUniforms& U = B.U;
     const float* __restrict__ pos = B.pos;
+    const uint4* __restrict__ recs = stream.recs;
+    const uint32_t* __restrict__ rec_of = stream.route->vals;
     const PixelState ps = item_pixel_state(ps_all, B);
     int32_t* __restrict__ out_ids = out_ids_all + B.pixel0 * max_per_pixel;
     const SubTile st = sub_tile(B, gsub);
@@ -803,7 +815,7 @@ __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __rest
         const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
         if (lane < cnt) {
             RecordData d;
-            const RecordIn r = load_record(recs, base + lane);
+            const RecordIn r = load_record(recs, rec_of[base + lane]);
             fetch_record_data(pos, nullptr, r, d);
             if (stash != nullptr)
                 store_record<true>(U, r, d, L, lane, stash);
@@ -821,7 +833,7 @@ __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __rest
             m &= m - 1u;
             if (base + j >= last) break;
             if (k < max_per_pixel)
-                out_ids[(int64_t)pix * max_per_pixel + k] = (int32_t)recs[2 * (int64_t)(base + j) + 1].x;
+                out_ids[(int64_t)pix * max_per_pixel + k] = (int32_t)recs[2 * (int64_t)rec_of[base + j] + 1].x;
             k++;
         }
         __syncthreads();
@@ -866,7 +878,7 @@ static void launch_tiles(Kernel grid_kernel, Kernel queue_kernel, int64_t ntiles
 
 template <bool kCell, bool kSub, int kRound>
 static void launch_forward_round(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                                 const uint4* recs, const uint2* ranges, PixelState ps, uint32_t* queue,
+                                 RecordStream recs, const uint2* ranges, PixelState ps, uint32_t* queue,
                                  hipStream_t s) {
     launch_tiles(k_render_forward<kCell, kRound, kSub, false>, k_render_forward<kCell, kRound, kSub, true>, ntiles,
                  queue, s, items, nitems, order, recs, ranges, ps);
@@ -874,7 +886,7 @@ static void launch_forward_round(const BatchItem* items, int nitems, int64_t nti
 
 template <bool kCell, bool kSub>
 static void launch_forward_kind(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                                const uint4* recs, const uint2* ranges, PixelState ps, int round, uint32_t* queue,
+                                RecordStream recs, const uint2* ranges, PixelState ps, int round, uint32_t* queue,
                                 hipStream_t s) {
     if (round == 64)
         launch_forward_round<kCell, kSub, 64>(items, nitems, ntiles, order, recs, ranges, ps, queue, s);
@@ -885,7 +897,7 @@ static void launch_forward_kind(const BatchItem* items, int nitems, int64_t ntil
 }
 
 template <int kEdge>
-static void launch_forward_parts(const BatchItem* items, int nitems, int64_t ntiles, const uint4* recs,
+static void launch_forward_parts(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
                                  const uint2* ranges, PixelState ps, uint32_t colour_kinds, hipStream_t s) {
     const dim3 grid((unsigned)(ntiles * PartOfTile<kEdge>::kParts));
     if (colour_kinds & kColoursPerVertex)
@@ -895,7 +907,7 @@ static void launch_forward_parts(const BatchItem* items, int nitems, int64_t nti
 }
 
 void launch_render_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
-                           const uint4* recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
+                           RecordStream recs, const uint2* ranges, PixelState ps, uint32_t colour_kinds,
                            hipStream_t s, int round, bool sub, uint32_t* queue, int edge) {
     if (ntiles <= 0) return;
     if (edge == 4) return launch_forward_parts<4>(items, nitems, ntiles, recs, ranges, ps, colour_kinds, s);
@@ -916,7 +928,7 @@ void launch_render_forward(const BatchItem* items, int nitems, int64_t ntiles, c
 
 template <bool kRef, bool kCell, bool kSub>
 static void launch_adjoint_kind(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
-                                const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps,
+                                const uint32_t* order, RecordStream recs, const uint2* ranges, PixelState ps,
                                 int use_abs, uint32_t* queue, hipStream_t s) {
     launch_tiles(k_render_adjoint<kRef, kCell, kSub, false>, k_render_adjoint<kRef, kCell, kSub, true>, ntiles,
                  queue, s, items, targets, nitems, order, recs, ranges, ps, use_abs);
@@ -924,7 +936,7 @@ static void launch_adjoint_kind(const BatchItem* items, const AdjointTarget* tar
 
 template <bool kSub>
 static void launch_adjoint_sub(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
-                               const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps,
+                               const uint32_t* order, RecordStream recs, const uint2* ranges, PixelState ps,
                                int use_abs, int mode, uint32_t colour_kinds, uint32_t* queue, hipStream_t s) {
     if (colour_kinds & kColoursPerVertex) {
         if (mode == 1)
@@ -941,7 +953,7 @@ static void launch_adjoint_sub(const BatchItem* items, const AdjointTarget* targ
 
 template <int kEdge>
 static void launch_adjoint_parts(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
-                                 const uint4* recs, const uint2* ranges, PixelState ps, int use_abs, int mode,
+                                 RecordStream recs, const uint2* ranges, PixelState ps, int use_abs, int mode,
                                  uint32_t colour_kinds, hipStream_t s) {
     const dim3 grid((unsigned)(ntiles * PartOfTile<kEdge>::kParts));
     if ((colour_kinds & kColoursPerVertex) && mode == 1)
@@ -956,7 +968,7 @@ static void launch_adjoint_parts(const BatchItem* items, const AdjointTarget* ta
 }
 
 void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
-                           const uint32_t* order, const uint4* recs, const uint2* ranges, PixelState ps, int use_abs,
+                           const uint32_t* order, RecordStream recs, const uint2* ranges, PixelState ps, int use_abs,
                            int mode, uint32_t colour_kinds, hipStream_t s, bool sub, uint32_t* queue, int edge) {
     if (ntiles <= 0) return;
     if (edge == 4)
@@ -998,7 +1010,7 @@ void launch_fold_vertex_grads(const float* acc, int64_t V, float* grad_pos, floa
                        reinterpret_cast<const float4*>(acc), V, grad_pos, grad_col);
 }
 
-void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, const uint4* recs,
+void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
                              const uint2* ranges, PixelState ps, int max_per_pixel, int32_t* out_ids, hipStream_t s) {
     if (ntiles <= 0) return;
     hipLaunchKernelGGL(k_export_fragments, dim3((unsigned)ntiles), dim3(64), 0, s, items, nitems, recs, ranges,

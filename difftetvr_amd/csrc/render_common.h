@@ -19,13 +19,15 @@ struct alignas(16) RecordLds {  // 16-byte aligned: vid[] is also read as int4
     int32_t vid[4][kBatch];
 };
 
-// One record of the tile renderer's stream (two uint4 per record): the tet's vertex indices, and
-// {tet * 4 + face, coverage mask low, high, 0}.
+// One record of the tile renderer (two uint4): the tet's vertex indices, and {tet * 4 + face, coverage mask low,
+// high, 0}.  Records lie in binning order; the sorted stream is a list of their indices (SortRoute::vals), so a
+// batch's indices are loaded one step ahead of its records.
 struct RecordIn {
     uint4 vid;
     uint4 rec;
 };
 
+// Record `i` of the binning order.
 __device__ __forceinline__ RecordIn load_record(const uint4* __restrict__ recs, uint32_t i) {
     RecordIn r;
     r.vid = recs[2 * (int64_t)i];
@@ -166,13 +168,6 @@ __device__ __forceinline__ SubTile sub_tile(const BatchItem& B, uint32_t gsub) {
     return t;
 }
 
-__device__ __forceinline__ void setup_record(const ViewUniforms& U, const float* __restrict__ pos,
-                                             const float* __restrict__ col, const RecordIn& r, RecordLds& L, int i) {
-    RecordData d;
-    fetch_record_data(pos, col, r, d);
-    store_record(U, r, d, L, i);
-}
-
 // 32-bit mask of the batch's records (bit j: record j, j < cnt) that cover this lane's pixel.
 __device__ __forceinline__ uint32_t lane_coverage(const RecordLds& L, int cnt, int lane) {
     const uint32_t* w = L.mask[lane >> 5];
@@ -219,6 +214,8 @@ struct PartOfTile {
 template <int kEdge, bool kReverse>
 struct PartFeed {
     const uint4* __restrict__ recs;
+    const uint32_t* __restrict__ order;  // the stream: record indices
+    const uint2* __restrict__ masks;     // the stream's coverage masks
     uint32_t begin, end;  // the records not yet passed
     uint32_t origin;
     uint2 cand[2];        // coverage masks of this lane's candidates
@@ -231,10 +228,7 @@ struct PartFeed {
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             cand[k] = make_uint2(0u, 0u);
-            if (within(k, lane)) {
-                const uint4* r = recs + 2 * (int64_t)index(k, lane) + 1;
-                cand[k] = make_uint2(r->y, r->z);
-            }
+            if (within(k, lane)) cand[k] = masks[index(k, lane)];
         }
     }
     // The next batch, from the candidates load requested: lane j < the returned count gets record j and its index.
@@ -271,7 +265,7 @@ struct PartFeed {
         __syncthreads();
         if (lane < cnt) {
             idx = pend[lane];
-            r = load_record(recs, idx);
+            r = load_record(recs, order[idx]);
         }
         return cnt;
     }
