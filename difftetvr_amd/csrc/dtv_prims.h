@@ -212,7 +212,7 @@ __device__ __forceinline__ void atomic_add_f32(float* p, float v) {
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // p in LDS.
-__device__ __forceinline__ void lds_add_f32(float* p, float v) {
+__device__ __forceinline__ void lds_add_f64(double* p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 

@@ -12,8 +12,10 @@
 // What bounds it: the float atomics.  One per value (12 a tet) go to the memory side at about 25 G/s, whatever
 // their addresses: 746 us for 1.57M tets, against about 20 us for the mesh's bytes.  Neighbouring tets of a mesh
 // file share most vertices, so a workgroup sums the tets of its range per vertex in LDS first (a hash table of
-// vertex ids) and issues one atomic per value of each distinct vertex: 146 us for the 1.57M tets of a 64^3 grid
-// (275 -> 54 us for a Delaunay ball of 401K tets; with the grid's tets shuffled, 929 -> 777 us).
+// vertex ids) and issues one atomic per value of each distinct vertex.  The sums are doubles: on gfx950 an LDS
+// addition of doubles takes about half a cycle per lane, one of floats about four (146 us with float sums).
+// 25 us for the 1.57M tets of a 64^3 grid; 275 -> 35 us for a Delaunay ball of 401K tets; with the grid's tets
+// shuffled, 929 -> 772 us.
 #include "dtv_kernels.h"
 #include "dtv_prims.h"
 
@@ -86,10 +88,10 @@ __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __r
                                                               float beta, float* __restrict__ grad_pos) {
     constexpr int kTab = kThreads * kRegPer;
     __shared__ int32_t keys[kTab];
-    __shared__ float sums[3 * kTab];
+    __shared__ double sums[3 * kTab];
     for (int e = threadIdx.x; e < kTab; e += kThreads) {
         keys[e] = -1;
-        sums[3 * e] = sums[3 * e + 1] = sums[3 * e + 2] = 0.f;
+        sums[3 * e] = sums[3 * e + 1] = sums[3 * e + 2] = 0.0;
     }
     __syncthreads();
     const int64_t t0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * kRegPer;
@@ -102,9 +104,9 @@ __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __r
         for (int k = 0; k < 4; k++) {
             const int e = reg_entry<kTab>(keys, vid[k]);
             if (e >= 0) {
-                lds_add_f32(&sums[3 * e + 0], g[k].x);
-                lds_add_f32(&sums[3 * e + 1], g[k].y);
-                lds_add_f32(&sums[3 * e + 2], g[k].z);
+                lds_add_f64(&sums[3 * e + 0], g[k].x);
+                lds_add_f64(&sums[3 * e + 1], g[k].y);
+                lds_add_f64(&sums[3 * e + 2], g[k].z);
             } else {
                 float* to = grad_pos + 3 * (int64_t)vid[k];
                 atomic_add_f32(&to[0], g[k].x);
@@ -117,18 +119,19 @@ __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __r
     for (int i = threadIdx.x; i < 3 * kTab; i += kThreads) {
         const int e = i / 3;
         const int32_t v = keys[e];
-        if (v >= 0 && sums[i] != 0.f) atomic_add_f32(&grad_pos[3 * (int64_t)v + (i - 3 * e)], sums[i]);
+        const float sum = (float)sums[i];
+        if (v >= 0 && sum != 0.f) atomic_add_f32(&grad_pos[3 * (int64_t)v + (i - 3 * e)], sum);
     }
 }
 
-// Ranges of 4,096 tets hold 0.37 distinct vertices a tet on a 64^3 cube grid (1,024 tets: 0.67), so the larger
-// workgroup issues about half the atomics; it is taken when its ranges still give every CU one.
+// Ranges of 2,048 tets hold 0.40 distinct vertices a tet on a 64^3 cube grid (1,024 tets: 0.47), so the larger
+// workgroup issues fewer atomics; it is taken when its ranges still give every CU one.
 void launch_tet_regularizer(const int32_t* cells, const float* pos, int64_t T, float lambda, float beta,
                             float* grad_pos, hipStream_t s) {
     if (T <= 0) return;
-    constexpr int64_t kLarge = 1024 * kRegPer, kSmall = 256 * kRegPer;
+    constexpr int64_t kLarge = 512 * kRegPer, kSmall = 256 * kRegPer;
     if (T >= 256 * kLarge)
-        hipLaunchKernelGGL(k_tet_regularizer<1024>, dim3((unsigned)((T + kLarge - 1) / kLarge)), dim3(1024), 0, s,
+        hipLaunchKernelGGL(k_tet_regularizer<512>, dim3((unsigned)((T + kLarge - 1) / kLarge)), dim3(512), 0, s,
                            cells, pos, T, lambda, beta, grad_pos);
     else
         hipLaunchKernelGGL(k_tet_regularizer<256>, dim3((unsigned)((T + kSmall - 1) / kSmall)), dim3(256), 0, s,
