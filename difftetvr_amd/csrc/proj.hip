@@ -587,7 +587,7 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
     if (valid) {
         Cw = ps.ray_color[pix].w;
         n = ps.frag_count[pix];
-        ck.start((int)ps.num_ckpt[pix], P, ps, pix);
+        ck.start((int)ps.num_ckpt[pix], n, Cw, P, ps, pix);
         const float4 di = dimage[pix];
         dC[0] = di.x;
         dC[1] = di.y;
@@ -651,10 +651,9 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
             const bool live = has && ((L.mask[cbit >> 5][j] >> (cbit & 31)) & 1u);
             PtFrag f;
             pt_eval(L, j, px, py, f);
-            ck.restore(n, Cw, P, ps, pix);
             float Tin = Cw < kPtTinyT ? 0.0f : div_nr(Cw, f.A);
-            Tin = n == 1 ? 1.0f : Tin;
-            Tin = ck.n1 == n - 1 ? ck.t1 : Tin;
+            const bool at_ckpt = live && ck.n1 == n - 1u;
+            Tin = at_ckpt ? ck.t1 : Tin;
             float g[5], lam[3];
             {
 #pragma clang fp contract(fast)
@@ -665,6 +664,7 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
                 dC[3] = live ? d3 : dC[3];
                 Cw = live ? Tin : Cw;
                 n -= live ? 1u : 0u;
+                if (at_ckpt) ck.advance(P, ps, pix);
                 // F = (alpha c.rgb, alpha), alpha = 1 - exp(-c.a d)
                 const float dal = dF[3] + (dF[0] * f.c[0] + dF[1] * f.c[1] + dF[2] * f.c[2]);
                 g[0] = a * dF[0];

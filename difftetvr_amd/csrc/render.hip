@@ -43,7 +43,7 @@ struct FragListLds {
 // The adjoint's: with the records, 13 KB per wave, so that three waves fit in each SIMD (a CU has 160 KB).  A
 // batch whose fragments exceed kAdjFrags is processed in two parts of 16 records; the per-fragment gradient rows
 // are reduced half a round (32 fragments) at a time; ray directions stay in registers and move between lanes by
-// permute.  The flush's vertex hash table spans entry and w, which are free by then.
+// permute.  The flush's vertex table spans entry and w, which are free by then.
 constexpr int kAdjFrags = 1024;
 struct AdjFragLds {
     uint16_t entry[kAdjFrags];  // (pixel lane << 5) | record index, one part of a batch
@@ -278,6 +278,13 @@ __global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __
                                                      blockIdx.x % kParts);
 }
 
+// What bounds it: vector instructions.  At 1,572,864 tets and 1024 x 1024 (110.0 M fragments) the kernel issues 2.02e9
+// of them, 1076 per round of 64 fragments, in nearly nine of ten issue slots, and the LDS is 64 % busy; memory traffic
+// and occupancy (three waves per SIMD) matter little.  So the phases are written for few instructions: A and C without
+// branches, the checkpoint test of B as one comparison, the owners' row masks for both halves of a round from one set
+// of ballots, and the flush as LDS additions of doubles: with those 2.19e9 -> 2.02e9 instructions, the whole step 7.80 ->
+// 7.62 ms, and 1.02 to 1.04 times faster from 24K tets on.
+//
 // kRef = false: exact derivative of the forward.  kRef = true: the reference's adjoint as written
 // (AdjointIntersectRasterization.glsl:111-362): per pixel from the blended output image, back to front, the
 // 'over' operator is inverted per sub-segment 3, 2, 1 (sub-segment 0 is skipped) with no checkpoints, and
@@ -315,6 +322,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     int32_t* stash = kSub ? reinterpret_cast<int32_t*>(A.entry) : nullptr;
     const float3_ ro = f3(U.camPos[0], U.camPos[1], U.camPos[2]);
     const float3_ my_rd = ray_direction(U, x, y);
+    const float my_scale = seg_scale(U, my_rd);
     const float att = U.attenuation;
     const uint2 rg = ranges[gtile];
     const int P = U.width * U.height;
@@ -326,21 +334,12 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     float4 C = make_float4(0.f, 0.f, 0.f, 1.0f);
     float dC[4] = {0.f, 0.f, 0.f, 0.f};
     uint32_t n = 0, last = 0;
-    int jck = -1;                // next checkpoint slot (back to front)
-    // Checkpoint jck's fragment count and transmittance, and the count of the one before it, are held in
-    // registers: the next checkpoint is always loaded well before it is needed.
-    uint32_t ck_n = 0xFFFFFFFFu, ck_n2 = 0xFFFFFFFFu;
-    float ck_t = 1.0f;
+    CheckpointCursor ck;
     if (valid) {
         C = ps.ray_color[pix];
         n = ps.frag_count[pix];
         last = ps.last_rec[pix];
-        jck = (int)ps.num_ckpt[pix] - 1;
-        if (jck >= 0) {
-            ck_n = ps.ckpt_n[(int64_t)jck * P + pix];
-            ck_t = ps.ckpt_t[(int64_t)jck * P + pix];
-            if (jck >= 1) ck_n2 = ps.ckpt_n[(int64_t)(jck - 1) * P + pix];
-        }
+        if constexpr (!kRef) ck.start((int)ps.num_ckpt[pix], n, C.w, P, ps, pix);
         const float4 di = dimage[pix];
         dC[0] = di.x;
         dC[1] = di.y;
@@ -351,7 +350,6 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             C = make_float4(C.x + T * U.clear[0], C.y + T * U.clear[1], C.z + T * U.clear[2],
                             (1.0f - T) + T * U.clear[3]);
             dC[3] = di.w;
-            jck = -1;
         } else {
             dC[3] = di.w * (1.0f - U.clear[3]) - (di.x * U.clear[0] + di.y * U.clear[1] + di.z * U.clear[2]);
         }
@@ -436,16 +434,19 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
         const uint32_t mine_end = off + (uint32_t)__popc(mask);
         __syncthreads();
         for (uint32_t r0 = 0; r0 < total; r0 += kRoundAdj) {
-            // A: fragment colours (one fragment per lane; E stays in registers for phase C)
+            // A: fragment colours (one fragment per lane; E stays in registers for phase C).  The exact adjoint's
+            // phases A and C run without branches: a lane behind the list's end evaluates the last fragment again
+            // and drops the result, so no register has to be cleared for it.
             FragEval E;
             E.hit = false;
             {
                 const uint32_t e = r0 + lane;
-                const uint32_t ent = e < total ? A.entry[e] : (uint32_t)(lane << 5);
+                const uint32_t ent = A.entry[min(e, total - 1u)];
                 const int pl = ent >> 5, j = ent & 31;
                 const float3_ rdp = lane_ray(my_rd, pl);
-                if (e < total) {
-                    eval_fragment<kCell, true, kRef>(L, j, ro, rdp, att, seg_scale(U, rdp), E);
+                const float tscale = U.linear_depth ? __shfl(my_scale, pl, 64) : 1.0f;
+                if (!kRef || e < total) {
+                    eval_fragment<kCell, true, kRef>(L, j, ro, rdp, att, tscale, E);
                     A.val[lane] = E.hit ? E.F : make_float4(0.f, 0.f, 0.f, kMissMarker);
                     if constexpr (kRef) {
 #pragma unroll
@@ -476,15 +477,6 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                     n--;
                     continue;
                 }
-                if (jck >= 0 && ck_n == n) {
-                    C.w = ck_t;
-                    jck--;
-                    ck_n = ck_n2;
-                    if (jck >= 0) {
-                        ck_t = ps.ckpt_t[(int64_t)jck * P + pix];
-                        ck_n2 = jck >= 1 ? ps.ckpt_n[(int64_t)(jck - 1) * P + pix] : 0xFFFFFFFFu;
-                    }
-                }
                 const float4 f = A.val[e - r0];
                 // the fragment's input transmittance: a checkpoint, 1 before the first fragment, or the output
                 // divided by the fragment's transmittance (a corrected quotient: the rounding compounds along the
@@ -494,31 +486,33 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                 // its slot's value is not read.
                 const bool hit = f.w != kMissMarker;
                 float Tin = C.w < kTinyT ? 0.0f : div_nr(C.w, f.w);
-                Tin = n == 1 ? 1.0f : Tin;
-                Tin = (jck >= 0 && ck_n == n - 1) ? ck_t : Tin;
+                C.w = hit ? Tin : C.w;
+                n--;
+                if (ck.n1 == n) {
+                    Tin = ck.t1;
+                    C.w = Tin;
+                    ck.advance(P, ps, pix);
+                }
                 A.val[e - r0] = make_float4(Tin * dC[0], Tin * dC[1], Tin * dC[2], Tin * dC[3]);
                 {
 #pragma clang fp contract(fast)
                     const float d3 = dC[3] * f.w - (dC[0] * f.x + dC[1] * f.y + dC[2] * f.z);
                     dC[3] = hit ? d3 : dC[3];
                 }
-                C.w = hit ? Tin : C.w;
-                n--;
             }
             if (n == 0) done = true;
             __syncthreads();
             // C: gradients of the fragments (one per lane).  Each fragment's 28 values are stored into A.w (half
             // a round at a time); the owner lanes of each record then add its rows.
             int key = kBatch;  // record index of this lane's fragment, kBatch = none
-            float g[28];
-#pragma unroll
-            for (int q = 0; q < 28; q++) g[q] = 0.f;
+            float g[28];  // set where key is
             {
                 const uint32_t e = r0 + lane;
-                const uint32_t ent = e < total ? A.entry[e] : (uint32_t)(lane << 5);
+                const uint32_t ent = A.entry[min(e, total - 1u)];
                 const int pl = ent >> 5, j = ent & 31;
                 const float3_ rdp = lane_ray(my_rd, pl);
-                if (e < total && E.hit) {
+                const float tscale = U.linear_depth ? __shfl(my_scale, pl, 64) : 1.0f;
+                if (!kRef || (e < total && E.hit)) {
                     if constexpr (kRef) {
                         const float4 dacc[3] = {s_seg[0][lane], s_seg[1][lane], s_seg[2][lane]};
                         frag_backward_reference(E, L, j, ro, rdp, att, dacc, use_abs != 0, g);
@@ -526,7 +520,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                         // positions in the usual slots; the tet's colour gradient in vertex 0's colour slots
                         float lam0[4], lam1[4], dcell[4];
                         float3_ Q0, Q1;
-                        frag_backward_cell(E, L, j, rdp, att, seg_scale(U, rdp), A.val[lane], lam0, lam1, dcell, Q0,
+                        frag_backward_cell(E, L, j, rdp, att, tscale, A.val[lane], lam0, lam1, dcell, Q0,
                                            Q1);
                         if (use_abs) {
 #pragma unroll
@@ -542,11 +536,14 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                             g[7 * v + 2] = l0 * Q0.z + l1 * Q1.z;
                         }
 #pragma unroll
-                        for (int ch = 0; ch < 4; ch++) g[3 + ch] = dcell[ch];
+                        for (int ch = 0; ch < 4; ch++) {
+                            g[3 + ch] = dcell[ch];
+                            g[10 + ch] = g[17 + ch] = g[24 + ch] = 0.f;
+                        }
                     } else {
                         float lam0[4], lam1[4], dcol0[4], dcol1[4];
                         float3_ Q0, Q1;
-                        frag_backward_exact(E, L, j, rdp, att, seg_scale(U, rdp), A.val[lane], lam0, lam1, dcol0,
+                        frag_backward_exact(E, L, j, rdp, att, tscale, A.val[lane], lam0, lam1, dcol0,
                                             dcol1, Q0, Q1);
                         if (use_abs) {
 #pragma unroll
@@ -567,22 +564,28 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                             for (int ch = 0; ch < 4; ch++) g[7 * v + 3 + ch] = l0 * dcol0[ch] + l1 * dcol1[ch];
                         }
                     }
-                    key = j;
+                    if (kRef || (e < total && E.hit)) key = j;
                 }
             }
             // Per half round (the fragments of lanes 0-31, then 32-63): each fragment stores its 28 values in
             // the row of its lane; the owner lanes of record j (j and j + 32) find the record's rows from a mask of
-            // the lanes whose key equals j, formed from five ballots of the key bits, and add them.
+            // the lanes whose key equals j, formed from ballots of the key bits for both halves at once, and add them.
+            uint32_t eq[2];
+            {
+                const uint64_t any = ballot(key < kBatch);
+                eq[0] = (uint32_t)any;
+                eq[1] = (uint32_t)(any >> 32);
+#pragma unroll
+                for (int b = 0; b < 5; b++) {
+                    const uint64_t ones = ballot((key >> b) & 1);
+                    const uint32_t flip = (((uint32_t)lane >> b) & 1u) - 1u;
+                    eq[0] &= (uint32_t)ones ^ flip;
+                    eq[1] &= (uint32_t)(ones >> 32) ^ flip;
+                }
+            }
 #pragma unroll 1
             for (int h = 0; h < 2; h++) {
                 const bool mine = (lane >> 5) == h && key < kBatch;
-                const uint32_t jj = (uint32_t)(lane & 31);
-                uint32_t eqj = (uint32_t)(ballot(mine) >> (32 * h));
-#pragma unroll
-                for (int b = 0; b < 5; b++) {
-                    const uint32_t ones = (uint32_t)(ballot(mine && ((key >> b) & 1)) >> (32 * h));
-                    eqj &= ((jj >> b) & 1u) ? ones : ~ones;
-                }
                 if (mine) {
 #pragma unroll
                     for (int q = 0; q < 28; q++) A.w[lane & 31][q] = g[q];
@@ -591,7 +594,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                 {
                     // two rows per step: 28 independent LDS reads in flight instead of 14
                     const int half = lane >> 5;
-                    uint32_t m = eqj;
+                    uint32_t m = h == 0 ? eq[0] : eq[1];
                     while (m) {
                         const int r1 = __ffs(m) - 1;
                         m &= m - 1u;
@@ -620,22 +623,22 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
         // slots, slot s = v * 32 + j.  Depth-adjacent tets share most vertices (typically 6-7 slots per distinct
         // vertex in a batch), so the slots of one vertex are summed before the global atomics: each slot finds
         // its vertex's entry in an LDS hash table keyed by vertex id (compare-and-swap; the first slot of a
-        // vertex creates the entry), stores its values in its own LDS row and links the row into the entry's
-        // list with one exchange; the entry's creator then sums the list.  (LDS float atomics, one per value and
-        // slot, cost about 2.5 cycles per lane.)
+        // vertex creates the entry) and adds its values to the entry's sums.  The sums are doubles: an LDS addition
+        // of doubles takes about half a cycle per lane, one of floats about four.  (Rows linked into a list per
+        // entry and summed by the entry's creator took 600 vector instructions more per batch, one in eleven of
+        // the kernel's.)
         {
             const int j = lane & 31, half = lane >> 5;
-            constexpr int kTab = 160;
-            // over entry and w, free after the rounds: keys[kTab], head[kTab], rows[128][8] (7 values, next slot)
-            int32_t* keys = reinterpret_cast<int32_t*>(&A.entry[0]);
-            int32_t* head = keys + kTab;
-            float* rows = reinterpret_cast<float*>(head + kTab);
-            static_assert(sizeof(int32_t) * 2 * kTab + sizeof(float) * 8 * 128 <= sizeof(A.entry) + sizeof(A.w),
-                          "flush tables exceed the fragment list space");
-            for (int e = lane; e < kTab; e += 64) {
-                keys[e] = -1;
-                head[e] = -1;
-            }
+            constexpr int kTab = 96;
+            // over entry and w, free after the rounds: sums[kTab][7], keys[kTab]
+            double* sums = reinterpret_cast<double*>(&A.entry[0]);
+            int32_t* keys = reinterpret_cast<int32_t*>(sums + 7 * kTab);
+            static_assert((sizeof(int32_t) + 7 * sizeof(double)) * kTab <= sizeof(A.entry) + sizeof(A.w),
+                          "the flush table exceeds the fragment list space");
+            static_assert(7 * kTab % 2 == 0 && offsetof(AdjFragLds, w) == sizeof(A.entry), "table layout");
+            for (int e = lane; e < 7 * kTab / 2; e += 64)
+                reinterpret_cast<double2*>(sums)[e] = make_double2(0.0, 0.0);
+            for (int e = lane; e < kTab; e += 64) keys[e] = -1;
             __syncthreads();
             const int s0 = (2 * half) * 32 + j, s1 = s0 + 32;
             const int32_t* vids = &L.vid[0][0];
@@ -676,33 +679,16 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 if (ent[k] < 0) continue;
-                const int sl = k == 0 ? s0 : s1;
 #pragma unroll
-                for (int c = 0; c < 7; c++) rows[8 * sl + c] = acc[7 * k + c];
-                rows[8 * sl + 7] = __int_as_float(atomicExch(&head[ent[k]], sl));
+                for (int c = 0; c < 7; c++) lds_add_f64(&sums[7 * ent[k] + c], acc[7 * k + c]);
             }
-            __syncthreads();
-            // each entry's creator sums its list into its own row
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-                if (!owner[k]) continue;
-                float sum[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                for (int sl = head[ent[k]]; sl >= 0;) {
-#pragma unroll
-                    for (int c = 0; c < 7; c++) sum[c] += rows[8 * sl + c];
-                    sl = __float_as_int(rows[8 * sl + 7]);
-                }
-                const int own = k == 0 ? s0 : s1;
-#pragma unroll
-                for (int c = 0; c < 7; c++) rows[8 * own + c] = sum[c];
-            }
-            // The creators' rows are listed compactly; then eight lanes per row add its seven sums to the
-            // vertex's 32-byte row of the interleaved accumulator, one wave instruction per eight vertices.
+            // The entries are listed compactly; then eight lanes per entry add its seven sums to the vertex's
+            // 32-byte row of the interleaved accumulator, one wave instruction per eight vertices.
             int32_t* list = reinterpret_cast<int32_t*>(&A.val[0]);  // free after the rounds: 256 words
             const uint64_t own0 = ballot(owner[0]), own1 = ballot(owner[1]);
             const uint32_t n0 = (uint32_t)popc64(own0), nown = n0 + (uint32_t)popc64(own1);
-            if (owner[0]) list[popc64(own0 & lanemask_lt())] = s0;
-            if (owner[1]) list[n0 + popc64(own1 & lanemask_lt())] = s1;
+            if (owner[0]) list[popc64(own0 & lanemask_lt())] = ent[0];
+            if (owner[1]) list[n0 + popc64(own1 & lanemask_lt())] = ent[1];
             __syncthreads();
             // The next batch's vertex data is requested before the atomics, so staging it does not wait for them.
             // Only lanes 0..31 hold that batch's record words (of a part: lanes 0 to its count).
@@ -713,10 +699,10 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                 for (uint32_t b0 = 0; b0 < nown; b0 += 8) {
                     const uint32_t li = b0 + (uint32_t)(lane >> 3);
                     if (li < nown && c < 7) {
-                        const int sl = list[li];
-                        const float val = rows[8 * sl + c];
+                        const int e = list[li];
+                        const float val = (float)sums[7 * e + c];
                         if (val != 0.f) {
-                            atomic_add_f32(&vacc[8 * (int64_t)vids[sl] + c], val);
+                            atomic_add_f32(&vacc[8 * (int64_t)keys[e] + c], val);
                             issued++;
                         }
                     }
@@ -724,7 +710,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             }
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                // a slot that found no entry (not possible with kTab > 128 ids) issues its own values
+                    // a slot that found no entry (more than kTab distinct vertices) issues its own values
                 if (!slot_live || ent[k] >= 0) continue;
                 const int64_t g = k == 0 ? v0 : v1;
 #pragma unroll

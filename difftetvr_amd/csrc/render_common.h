@@ -541,12 +541,15 @@ __device__ __forceinline__ void eval_fragment(const RecordLds& L, int j, float3_
     float tin, tout, bary[4];
     bool have_bary;
     E.hit = ray_tet(L, j, ro, rd, fi, fo, tin, tout, bary, have_bary);
-    if (!E.hit) {
+    E.f0 = fi;  // valid faces on a miss too
+    E.f1 = fo;
+    if (!E.hit) {  // an empty segment
+        E.t0 = E.t1 = 0.f;
+        E.u0 = E.v0 = E.u1 = E.v1 = 0.f;
+        E.col0 = E.col1 = make_float4(0.f, 0.f, 0.f, 0.f);
         E.F = make_float4(0.f, 0.f, 0.f, 1.0f);
         return;
     }
-    E.f0 = fi;
-    E.f1 = fo;
     E.t0 = tin;
     E.t1 = tout;
     if constexpr (kCell) {
@@ -627,35 +630,35 @@ __device__ __forceinline__ PixelState item_pixel_state(const PixelState& all, co
     return ps;
 }
 
-// A pixel's stored checkpoints, walked back to front: the next one's fragment count and transmittance (n1, t1; n1 =
-// 0xFFFFFFFF: none left), and those of the one before it, requested a checkpoint ahead: the step that passes a
-// checkpoint then waits for no load.
+// A pixel's stored checkpoints, walked back to front: the next one's fragment count and transmittance (n1, t1), and
+// those of the one before it (n2, t2), requested a checkpoint ahead: the step that passes a checkpoint then waits for
+// no load.  Behind the last stored one comes the state before the first fragment (0, 1).
 struct CheckpointCursor {
-    uint32_t n1 = 0xFFFFFFFFu, n2 = 0xFFFFFFFFu;
+    uint32_t n1 = 0u, n2 = 0u;
     float t1 = 1.0f, t2 = 1.0f;
     int left = 0;  // checkpoints before (n2, t2)
     __device__ __forceinline__ void request(int64_t P, const PixelState& ps, int pix) {
-        n2 = 0xFFFFFFFFu;
+        n2 = 0u;
+        t2 = 1.0f;
         left--;
         if (left >= 0) {
             n2 = ps.ckpt_n[(int64_t)left * P + pix];
             t2 = ps.ckpt_t[(int64_t)left * P + pix];
         }
     }
-    __device__ __forceinline__ void start(int count, int64_t P, const PixelState& ps, int pix) {
-        left = count;
-        request(P, ps, pix);
+    __device__ __forceinline__ void advance(int64_t P, const PixelState& ps, int pix) {
         n1 = n2;
         t1 = t2;
         request(P, ps, pix);
     }
-    // With n fragments still to undo: the transmittance behind them from a checkpoint taken there.
-    __device__ __forceinline__ void restore(uint32_t n, float& T, int64_t P, const PixelState& ps, int pix) {
-        if (n1 == n) {
+    // n: the pixel's fragments, T: the transmittance behind them.
+    __device__ __forceinline__ void start(int count, uint32_t n, float& T, int64_t P, const PixelState& ps, int pix) {
+        left = count;
+        request(P, ps, pix);
+        advance(P, ps, pix);
+        if (n1 == n && count > 0) {
             T = t1;
-            n1 = n2;
-            t1 = t2;
-            request(P, ps, pix);
+            advance(P, ps, pix);
         }
     }
 };
