@@ -278,12 +278,14 @@ __global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __
                                                      blockIdx.x % kParts);
 }
 
-// What bounds it: vector instructions.  At 1,572,864 tets and 1024 x 1024 (110.0 M fragments) the kernel issues 2.02e9
-// of them, 1076 per round of 64 fragments, in nearly nine of ten issue slots, and the LDS is 64 % busy; memory traffic
-// and occupancy (three waves per SIMD) matter little.  So the phases are written for few instructions: A and C without
-// branches, the checkpoint test of B as one comparison, the owners' row masks for both halves of a round from one set
-// of ballots, and the flush as LDS additions of doubles: with those 2.19e9 -> 2.02e9 instructions, the whole step 7.80 ->
-// 7.62 ms, and 1.02 to 1.04 times faster from 24K tets on.
+// What bounds it: vector instructions first (1,572,864 tets at 1024 x 1024, 110.0 M fragments: about 980 per round of 64
+// fragments, 85 to 90 % of the issue slots), then the LDS (64 % busy); memory traffic matters little, and three waves
+// per SIMD are all that the registers of a fragment's gradients allow.  So the phases are written for few
+// instructions: A and C without branches, the checkpoint test of B as one comparison, the owners' row masks for both
+// halves of a round from one set of ballots, the flush as LDS additions of doubles (2.19e9 -> 2.02e9 instructions in
+// all, the whole step 7.80 -> 7.62 ms, and 1.02 to 1.04 times faster from 24K tets on), and the sub-segments' adjoint
+// as running sums shared with the composite (frag_backward_exact: a fragment's backward 537 -> 441 instructions; the
+// step 7.04 -> 6.90 ms).
 //
 // kRef = false: exact derivative of the forward.  kRef = true: the reference's adjoint as written
 // (AdjointIntersectRasterization.glsl:111-362): per pixel from the blended output image, back to front, the
@@ -530,6 +532,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                         }
 #pragma unroll
                         for (int v = 0; v < 4; v++) {
+#pragma clang fp contract(fast)
                             const float l0 = lam0[v], l1 = lam1[v];
                             g[7 * v + 0] = l0 * Q0.x + l1 * Q1.x;
                             g[7 * v + 1] = l0 * Q0.y + l1 * Q1.y;
@@ -556,6 +559,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
                         }
 #pragma unroll
                         for (int v = 0; v < 4; v++) {
+#pragma clang fp contract(fast)
                             const float l0 = lam0[v], l1 = lam1[v];
                             g[7 * v + 0] = l0 * Q0.x + l1 * Q1.x;
                             g[7 * v + 1] = l0 * Q0.y + l1 * Q1.y;
@@ -692,6 +696,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             __syncthreads();
             // The next batch's vertex data is requested before the atomics, so staging it does not wait for them.
             // Only lanes 0..31 hold that batch's record words (of a part: lanes 0 to its count).
+            nd = RecordData{};  // or its old values would be live, and spilled, throughout the batch
             if (more && lane < (kPart ? nnxt : kBatch)) fetch_record_data<kCell>(pos, col, nxt, nd);
             uint32_t issued = 0;
             {

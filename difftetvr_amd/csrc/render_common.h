@@ -692,82 +692,68 @@ __device__ __forceinline__ void face_side_q(const RecordLds& L, int j, int f, fl
     Q = caxpy(s, n, scale(gtdc, -1.0f));
 }
 
+// Weights over the 4 local vertices of a point with barycentrics m0, m1, m2 in face f: kFaceTable's vertices in order,
+// 0 at the face's opposite vertex.
+__device__ __forceinline__ void face_weights(int f, float m0, float m1, float m2, float lam[4]) {
+    lam[0] = f == 3 ? 0.f : f == 1 ? m1 : m0;
+    lam[1] = f == 2 ? 0.f : f == 1 ? m0 : m1;
+    lam[2] = f == 1 ? 0.f : f == 0 ? m2 : f == 2 ? m1 : m0;
+    lam[3] = f == 0 ? 0.f : m2;
+}
+
 __device__ __forceinline__ void frag_backward_exact(const FragEval& E, const RecordLds& L, int j, float3_ rd,
                                                     float att, float tscale, float4 dF, float lam0[4],
                                                     float lam1[4], float dcol0[4], float dcol1[4], float3_& Q0,
                                                     float3_& Q1) {
 #pragma clang fp contract(fast)
-    float dR[4] = {dF.x, dF.y, dF.z, dF.w};
-#pragma unroll
-    for (int ch = 0; ch < 4; ch++) {
-        dcol0[ch] = 0.f;
-        dcol1[ch] = 0.f;
-    }
-    float dLdt = 0.f;
     const float tSeg = ((E.t1 - E.t0) / 4.0f) * tscale;
     float a_s[4], A_s[4], ia_s[4], kq_s[4], T_s[4];
     // as in eval_fragment: not kept live since phase A
-    (void)sub_segments_w(E.col0, E.col1, tSeg, att, a_s, A_s, ia_s, kq_s, T_s);
-    // dR.rgb is the same for every sub-segment: sum over RGB of dR c0 (sub-segment s starts at col0 + s/4
-    // (col1 - col0)) = p0 + (s/4) p1, and of dR (c0 - c1) = -p1 / 4
-    const float p0 = (dR[0] * E.col0.x + dR[1] * E.col0.y) + dR[2] * E.col0.z;
-    const float p1 =
-        (dR[0] * (E.col1.x - E.col0.x) + dR[1] * (E.col1.y - E.col0.y)) + dR[2] * (E.col1.z - E.col0.z);
-    const float sdf = -0.25f * p1;
-    float w0s = 0.f, w1s = 0.f;  // the RGB colour weights summed over the sub-segments
+    float Tn = sub_segments_w(E.col0, E.col1, tSeg, att, a_s, A_s, ia_s, kq_s, T_s);
+    // dF.rgb is the same for every sub-segment: sum over RGB of dF c0 (sub-segment s starts at col0 + s/4
+    // (col1 - col0)) = p0 + (s/4) p1, and of dF (c0 - c1) = -p1 / 4
+    const float p0 = (dF.x * E.col0.x + dF.y * E.col0.y) + dF.z * E.col0.z;
+    const float p1 = (dF.x * (E.col1.x - E.col0.x) + dF.y * (E.col1.y - E.col0.y)) + dF.z * (E.col1.z - E.col0.z);
+    const float tp = 0.25f * tSeg * p1;
+    // Sub-segment s, with T the transmittance before it, Tn = T A the one behind it and D the derivative with respect
+    // to the latter (as alpha): its colour is (1 - A) c0 + K (c0 - c1), A = exp(-a t), K = (t + 1/a) A - 1/a = -4 kq,
+    // with dA/dt = -a A, dA/da = -t A, dK/dt = -a t A, dK/da = -(K / a + t^2 A).  Hence, with
+    // h = Tn (D + dF c0 + (t/4) p1), dL/dt = a h, dL/da = t h - p1 T kq / a, and the weights of the entry and exit
+    // colours are those of the composite (sub_segments_F): sum T (1 - A), and sum T ((1 - A) s/4 + kq).
+    float S0 = 0.f, S1 = 0.f, St = 0.f, Sa = 0.f, Sb = 0.f;
+    float D = dF.w;
 #pragma unroll
     for (int s = 3; s >= 0; s--) {
-        const float omA = T_s[s];  // transmittance before s: dL/d(sub-segment s) = omA dR
-        const float fb = (float)s * 0.25f, fm = ((float)s + 0.5f) * 0.25f, fe = ((float)s + 1.0f) * 0.25f;
+        const float fb = (float)s * 0.25f, fm = ((float)s + 0.5f) * 0.25f;
+        const float a = a_s[s], T = T_s[s];
+        const float om = 1.0f - A_s[s];
         const float sc0 = p0 + fb * p1;
-        const float dsw = omA * dR[3];
-        // dR.rgb . seg[s].rgb = (1 - A) sc0 + kq p1
-        dR[3] = dR[3] * A_s[s] - ((1.0f - A_s[s]) * sc0 + kq_s[s] * p1);
-        const float a = a_s[s];
-        float da = 0.f, dts = 0.f, w0 = 0.f, w1 = 0.f;
-        if (!(a < 1e-6f)) {
-            // accumulateLinearConst: out = (1 - A) c0 + K (c0 - c1), alpha 1 - A, A = exp(-a t),
-            // K = (t + 1/a) A - 1/a; dA/dt = -a A, dA/da = -t A, dK/dt = -a t A, dK/da below
-            const float A = A_s[s];
-            const float ia = ia_s[s];
-            const float K = (tSeg + ia) * A - ia;
-            const float aA = a * A, tA = tSeg * A;
-            const float dKda = ia * ia * (1.0f - A) - tA * (tSeg + ia);
-            dts = aA * (omA * (sc0 - tSeg * sdf) + dsw);
-            da = omA * (tA * sc0 + dKda * sdf) + dsw * tA;
-            // d/dc0 = (1 - A + K), d/dc1 = -K; c0, c1 mix the entry/exit colours at fb, fe
-            const float kc0 = 1.0f - A + K;
-            w0 = omA * ((1.0f - fb) * kc0 - (1.0f - fe) * K);
-            w1 = omA * (fb * kc0 - fe * K);
-        }
-        w0s += w0;
-        w1s += w1;
-        dcol0[3] += (1.0f - fm) * att * da;
-        dcol1[3] += fm * att * da;
-        dLdt += 0.25f * dts;
+        const float Tom = T * om, Tk = T * kq_s[s];
+        float h = Tn * (D + (sc0 + tp));
+        h = a < 1e-6f ? 0.0f : h;  // an empty sub-segment
+        const float da = tSeg * h - p1 * (ia_s[s] * Tk);
+        S0 += Tom;
+        S1 += fb * Tom + Tk;
+        St += a * h;
+        Sa += da;
+        Sb += fm * da;
+        D = D * A_s[s] - (om * sc0 + kq_s[s] * p1);
+        Tn = T;
     }
-#pragma unroll
-    for (int ch = 0; ch < 3; ch++) {
-        dcol0[ch] = w0s * dR[ch];
-        dcol1[ch] = w1s * dR[ch];
-    }
-    dLdt *= tscale;  // d tSeg / d t1 = tscale / 4
+    const float w0 = S0 - S1;
+    dcol0[0] = w0 * dF.x;
+    dcol0[1] = w0 * dF.y;
+    dcol0[2] = w0 * dF.z;
+    dcol0[3] = att * (Sa - Sb);
+    dcol1[0] = S1 * dF.x;
+    dcol1[1] = S1 * dF.y;
+    dcol1[2] = S1 * dF.z;
+    dcol1[3] = att * Sb;
+    const float dLdt = (0.25f * tscale) * St;  // d tSeg / d t1 = tscale / 4
     face_side_q(L, j, E.f0, rd, dcol0, -dLdt, Q0);
     face_side_q(L, j, E.f1, rd, dcol1, dLdt, Q1);
-    // barycentric weights over the 4 local vertices (0 at the face's opposite vertex)
-    const float mu0[3] = {E.u0, E.v0, 1.0f - E.u0 - E.v0};
-    const float mu1[3] = {E.u1, E.v1, 1.0f - E.u1 - E.v1};
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        float l0 = 0.f, l1 = 0.f;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            l0 = face_vertex(E.f0, k) == v ? mu0[k] : l0;
-            l1 = face_vertex(E.f1, k) == v ? mu1[k] : l1;
-        }
-        lam0[v] = l0;
-        lam1[v] = l1;
-    }
+    face_weights(E.f0, E.u0, E.v0, 1.0f - E.u0 - E.v0, lam0);
+    face_weights(E.f1, E.u1, E.v1, 1.0f - E.u1 - E.v1, lam1);
 }
 
 // Exact adjoint of one per-cell fragment (eval_fragment<true>) given dL/dF, whose .w is the derivative with
@@ -799,19 +785,8 @@ __device__ __forceinline__ void frag_backward_cell(const FragEval& E, const Reco
         const float3_ n = f3(L.N[3 * f][j], L.N[3 * f + 1][j], L.N[3 * f + 2][j]);
         Q1 = scale(n, fast_div(dLdt, cdot(n, rd)));
     }
-    const float mu0[3] = {E.u0, E.v0, 1.0f - E.u0 - E.v0};
-    const float mu1[3] = {E.u1, E.v1, 1.0f - E.u1 - E.v1};
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        float l0 = 0.f, l1 = 0.f;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            l0 = face_vertex(E.f0, k) == v ? mu0[k] : l0;
-            l1 = face_vertex(E.f1, k) == v ? mu1[k] : l1;
-        }
-        lam0[v] = l0;
-        lam1[v] = l1;
-    }
+    face_weights(E.f0, E.u0, E.v0, 1.0f - E.u0 - E.v0, lam0);
+    face_weights(E.f1, E.u1, E.v1, 1.0f - E.u1 - E.v1, lam1);
 }
 
 // ---------------------------------------------------------------------------------------------------------
