@@ -472,9 +472,12 @@ constexpr float kEdgeMargin = 1e-4f;
 // inside the tet).  On the fast path bary = {u, v} at the entry and exit points (face_bary) and have_bary = true.
 __device__ __forceinline__ bool ray_tet(const RecordLds& L, int j, float3_ ro, float3_ rd, int& f0, int& f1, float& t0,
                                         float& t1, float bary[4], bool& have_bary) {
-    const bool outward = (L.meta[j] >> 3) & 1u;
+    // Without branches up to the slow path: nearly every wave has a lane on either side of each face's test, so they
+    // skipped nothing and cost 294 -> 218 vector instructions and as many scalar ones per 64 fragments (a render of
+    // 5.3M tets at 1920 x 1080 4.57 -> 4.24 ms, the step of 1.57M tets at 1024 x 1024 6.35 -> 6.01 ms).
+    const uint32_t flip = (L.meta[j] << 28) & 0x80000000u;  // outward normals: entering where N . rd < 0
     float tin = -__builtin_inff(), tout = __builtin_inff();
-    int fi = -1, fo = -1;
+    int fi = 0, fo = 0;  // set once tin, tout are finite
     float tf[4];
     bool par[4];
 #pragma unroll
@@ -483,18 +486,19 @@ __device__ __forceinline__ bool ray_tet(const RecordLds& L, int j, float3_ ro, f
         const float den = dot(n, rd);
         par[g] = fabsf(den) < 1e-9f;
         tf[g] = -L.k[g][j] / den;
-        if (par[g]) continue;
-        const bool entering = outward ? (den < 0.0f) : (den > 0.0f);
-        if (entering) {
-            if (tf[g] > tin) { tin = tf[g]; fi = g; }
-        } else {
-            if (tf[g] < tout) { tout = tf[g]; fo = g; }
-        }
+        const bool entering = __uint_as_float(__float_as_uint(den) ^ flip) > 0.0f;
+        const bool later = !par[g] & entering & (tf[g] > tin);
+        const bool sooner = !par[g] & !entering & (tf[g] < tout);
+        tin = later ? tf[g] : tin;
+        fi = later ? g : fi;
+        tout = sooner ? tf[g] : tout;
+        fo = sooner ? g : fo;
     }
-    if (fi >= 0 && fo >= 0 && tout >= tin && tin >= 0.0f && face_bary(L, j, fi, ro, rd, tin, bary[0], bary[1]) &&
-        face_bary(L, j, fo, ro, rd, tout, bary[2], bary[3]) &&
-        fminf(fminf(fminf(bary[0], bary[1]), 1.0f - bary[0] - bary[1]),
-              fminf(fminf(bary[2], bary[3]), 1.0f - bary[2] - bary[3])) >= kEdgeMargin) {
+    const bool area0 = face_bary(L, j, fi, ro, rd, tin, bary[0], bary[1]);
+    const bool area1 = face_bary(L, j, fo, ro, rd, tout, bary[2], bary[3]);
+    const float inner = fminf(fminf(fminf(bary[0], bary[1]), 1.0f - bary[0] - bary[1]),
+                              fminf(fminf(bary[2], bary[3]), 1.0f - bary[2] - bary[3]));
+    if ((tin >= 0.0f) & (tout < __builtin_inff()) & (tout >= tin) & area0 & area1 & (inner >= kEdgeMargin)) {
         f0 = fi;
         f1 = fo;
         t0 = tin;
