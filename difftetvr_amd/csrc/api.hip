@@ -218,7 +218,10 @@ struct dtv_view {
     bool sub_tiles = false;         // the last render binned tiles larger than 8x8
     bool queued = false;            // the last render took its tiles from a work queue (the adjoint does too)
     bool cost_ordered = true;       // the last render launched its tiles heaviest first
-    int edge = 8;                   // pixels per side a wave of the last render took (8: a tile, less: a part of one)
+    // Pixels per side that a wave of the last render took (8: a tile, less: a part of one), and one of its adjoint takes.
+    int edge = 8, adjoint_edge = 8;
+    int64_t sorted_room = 0;        // the last render's records, or in planned mode the room for them
+    bool sorted_planned = false;
     int64_t planned_cap = 0;  // > 0: planned (synchronisation-free) rendering with this record capacity
     // state of the last render
     bool rendered = false;
@@ -316,10 +319,16 @@ bool make_uniforms(const dtv_camera& camera, const dtv_render_params& params, Vi
 // 1315 / 549 / 379, 625 tiles 2361 / 962 / 842, 1,024 tiles 1193 / 599 / 625, 2,304 tiles 1718 / 1071 / 1367,
 // 4,096 tiles 2264 / 1862 / 2760, 5,000 tiles 3750 / 3054 / 3797, 9,216 tiles 2660 / 3232 / 5478.  (A batch's
 // records cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)
-int wave_edge(const dtv_render_params& prm, int64_t tiles) {
-    if (prm.renderer != DTV_RENDERER_TILE || prm.tile_launch != DTV_TILE_LAUNCH_GRID ||
-        (prm.tile_size != 0 && prm.tile_size != 8) || (prm.segments_per_pass != 0 && prm.segments_per_pass != 128))
+//
+// The Projection renderer's waves take 8x8 or 4x4 pixels.  Its adjoint gains the more (a wave's rows then share out
+// the records too) and keeps gaining where its forward no longer does, so each has its own line.  Measured, 8x8 / 4x4:
+// render 96 tiles 158 / 114, 1,344 tiles 376 / 275, 2,304 tiles 360 / 316, 4,096 tiles 513 / 538; step 96 tiles
+// 451 / 222, 1,344 tiles 1098 / 562, 2,304 tiles 905 / 597, 4,096 tiles 1251 / 1113, 5,625 tiles 1196 / 1274.
+int wave_edge(const dtv_render_params& prm, int64_t tiles, bool adjoint = false) {
+    if (prm.tile_launch != DTV_TILE_LAUNCH_GRID || (prm.tile_size != 0 && prm.tile_size != 8) ||
+        (prm.segments_per_pass != 0 && prm.segments_per_pass != 128))
         return 8;
+    if (prm.renderer == DTV_RENDERER_PROJECTION) return tiles <= (adjoint ? 5120 : 3072) ? 4 : 8;
     return tiles <= 768 ? 2 : tiles <= 5120 ? 4 : 8;
 }
 
@@ -513,7 +522,7 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     const uint32_t* fwd_order = view->cost_ordered ? view->tile_order.as<uint32_t>() : nullptr;
     view->mark(DTV_STAGE_RANGES, 0, s);
     launch_tile_ranges(&scratch->route, K, n_dev, view->ranges.as<uint2>(), edge < 8 ? view->recs.as<uint4>() : nullptr,
-                       s);
+                       proj ? 1 : 2, s);
     if (fwd_order) {
         if (tile == 8) {
             launch_tile_order(view->ranges.as<uint2>(), nullptr, tiles, view->tile_order.as<uint32_t>(), s);
@@ -535,12 +544,15 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     view->mark(DTV_STAGE_FORWARD, 0, s);
     if (proj)
         launch_pt_forward(dI, n, tiles, fwd_order, view->pt_vert.as<float4>(), view->pt_col.as<float4>(),
-                          view->stream(), view->ranges.as<uint2>(), view->pixel_state(), s);
+                          view->stream(), view->ranges.as<uint2>(), view->pixel_state(), edge, s);
     else
         launch_render_forward(dI, n, subtiles, fwd_order, view->stream(), view->ranges.as<uint2>(),
                               view->pixel_state(), kinds, s, spp, tile != 8,
                               params->tile_launch == DTV_TILE_LAUNCH_QUEUE ? view->tile_queue() : nullptr, edge);
     view->edge = edge;
+    view->adjoint_edge = wave_edge(*params, tiles, true);
+    view->sorted_room = K;
+    view->sorted_planned = planned;
     view->mark(DTV_STAGE_FORWARD, 1, s);
     DTV_HIP(hipGetLastError());
     view->colour_kinds = kinds;
@@ -666,7 +678,11 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
                  staged ? nullptr : view->dTargets.as<AdjointTarget>(), s);
     // adjoint launch order: tiles by the forward's composited fragments, heaviest first
     const uint32_t* adj_order = nullptr;
-    if (view->cost_ordered) {
+    if (view->adjoint_edge < view->edge)  // the coverage masks that a part's wave picks its records by
+        launch_tile_ranges(&view->scratch()->route, view->sorted_room,
+                           view->sorted_planned ? &view->scratch()->total : nullptr, view->ranges.as<uint2>(),
+                           view->recs.as<uint4>(), view->projection ? 1 : 2, s);
+    if (view->cost_ordered && view->adjoint_edge == 8) {
         uint32_t* o = view->tile_order.as<uint32_t>() + view->total_subtiles;
         launch_tile_order(nullptr, view->tile_frags.as<uint32_t>(), view->total_subtiles, o, s);
         adj_order = o;
@@ -678,12 +694,12 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         launch_pt_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n, view->total_tiles,
                           view->total_blocks, adj_order, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
                           view->pt_col.as<float4>(), view->stream(), view->ranges.as<uint2>(), ps,
-                          view->tri_grad.as<float>(), tg_floats, use_abs_grad ? 1 : 0, s);
+                          view->tri_grad.as<float>(), tg_floats, use_abs_grad ? 1 : 0, view->adjoint_edge, s);
     } else {
         launch_render_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n,
                               view->total_subtiles, adj_order, view->stream(), view->ranges.as<uint2>(), ps,
                               use_abs_grad ? 1 : 0, adjoint_mode, view->colour_kinds, s, view->sub_tiles,
-                              view->queued ? view->tile_queue() : nullptr, view->edge);
+                              view->queued ? view->tile_queue() : nullptr, view->adjoint_edge);
     }
     for (const Fold& fo : folds) launch_fold_vertex_grads(fo.acc, fo.V, fo.grad_pos, fo.grad_col, s);
     view->mark(DTV_STAGE_ADJOINT, 1, s);
@@ -869,7 +885,7 @@ int dtv_render_noalloc(dtv_ctx* ctx, const dtv_mesh* mesh, const dtv_camera* cam
     const SortInput in{out.keys, reinterpret_cast<uint64_t*>(base + o_keys2), reinterpret_cast<uint32_t*>(base + o_vals),
                        reinterpret_cast<uint32_t*>(base + o_vals2), K, &scratch->total, scratch->slots, 0u, 0, tbits};
     sort_records(in, hist, hist + 8 * 256, reinterpret_cast<uint32_t*>(base + o_lookback), &scratch->route, s);
-    launch_tile_ranges(&scratch->route, K, &scratch->total, ranges, edge < 8 ? recs.recs : nullptr, s);
+    launch_tile_ranges(&scratch->route, K, &scratch->total, ranges, edge < 8 ? recs.recs : nullptr, 2, s);
     if (order) launch_tile_order(ranges, nullptr, tiles, order, s);
     PixelState ps;
     ps.ray_color = reinterpret_cast<float4*>(base + o_color);

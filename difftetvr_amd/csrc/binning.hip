@@ -43,11 +43,12 @@ __global__ __launch_bounds__(kBinBlock) void k_bin(const BatchItem* __restrict__
     bin_emit<true>(B, L, nfaces, part, gridDim.x, out);
 }
 
-// ranges[t] = the sorted records of tile t; masks (kMasks): their coverage masks in sorted order.
+// ranges[t] = the sorted records of tile t; masks (kMasks): their coverage masks in sorted order, from the last uint4
+// of each record of rec_len.
 template <bool kMasks>
 __global__ __launch_bounds__(256) void k_tile_ranges(const SortRoute* __restrict__ route, int64_t n_cap,
                                                      const uint64_t* __restrict__ n_dev, uint2* __restrict__ ranges,
-                                                     const uint4* __restrict__ recs) {
+                                                     const uint4* __restrict__ recs, int rec_len) {
     const uint32_t* __restrict__ keys = route->keys;
     const uint32_t* __restrict__ vals = route->vals;
     uint2* __restrict__ masks = route->masks;
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const SortRoute* __restrict
         if (i == 0 || keys[i - 1] >> shift != t) ranges[t].x = (uint32_t)i;
         if (i == n - 1 || keys[i + 1] >> shift != t) ranges[t].y = (uint32_t)(i + 1);
         if constexpr (kMasks) {
-            const uint4 r = recs[2 * (int64_t)vals[i] + 1];
+            const uint4 r = recs[rec_len * ((int64_t)vals[i] + 1) - 1];
             masks[i] = make_uint2(r.y, r.z);
         }
     }
@@ -194,15 +195,16 @@ void launch_bin(const BatchItem* items, int nitems, int64_t nblocks, bool small,
 }
 
 void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, uint2* ranges, const uint4* recs,
-                        hipStream_t s) {
+                        int rec_len, hipStream_t s) {
     if (n <= 0) return;
     int64_t blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     if (recs != nullptr)
-        hipLaunchKernelGGL(k_tile_ranges<true>, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges, recs);
+        hipLaunchKernelGGL(k_tile_ranges<true>, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges, recs,
+                           rec_len);
     else
         hipLaunchKernelGGL(k_tile_ranges<false>, dim3((unsigned)blocks), dim3(256), 0, s, route, n, n_dev, ranges,
-                           recs);
+                           recs, rec_len);
 }
 
 void launch_tile_order(const uint2* ranges, const uint32_t* cost, int64_t num_tiles, uint32_t* order,

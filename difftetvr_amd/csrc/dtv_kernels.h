@@ -87,10 +87,10 @@ struct BinOut {
 // Bins the tets of all items (item i owns blocks [block0_i, block0_{i+1}) of 256 tets): scratch->total records, of
 // which those below cap are written, in (tet, face, tile) order.
 void launch_bin(const BatchItem* items, int nitems, int64_t nblocks, bool small, const BinOut& out, hipStream_t s);
-// ranges[t] (zeroed): the sorted records of tile t.  recs (may be NULL): the unsorted records of the tile renderer,
+// ranges[t] (zeroed): the sorted records of tile t.  recs (may be NULL): the unsorted records, rec_len uint4 each,
 // whose coverage masks then go to route->masks in sorted order.
 void launch_tile_ranges(const SortRoute* route, int64_t n, const uint64_t* n_dev, uint2* ranges, const uint4* recs,
-                        hipStream_t s);
+                        int rec_len, hipStream_t s);
 // cost[g] = record count of the binning tile holding 8x8 sub-tile g, for g < nsub.
 void launch_subtile_cost(const BatchItem* items, int nitems, int64_t nsub, const uint2* ranges, uint32_t* cost,
                          hipStream_t s);
@@ -150,13 +150,14 @@ void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles,
 // {triangle slot id (tet * 4 + k, item-local tet), coverage mask low, high, corner slots}.
 void launch_pt_bin(const BatchItem* items, int nitems, int64_t nblocks, uint32_t* pt_info, float4* pt_vert,
                    float4* pt_col, bool small, const BinOut& out, hipStream_t s);
+// edge: 8, or 4 for four waves per tile, each rendering 4x4 pixels (order is then not used).
 void launch_pt_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
                        const float4* pt_vert, const float4* pt_col, RecordStream recs, const uint2* ranges,
-                       PixelState ps, hipStream_t s);
+                       PixelState ps, int edge, hipStream_t s);
 void launch_pt_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                        int64_t nblocks, const uint32_t* order, const uint32_t* pt_info, const float4* pt_vert,
                        const float4* pt_col, RecordStream recs, const uint2* ranges, PixelState ps, float* tri_grad,
-                       int64_t tri_grad_floats, int use_abs, hipStream_t s);
+                       int64_t tri_grad_floats, int use_abs, int edge, hipStream_t s);
 
 // optim.hip
 struct AdamGroupDev {

@@ -424,6 +424,8 @@ struct PtFragLds {
 // pixel lane), rank r holding the r-th fragment of every pixel that has more than r; rounds of kPtRound
 // fragments are evaluated across the lanes, then each pixel lane composites its fragments of the round front
 // to back (about one per pixel per round).
+// kEdge = 4: four waves per tile, one per 4x4 pixels (PartOfTile), whose batches hold the records that cover them.
+template <int kEdge>
 __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__ items, int nitems,
                                                     const uint32_t* __restrict__ order,
                                                     const float4* __restrict__ pt_vert,
@@ -431,7 +433,9 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
                                                     const uint2* __restrict__ ranges, PixelState ps_all) {
     __shared__ PtRecLds L;
     __shared__ PtFragLds F;
-    const uint32_t gtile = global_tile_of_block(order);
+    constexpr bool kPart = kEdge < kTileEdge;
+    const uint32_t gtile = kPart ? blockIdx.x / PartOfTile<kEdge>::kParts : global_tile_of_block(order);
+    const PartOfTile<kEdge> pt(kPart ? blockIdx.x % PartOfTile<kEdge>::kParts : 0u);
     const BatchItem& B = items[item_of_tile(items, nitems, gtile)];
     const ViewUniforms& U = B.U;
     float4* __restrict__ out_image = reinterpret_cast<float4*>(B.image);
@@ -439,9 +443,10 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
     const int tile = (int)(gtile - B.tile0);
     const int lane = threadIdx.x;
     const uint64_t lt = lanemask_lt();
-    const int x0 = (tile % U.tiles_x) * kTileEdge, y0 = (tile / U.tiles_x) * kTileEdge;
-    const int x = x0 + (lane & 7), y = y0 + (lane >> 3);
-    const bool valid = x < U.width && y < U.height;
+    const int x0 = (tile % U.tiles_x) * kTileEdge + pt.x0, y0 = (tile / U.tiles_x) * kTileEdge + pt.y0;
+    const int x = x0 + lane % kEdge, y = y0 + lane / kEdge;
+    const bool valid = lane < pt.kPixels && x < U.width && y < U.height;
+    if (kPart && ballot(valid) == 0ull) return;
     const uint2 rg = ranges[gtile];
     const int P = U.width * U.height;
     const int pix = valid ? pixel_index(U, x, y) : 0;
@@ -455,25 +460,54 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
     uint4 cur = make_uint4(0u, 0u, 0u, 0u), nxt = cur;
     uint32_t ahead = 0u;
     PtRecData cd;
-    if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = recs[rec_of[rg.x + kBatch + lane]];
-    if (lane < kBatch && rg.x + lane < rg.y) {
-        cur = recs[rec_of[rg.x + lane]];
-        pt_fetch(pt_vert, pt_col, slot0, cur, cd);
-    }
-    if (lane < kBatch && rg.x + 2 * kBatch + lane < rg.y) ahead = rec_of[rg.x + 2 * kBatch + lane];
-    for (uint32_t base = rg.x; base < rg.y; base += kBatch) {
-        const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
-        if (lane < cnt) pt_store(slot0, cur, cd, L, lane);
-        if (lane < kBatch && base + kBatch + lane < rg.y) {
-            cur = nxt;
+    PartFeed<kEdge, false> feed{recs, rec_of, stream.route->masks, rg.x, rg.y, pt.origin, {}};
+    // a part's batch: the stream indices of its records (the entries of a part fill at most half the list)
+    static_assert(!kPart || PartOfTile<kEdge>::kPixels <= 32, "no room for a part's indices");
+    uint32_t* const part_idx = reinterpret_cast<uint32_t*>(F.entry + kBatch * 32);
+    uint32_t* const pend = part_idx + kBatch;
+    uint32_t cur_idx = 0u, nxt_idx = 0u;
+    int ncur = 0, nnxt = 0;
+    if constexpr (kPart) {
+        feed.load(lane);
+        ncur = feed.next(pend, lane, cur, cur_idx);
+        feed.load(lane);
+        if (lane < ncur) pt_fetch(pt_vert, pt_col, slot0, cur, cd);
+        nnxt = feed.next(pend, lane, nxt, nxt_idx);
+        feed.load(lane);
+    } else {
+        if (lane < kBatch && rg.x + kBatch + lane < rg.y) nxt = recs[rec_of[rg.x + kBatch + lane]];
+        if (lane < kBatch && rg.x + lane < rg.y) {
+            cur = recs[rec_of[rg.x + lane]];
             pt_fetch(pt_vert, pt_col, slot0, cur, cd);
         }
-        if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = recs[ahead];
-        if (lane < kBatch && base + 3 * kBatch + lane < rg.y) ahead = rec_of[base + 3 * kBatch + lane];
-        __syncthreads();
+        if (lane < kBatch && rg.x + 2 * kBatch + lane < rg.y) ahead = rec_of[rg.x + 2 * kBatch + lane];
+    }
+    for (uint32_t base = rg.x; kPart ? ncur > 0 : base < rg.y; base += kBatch) {
+        const int cnt = kPart ? ncur : (int)min((uint32_t)kBatch, rg.y - base);
+        if (lane < cnt) pt_store(slot0, cur, cd, L, lane);
         uint32_t mask = 0u;
-        if (valid)
-            for (int j = 0; j < cnt; j++) mask |= (uint32_t)pt_covers(L, j, lane) << j;
+        if constexpr (kPart) {
+            if (lane < cnt) part_idx[lane] = cur_idx;
+            const uint32_t cover = pt.coverage(cur, cnt, lane);
+            if (valid) mask = cover;
+            cur = nxt;
+            cur_idx = nxt_idx;
+            ncur = nnxt;
+            if (lane < ncur) pt_fetch(pt_vert, pt_col, slot0, cur, cd);
+            nnxt = feed.next(pend, lane, nxt, nxt_idx);
+            feed.load(lane);
+            __syncthreads();
+        } else {
+            if (lane < kBatch && base + kBatch + lane < rg.y) {
+                cur = nxt;
+                pt_fetch(pt_vert, pt_col, slot0, cur, cd);
+            }
+            if (lane < kBatch && base + 2 * kBatch + lane < rg.y) nxt = recs[ahead];
+            if (lane < kBatch && base + 3 * kBatch + lane < rg.y) ahead = rec_of[base + 3 * kBatch + lane];
+            __syncthreads();
+            if (valid)
+                for (int j = 0; j < cnt; j++) mask |= (uint32_t)pt_covers(L, j, lane) << j;
+        }
         // the coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
         const uint32_t total = build_fragment_list(F.entry, rank_mask, mask, false, lane);
@@ -485,9 +519,10 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
                 const uint32_t e = r0 + (uint32_t)i;
                 if (e >= total) break;
                 const uint32_t ent = F.entry[e];
-                const int pl = (int)(ent >> 5), j = (int)(ent & 31u);
-                const float px = 2.0f * (((float)(x0 + (pl & 7)) + 0.5f) / (float)U.width) - 1.0f;
-                const float py = 2.0f * (((float)(y0 + (pl >> 3)) + 0.5f) / (float)U.height) - 1.0f;
+                const uint32_t pl = ent >> 5;
+                const int j = (int)(ent & 31u);
+                const float px = 2.0f * (((float)(x0 + (int)(pl % kEdge)) + 0.5f) / (float)U.width) - 1.0f;
+                const float py = 2.0f * (((float)(y0 + (int)(pl / kEdge)) + 0.5f) / (float)U.height) - 1.0f;
                 PtFrag f;
                 pt_eval(L, j, px, py, f);
                 const float a = 1.0f - f.A;
@@ -513,7 +548,7 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
                 }
                 C.w = Tout;
                 n++;
-                last = base + (F.entry[e] & 31u) + 1;
+                last = (kPart ? part_idx[F.entry[e] & 31u] : base + (F.entry[e] & 31u)) + 1;
                 if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kPtTinyT && (int)nck < U.max_ckpt - 1) {
                     ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
                     ps.ckpt_n[(int64_t)nck * P + pix] = n;
@@ -533,8 +568,77 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
         ps.last_rec[pix] = last;
         ps.num_ckpt[pix] = nck;
     }
-    const uint32_t tile_total = wave_inclusive_scan(n);
-    if (lane == 63) ps.tile_frags[gtile] = tile_total;
+    if constexpr (!kPart) {  // the adjoint's launch order ranks tiles by them
+        const uint32_t tile_total = wave_inclusive_scan(n);
+        if (lane == 63) ps.tile_frags[gtile] = tile_total;
+    }
+}
+
+// A batch's gradients into tri_grad: record j's 21, from its 15 sums (corner k at sums[16 j + 5 k]), by way of
+// out[21 j], nonzero ones with one atomic each.  Loads issued before have arrived first.
+__device__ __forceinline__ void pt_scatter(const PtRecLds& L, const float* sums, float* __restrict__ out, int cnt,
+                                           bool per_cell, int lane, float* __restrict__ tri_grad) {
+    for (int e = lane; e < 3 * cnt; e += 64) {
+#pragma clang fp contract(fast)
+        const int j = e / 3, k = e - 3 * j;
+        float S[5], gl[3];
+#pragma unroll
+        for (int q = 0; q < 5; q++) S[q] = sums[16 * j + 5 * k + q];
+#pragma unroll
+        for (int m = 0; m < 3; m++) {
+            gl[m] = S[4] * L.d[m][j];
+            // per-cell colours are the same at every corner, and sum_m grad lambda_m = 0
+            if (!per_cell)
+                gl[m] += (S[0] * L.c[4 * m][j] + S[1] * L.c[4 * m + 1][j]) +
+                         (S[2] * L.c[4 * m + 2][j] + S[3] * L.c[4 * m + 3][j]);
+        }
+        const float X0 = L.X[0][j], X1 = L.X[1][j], X2 = L.X[2][j];
+        const float Y0 = L.Y[0][j], Y1 = L.Y[1][j], Y2 = L.Y[2][j];
+        const float iD = L.invD[j];
+        out[7 * e] = -(gl[0] * (Y1 - Y2) + gl[1] * (Y2 - Y0) + gl[2] * (Y0 - Y1)) * iD;
+        out[7 * e + 1] = -(gl[0] * (X2 - X1) + gl[1] * (X0 - X2) + gl[2] * (X1 - X0)) * iD;
+#pragma unroll
+        for (int q = 0; q < 5; q++) out[7 * e + 2 + q] = S[q];
+    }
+    __syncthreads();
+    wait_for_loads();
+    for (int e = lane; e < cnt * 21; e += 64) {
+        const float v = out[e];
+        const int j = e / 21;
+        if (v != 0.f) atomic_add_f32(&tri_grad[21 * (int64_t)L.id[j] + (e - 21 * j)], v);
+    }
+}
+
+// One fragment's gradient terms given the transmittance Tin before it and D, the alpha derivative behind it:
+// p[5 k + q] = lambda_k dL/d(c.rgba, d)[q], zero unless live.
+template <bool kAbs>
+__device__ __forceinline__ void pt_terms(const PtFrag& f, bool live, float Tin, float D, const float dC[3],
+                                         float p[15]) {
+    float g[5];
+    {
+#pragma clang fp contract(fast)
+        // F = (alpha c.rgb, alpha), alpha = 1 - exp(-c.a d); dL/dF in alpha form
+        const float a = 1.0f - f.A;
+        const float dF[4] = {Tin * dC[0], Tin * dC[1], Tin * dC[2], Tin * D};
+        const float dal = dF[3] + (dF[0] * f.c[0] + dF[1] * f.c[1] + dF[2] * f.c[2]);
+        g[0] = a * dF[0];
+        g[1] = a * dF[1];
+        g[2] = a * dF[2];
+        g[3] = dal * f.d * f.A;
+        g[4] = dal * f.c[3] * f.A;
+    }
+    if constexpr (kAbs) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) g[q] = fabsf(g[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 5; q++) g[q] = live ? g[q] : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const float lam = live ? f.l[k] : 0.0f;
+#pragma unroll
+        for (int q = 0; q < 5; q++) p[5 * k + q] = lam * g[q];
+    }
 }
 
 // Adjoint, per pixel back to front.  The wave's lanes cover the tile as four 4x4 sub-tiles, one per row of 16
@@ -550,7 +654,8 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
 // pixels of lambda_k G, G = sum_m dL/dlambda_m grad lambda_m with dL/dlambda_m = dL/dc . c_m + dL/dd d_m.  The
 // c_m, d_m and grad lambda_m are constant over the triangle, so the sum needs only the corner's colour and thickness
 // sums: 15 terms a pixel instead of 21, and G once per record instead of once per pixel.  The kernel is VALU-bound:
-//   measured (1.57M tets at 1024 x 1024): 2.95 -> 2.09 ms (with the loads ahead of the atomics and the loop without branches)
+//   measured (1.57M tets at 1024 x 1024): 2.95 -> 2.09 ms (with the loads ahead of the atomics and the loop without
+//   branches); without register copies in the loop (169 -> 157 instructions a step) the whole step 4.46 -> 4.31 ms.
 template <bool kAbs>
 __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__ items,
                                                     const AdjointTarget* __restrict__ targets, int nitems,
@@ -581,7 +686,7 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
     const int P = U.width * U.height;
     const int pix = valid ? pixel_index(U, x, y) : 0;
     float Cw = 1.0f;
-    float dC[4] = {0.f, 0.f, 0.f, 0.f};
+    float dC[3] = {0.f, 0.f, 0.f}, D = 0.f;  // dL/dC: RGB, and the alpha behind the current fragment
     uint32_t n = 0;
     CheckpointCursor ck;
     if (valid) {
@@ -592,7 +697,7 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
         dC[0] = di.x;
         dC[1] = di.y;
         dC[2] = di.z;
-        dC[3] = di.w * (1.0f - U.clear[3]) - (di.x * U.clear[0] + di.y * U.clear[1] + di.z * U.clear[2]);
+        D = di.w * (1.0f - U.clear[3]) - (di.x * U.clear[0] + di.y * U.clear[1] + di.z * U.clear[2]);
     }
     if (ballot(valid && n > 0) == 0ull) return;
     // kAbs, AbsGS-style absolute colour gradients: the per-cell variant only, as the reference's
@@ -641,51 +746,30 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
         for (int e = lane; e < kBatch * 16; e += 64)
             reinterpret_cast<float4*>(&s_acc[0][0])[e] = make_float4(0.f, 0.f, 0.f, 0.f);  // all four copies
         __syncthreads();
-        while (ballot(gm != 0u) != 0ull) {
+        for (uint64_t more = ballot(gm != 0u); more != 0ull; more = ballot(gm != 0u)) {
             // Without branches but the checkpoint's: lanes whose row has no record left, or whose pixel the record
             // does not cover, run along on record j and contribute zeros.  (Every covering record was composited,
             // so coverage alone decides.)
             const bool has = gm != 0u;
             const int j = has ? 31 - __clz(gm) : 0;  // back to front
             gm &= ~(1u << j);
-            const bool live = has && ((L.mask[cbit >> 5][j] >> (cbit & 31)) & 1u);
+            const bool live = has & (((L.mask[cbit >> 5][j] >> (cbit & 31)) & 1u) != 0u);
             PtFrag f;
             pt_eval(L, j, px, py, f);
             float Tin = Cw < kPtTinyT ? 0.0f : div_nr(Cw, f.A);
             const bool at_ckpt = live && ck.n1 == n - 1u;
             Tin = at_ckpt ? ck.t1 : Tin;
-            float g[5], lam[3];
-            {
+            float p[15];
+            pt_terms<kAbs>(f, live, Tin, D, dC, p);
+            {  // the composite's adjoint moves past this fragment
 #pragma clang fp contract(fast)
                 const float a = 1.0f - f.A;
-                // dL/dF (alpha form in .w), then the composite's adjoint moves past this fragment
-                const float dF[4] = {Tin * dC[0], Tin * dC[1], Tin * dC[2], Tin * dC[3]};
-                const float d3 = dC[3] * f.A - (dC[0] * (a * f.c[0]) + dC[1] * (a * f.c[1]) + dC[2] * (a * f.c[2]));
-                dC[3] = live ? d3 : dC[3];
+                const float d3 = D * f.A - (dC[0] * (a * f.c[0]) + dC[1] * (a * f.c[1]) + dC[2] * (a * f.c[2]));
+                D = live ? d3 : D;
                 Cw = live ? Tin : Cw;
                 n -= live ? 1u : 0u;
                 if (at_ckpt) ck.advance(P, ps, pix);
-                // F = (alpha c.rgb, alpha), alpha = 1 - exp(-c.a d)
-                const float dal = dF[3] + (dF[0] * f.c[0] + dF[1] * f.c[1] + dF[2] * f.c[2]);
-                g[0] = a * dF[0];
-                g[1] = a * dF[1];
-                g[2] = a * dF[2];
-                g[3] = dal * f.d * f.A;
-                g[4] = dal * f.c[3] * f.A;
             }
-            if constexpr (kAbs) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) g[q] = fabsf(g[q]);
-            }
-#pragma unroll
-            for (int q = 0; q < 5; q++) g[q] = live ? g[q] : 0.0f;
-#pragma unroll
-            for (int k = 0; k < 3; k++) lam[k] = live ? f.l[k] : 0.0f;
-            float p[15];
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-#pragma unroll
-                for (int q = 0; q < 5; q++) p[5 * k + q] = lam[k] * g[q];
             float s[1];
             row_reduce_scatter(p, s);
             if (has && qs < 15) s_acc[grp][16 * j + qs] += s[0];
@@ -695,38 +779,124 @@ __global__ __launch_bounds__(64) void k_pt_adjoint(const BatchItem* __restrict__
         for (int e = lane; e < cnt * 16; e += 64)
             s_acc[0][e] = (s_acc[0][e] + s_acc[1][e]) + (s_acc[2][e] + s_acc[3][e]);
         __syncthreads();
-        // record j's 21 gradients at out[21 j]
         float* __restrict__ out = &s_acc[1][0];
         static_assert(21 * kBatch <= 3 * 16 * kBatch, "the gradients exceed the row copies' space");
-        for (int e = lane; e < 3 * cnt; e += 64) {
+        pt_scatter(L, &s_acc[0][0], out, cnt, per_cell, lane, tri_grad);
+        __syncthreads();
+    }
+}
+
+// The adjoint with four waves per tile, one per 4x4 pixels: the wave's four rows hold the same 16 pixels, and each row
+// takes one of four successive records, so that the evaluation, the gradient terms and their sums advance four records
+// a step.  Only the walk along the pixel's fragments is serial: every row follows it over all four records, from their
+// transmittances and composite terms, and keeps the state in front of its own.  A record is met by one row once, so
+// its sums are stored, not added.  With few tiles the kernel is bound by its waves' serial steps, not by throughput
+// (1,344 tiles: 1.3 waves per SIMD): a step of 82,944 tets at 333 x 250 1098 -> 562 us (with the forward's parts).
+template <bool kAbs>
+__global__ __launch_bounds__(64) void k_pt_adjoint_parts(const BatchItem* __restrict__ items,
+                                                          const AdjointTarget* __restrict__ targets, int nitems,
+                                                          const float4* __restrict__ pt_vert,
+                                                          const float4* __restrict__ pt_col, RecordStream stream,
+                                                          const uint2* __restrict__ ranges, PixelState ps_all,
+                                                          float* __restrict__ tri_grad, int use_abs) {
+    constexpr int kEdge = 4;
+    using Part = PartOfTile<kEdge>;
+    static_assert(Part::kPixels == 16, "a row of 16 lanes holds a part's pixels");
+    __shared__ PtRecLds L;
+    __shared__ float s_sum[kBatch * 16], s_out[kBatch * 21];
+    __shared__ uint32_t s_pend[kBatch];
+    const uint32_t gtile = blockIdx.x / Part::kParts;
+    const Part pt(blockIdx.x % Part::kParts);
+    const int item = item_of_tile(items, nitems, gtile);
+    const BatchItem& B = items[item];
+    const ViewUniforms& U = B.U;
+    const float4* __restrict__ dimage = reinterpret_cast<const float4*>(targets[item].dimage);
+    if (dimage == nullptr) return;
+    if (kAbs != (use_abs && B.cell_col != nullptr)) return;  // as in k_pt_adjoint
+    const PixelState ps = item_pixel_state(ps_all, B);
+    const int tile = (int)(gtile - B.tile0);
+    const int lane = threadIdx.x, row = lane >> 4, p16 = lane & 15;
+    const int lx = pt.x0 + p16 % kEdge, ly = pt.y0 + p16 / kEdge;
+    const int cbit = kTileEdge * ly + lx;  // the pixel's bit in a record's coverage mask
+    const int x = (tile % U.tiles_x) * kTileEdge + lx, y = (tile / U.tiles_x) * kTileEdge + ly;
+    const bool valid = x < U.width && y < U.height;
+    const float px = 2.0f * (((float)x + 0.5f) / (float)U.width) - 1.0f;
+    const float py = 2.0f * (((float)y + 0.5f) / (float)U.height) - 1.0f;
+    const uint2 rg = ranges[gtile];
+    const int P = U.width * U.height;
+    const int pix = valid ? pixel_index(U, x, y) : 0;
+    float Cw = 1.0f;
+    float dC[3] = {0.f, 0.f, 0.f}, D = 0.f;  // dL/dC: RGB, and the alpha behind the current fragment
+    uint32_t n = 0;
+    CheckpointCursor ck;
+    if (valid) {
+        Cw = ps.ray_color[pix].w;
+        n = ps.frag_count[pix];
+        ck.start((int)ps.num_ckpt[pix], n, Cw, P, ps, pix);
+        const float4 di = dimage[pix];
+        dC[0] = di.x;
+        dC[1] = di.y;
+        dC[2] = di.z;
+        D = di.w * (1.0f - U.clear[3]) - (di.x * U.clear[0] + di.y * U.clear[1] + di.z * U.clear[2]);
+    }
+    if (ballot(valid && n > 0) == 0ull) return;
+    const int qs = row_scatter_index(lane);  // this lane's term of the row's sums (15: none)
+    const bool per_cell = B.cell_col != nullptr;
+    const int64_t slot0 = (int64_t)B.block0 * 256;
+    PartFeed<kEdge, true> feed{stream.recs, stream.route->vals, stream.route->masks, rg.x, rg.y, pt.origin, {}};
+    uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t idx = 0u;
+    PtRecData R;
+    feed.load(lane);
+    int nnxt = feed.next(s_pend, lane, rec, idx);
+    if (lane < nnxt) pt_fetch(pt_vert, pt_col, slot0, rec, R);
+    while (nnxt > 0) {
+        const int cnt = nnxt;
+        if (lane < cnt) pt_store(slot0, rec, R, L, lane);
+        feed.load(lane);
+        nnxt = feed.next(s_pend, lane, rec, idx);
+        __syncthreads();
+        for (int j0 = 0; j0 < cnt; j0 += 4) {
+            // Rows without a record left, and pixels that the record does not cover, run along and contribute zeros.
+            const bool has = j0 + row < cnt;
+            const int j = has ? j0 + row : j0;
+            const bool live = has & valid & (((L.mask[cbit >> 5][j] >> (cbit & 31)) & 1u) != 0u);
+            PtFrag f;
+            pt_eval(L, j, px, py, f);
+            const uint64_t lives = ballot(live) >> p16;  // bit 16 k: row k's record covers this lane's pixel
+            float q;
+            {
 #pragma clang fp contract(fast)
-            const int j = e / 3, k = e - 3 * j;
-            float S[5], gl[3];
-#pragma unroll
-            for (int q = 0; q < 5; q++) S[q] = s_acc[0][16 * j + 5 * k + q];
-#pragma unroll
-            for (int m = 0; m < 3; m++) {
-                gl[m] = S[4] * L.d[m][j];
-                // per-cell colours are the same at every corner, and sum_m grad lambda_m = 0
-                if (!per_cell)
-                    gl[m] += (S[0] * L.c[4 * m][j] + S[1] * L.c[4 * m + 1][j]) +
-                             (S[2] * L.c[4 * m + 2][j] + S[3] * L.c[4 * m + 3][j]);
+                const float a = 1.0f - f.A;
+                q = dC[0] * (a * f.c[0]) + dC[1] * (a * f.c[1]) + dC[2] * (a * f.c[2]);
             }
-            const float X0 = L.X[0][j], X1 = L.X[1][j], X2 = L.X[2][j];
-            const float Y0 = L.Y[0][j], Y1 = L.Y[1][j], Y2 = L.Y[2][j];
-            const float iD = L.invD[j];
-            out[7 * e] = -(gl[0] * (Y1 - Y2) + gl[1] * (Y2 - Y0) + gl[2] * (Y0 - Y1)) * iD;
-            out[7 * e + 1] = -(gl[0] * (X2 - X1) + gl[1] * (X0 - X2) + gl[2] * (X1 - X0)) * iD;
+            float Tmine = 0.f, Dmine = 0.f;
 #pragma unroll
-            for (int q = 0; q < 5; q++) out[7 * e + 2 + q] = S[q];
+            for (int k = 0; k < 4; k++) {
+                const float Ak = __shfl(f.A, 16 * k + p16, 64), qk = __shfl(q, 16 * k + p16, 64);
+                const bool lv = (lives >> (16 * k)) & 1ull;
+                float Tin = Cw < kPtTinyT ? 0.0f : div_nr(Cw, Ak);
+                const bool at_ckpt = lv && ck.n1 == n - 1u;
+                Tin = at_ckpt ? ck.t1 : Tin;
+                Tmine = row == k ? Tin : Tmine;
+                Dmine = row == k ? D : Dmine;
+                {
+#pragma clang fp contract(fast)
+                    const float d3 = D * Ak - qk;
+                    D = lv ? d3 : D;
+                }
+                Cw = lv ? Tin : Cw;
+                n -= lv ? 1u : 0u;
+                if (at_ckpt) ck.advance(P, ps, pix);
+            }
+            float p[15], s[1];
+            pt_terms<kAbs>(f, live, Tmine, Dmine, dC, p);
+            row_reduce_scatter(p, s);
+            if (has && qs < 15) s_sum[16 * j + qs] = s[0];
         }
         __syncthreads();
-        wait_for_loads();
-        for (int e = lane; e < cnt * 21; e += 64) {
-            const float v = out[e];
-            const int j = e / 21;
-            if (v != 0.f) atomic_add_f32(&tri_grad[21 * (int64_t)L.id[j] + (e - 21 * j)], v);
-        }
+        if (lane < nnxt) pt_fetch(pt_vert, pt_col, slot0, rec, R);
+        pt_scatter(L, s_sum, s_out, cnt, per_cell, lane, tri_grad);
         __syncthreads();
     }
 }
@@ -1114,23 +1284,35 @@ void launch_pt_bin(const BatchItem* items, int nitems, int64_t nblocks, uint32_t
 
 void launch_pt_forward(const BatchItem* items, int nitems, int64_t ntiles, const uint32_t* order,
                        const float4* pt_vert, const float4* pt_col, RecordStream recs, const uint2* ranges,
-                       PixelState ps, hipStream_t s) {
+                       PixelState ps, int edge, hipStream_t s) {
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(k_pt_forward, dim3((unsigned)ntiles), dim3(64), 0, s, items, nitems, order, pt_vert, pt_col,
-                       recs, ranges, ps);
+    if (edge == 4)
+        hipLaunchKernelGGL(k_pt_forward<4>, dim3((unsigned)(4 * ntiles)), dim3(64), 0, s, items, nitems, order,
+                           pt_vert, pt_col, recs, ranges, ps);
+    else
+        hipLaunchKernelGGL(k_pt_forward<8>, dim3((unsigned)ntiles), dim3(64), 0, s, items, nitems, order, pt_vert,
+                           pt_col, recs, ranges, ps);
 }
 
 void launch_pt_adjoint(const BatchItem* items, const AdjointTarget* targets, int nitems, int64_t ntiles,
                        int64_t nblocks, const uint32_t* order, const uint32_t* pt_info, const float4* pt_vert,
                        const float4* pt_col, RecordStream recs, const uint2* ranges, PixelState ps, float* tri_grad,
-                       int64_t tri_grad_floats, int use_abs, hipStream_t s) {
+                       int64_t tri_grad_floats, int use_abs, int edge, hipStream_t s) {
     if (ntiles <= 0) return;
     fill_u32(reinterpret_cast<uint32_t*>(tri_grad), 0u, tri_grad_floats, s);
-    hipLaunchKernelGGL(k_pt_adjoint<false>, dim3((unsigned)ntiles), dim3(64), 0, s, items, targets, nitems, order,
-                       pt_vert, pt_col, recs, ranges, ps, tri_grad, use_abs);
-    if (use_abs)
-        hipLaunchKernelGGL(k_pt_adjoint<true>, dim3((unsigned)ntiles), dim3(64), 0, s, items, targets, nitems, order,
+    if (edge == 4) {
+        hipLaunchKernelGGL(k_pt_adjoint_parts<false>, dim3((unsigned)(4 * ntiles)), dim3(64), 0, s, items, targets,
+                           nitems, pt_vert, pt_col, recs, ranges, ps, tri_grad, use_abs);
+        if (use_abs)
+            hipLaunchKernelGGL(k_pt_adjoint_parts<true>, dim3((unsigned)(4 * ntiles)), dim3(64), 0, s, items, targets,
+                               nitems, pt_vert, pt_col, recs, ranges, ps, tri_grad, use_abs);
+    } else {
+        hipLaunchKernelGGL(k_pt_adjoint<false>, dim3((unsigned)ntiles), dim3(64), 0, s, items, targets, nitems, order,
                            pt_vert, pt_col, recs, ranges, ps, tri_grad, use_abs);
+        if (use_abs)
+            hipLaunchKernelGGL(k_pt_adjoint<true>, dim3((unsigned)ntiles), dim3(64), 0, s, items, targets, nitems,
+                               order, pt_vert, pt_col, recs, ranges, ps, tri_grad, use_abs);
+    }
     if (nblocks > 0)
         hipLaunchKernelGGL(k_pt_backprop, dim3((unsigned)(4 * nblocks)), dim3(64), 0, s, items, targets, nitems,
                            pt_info, tri_grad);

@@ -35,6 +35,12 @@ __device__ __forceinline__ RecordIn load_record(const uint4* __restrict__ recs, 
     return r;
 }
 
+__device__ __forceinline__ void load_record(const uint4* __restrict__ recs, uint32_t i, RecordIn& r) {
+    r = load_record(recs, i);
+}
+// As a record of one uint4 (the Projection renderer's).
+__device__ __forceinline__ void load_record(const uint4* __restrict__ recs, uint32_t i, uint4& r) { r = recs[i]; }
+
 // Stages record r in slot i (world-space data only: the coverage was decided at binning).
 // Vertex data of one record, fetched ahead of its staging so that the loads overlap other work.  (On CDNA one
 // counter tracks loads and stores alike: a load issued after the gradient atomics would wait for them too.)
@@ -232,8 +238,9 @@ struct PartFeed {
         }
     }
     // The next batch, from the candidates load requested: lane j < the returned count gets record j and its index.
-    // pend: 32 words of LDS.
-    __device__ __forceinline__ int next(uint32_t* pend, int lane, RecordIn& r, uint32_t& idx) {
+    // pend: 32 words of LDS.  Record: RecordIn, or uint4 (the Projection renderer's).
+    template <typename Record>
+    __device__ __forceinline__ int next(uint32_t* pend, int lane, Record& r, uint32_t& idx) {
         const uint64_t lt = lanemask_lt();
         int cnt = 0;
         while (end != begin) {
@@ -265,7 +272,7 @@ struct PartFeed {
         __syncthreads();
         if (lane < cnt) {
             idx = pend[lane];
-            r = load_record(recs, order[idx]);
+            load_record(recs, order[idx], r);
         }
         return cnt;
     }
