@@ -329,6 +329,8 @@ __device__ __forceinline__ float div_nr(float x, float y) {
     return __builtin_fmaf(__builtin_fmaf(-q, y, x), r, q);
 }
 
+constexpr float kLog2e = 1.44269504f;  // the sub-segments' exp(-a t) = 2^(-a t log2 e), t log2 e once per fragment
+
 // The 4 sub-segments of a segment of length 4 tSeg between the entry and exit colours (RGB + density):
 // seg[s] = accumulateLinearConst of sub-segment s (ForwardCommon.glsl:42-49, colour endpoints mixed at s/4 and
 // (s+1)/4, density at the midpoint, IntersectRasterization.glsl:228-241), pre[s] = their composite before s,
@@ -344,6 +346,7 @@ __device__ __forceinline__ void sub_segments_ex(float4 col0, float4 col1, float 
                                                 float ia_s[4]) {
 #pragma clang fp contract(fast)
     const float dx = col1.x - col0.x, dy = col1.y - col0.y, dz = col1.z - col0.z, dw = col1.w - col0.w;
+    const float t2 = tSeg * kLog2e;
     float4 rc = make_float4(0.f, 0.f, 0.f, 1.0f);
 #pragma unroll
     for (int s = 0; s < 4; s++) {
@@ -355,7 +358,7 @@ __device__ __forceinline__ void sub_segments_ex(float4 col0, float4 col1, float 
         A_s[s] = 1.0f;
         ia_s[s] = 0.0f;
         if (!(a < 1e-6f)) {
-            const float A = __expf(-a * tSeg);
+            const float A = __builtin_amdgcn_exp2f(-a * t2);
             const float ia = fast_rcp(a);
             // accumulateLinearConst: (1 - A) c0 + ((tSeg + 1/a) A - 1/a) (c0 - c1), c0 - c1 = -(c1 - c0) / 4
             const float kq = -0.25f * ((tSeg + ia) * A - ia);
@@ -380,13 +383,14 @@ __device__ __forceinline__ void sub_segments(float4 col0, float4 col1, float tSe
     sub_segments_ex(col0, col1, tSeg, att, seg, pre, F, a_s, A_s, ia_s);
 }
 
-// The scalar part of sub_segments_ex: per sub-segment s the density a[s], transmittance A[s], 1 / a, the weight
-// kq[s] of the colour step in its colour (seg[s].rgb = (1 - A[s]) c0_s + kq[s] (col1 - col0), c0_s = col0 + s/4
+// The scalar part of sub_segments_ex: per sub-segment s the density a[s], transmittance A[s], 1 / a, four times the
+// weight of the colour step in its colour (seg[s].rgb = (1 - A[s]) c0_s + k4[s] / 4 (col1 - col0), c0_s = col0 + s/4
 // (col1 - col0)) and the transmittance T[s] before it; returns the fragment's transmittance.
 __device__ __forceinline__ float sub_segments_w(float4 col0, float4 col1, float tSeg, float att, float a_s[4],
-                                                float A_s[4], float ia_s[4], float kq_s[4], float T_s[4]) {
+                                                float A_s[4], float ia_s[4], float k4_s[4], float T_s[4]) {
 #pragma clang fp contract(fast)
     const float dw = col1.w - col0.w;
+    const float t2 = tSeg * kLog2e;
     float T = 1.0f;
 #pragma unroll
     for (int s = 0; s < 4; s++) {
@@ -395,14 +399,14 @@ __device__ __forceinline__ float sub_segments_w(float4 col0, float4 col1, float 
         a_s[s] = a;
         A_s[s] = 1.0f;
         ia_s[s] = 0.0f;
-        kq_s[s] = 0.0f;
+        k4_s[s] = 0.0f;
         T_s[s] = T;
         if (!(a < 1e-6f)) {
-            const float A = __expf(-a * tSeg);
+            const float A = __builtin_amdgcn_exp2f(-a * t2);
             const float ia = fast_rcp(a);
             A_s[s] = A;
             ia_s[s] = ia;
-            kq_s[s] = -0.25f * ((tSeg + ia) * A - ia);
+            k4_s[s] = ia - (tSeg + ia) * A;
         }
         T = T * A_s[s];
     }
@@ -410,18 +414,19 @@ __device__ __forceinline__ float sub_segments_w(float4 col0, float4 col1, float 
 }
 
 // sub_segments_ex's F alone: the RGB composite sum_s T[s] seg[s].rgb is col0 times sum_s T[s] (1 - A[s]) plus
-// (col1 - col0) times sum_s T[s] ((1 - A[s]) s/4 + kq[s]): two scalar sums instead of a composite per channel.
+// (col1 - col0) / 4 times sum_s T[s] ((1 - A[s]) s + k4[s]): two scalar sums instead of a composite per channel.
 __device__ __forceinline__ float4 sub_segments_F(float4 col0, float4 col1, float tSeg, float att) {
 #pragma clang fp contract(fast)
-    float a_s[4], A_s[4], ia_s[4], kq_s[4], T_s[4];
-    const float Tend = sub_segments_w(col0, col1, tSeg, att, a_s, A_s, ia_s, kq_s, T_s);
-    float S0 = 0.f, S1 = 0.f;
+    float a_s[4], A_s[4], ia_s[4], k4_s[4], T_s[4];
+    const float Tend = sub_segments_w(col0, col1, tSeg, att, a_s, A_s, ia_s, k4_s, T_s);
+    float S0 = 1.0f - A_s[0], S1 = k4_s[0];
 #pragma unroll
-    for (int s = 0; s < 4; s++) {
+    for (int s = 1; s < 4; s++) {
         const float om = 1.0f - A_s[s];
         S0 += T_s[s] * om;
-        S1 += T_s[s] * (om * ((float)s * 0.25f) + kq_s[s]);
+        S1 += T_s[s] * (om * (float)s + k4_s[s]);
     }
+    S1 *= 0.25f;
     return make_float4(S0 * col0.x + S1 * (col1.x - col0.x), S0 * col0.y + S1 * (col1.y - col0.y),
                        S0 * col0.z + S1 * (col1.z - col0.z), Tend);
 }
@@ -718,39 +723,41 @@ __device__ __forceinline__ void frag_backward_exact(const FragEval& E, const Rec
                                                     float3_& Q1) {
 #pragma clang fp contract(fast)
     const float tSeg = ((E.t1 - E.t0) / 4.0f) * tscale;
-    float a_s[4], A_s[4], ia_s[4], kq_s[4], T_s[4];
+    float a_s[4], A_s[4], ia_s[4], k4_s[4], T_s[4];
     // as in eval_fragment: not kept live since phase A
-    float Tn = sub_segments_w(E.col0, E.col1, tSeg, att, a_s, A_s, ia_s, kq_s, T_s);
+    float Tn = sub_segments_w(E.col0, E.col1, tSeg, att, a_s, A_s, ia_s, k4_s, T_s);
     // dF.rgb is the same for every sub-segment: sum over RGB of dF c0 (sub-segment s starts at col0 + s/4
-    // (col1 - col0)) = p0 + (s/4) p1, and of dF (c0 - c1) = -p1 / 4
+    // (col1 - col0)) = p0 + s p1, and of dF (c0 - c1) = -p1
     const float p0 = (dF.x * E.col0.x + dF.y * E.col0.y) + dF.z * E.col0.z;
-    const float p1 = (dF.x * (E.col1.x - E.col0.x) + dF.y * (E.col1.y - E.col0.y)) + dF.z * (E.col1.z - E.col0.z);
-    const float tp = 0.25f * tSeg * p1;
+    const float p1 = 0.25f * ((dF.x * (E.col1.x - E.col0.x) + dF.y * (E.col1.y - E.col0.y)) +
+                              dF.z * (E.col1.z - E.col0.z));
+    const float tp = tSeg * p1;
     // Sub-segment s, with T the transmittance before it, Tn = T A the one behind it and D the derivative with respect
-    // to the latter (as alpha): its colour is (1 - A) c0 + K (c0 - c1), A = exp(-a t), K = (t + 1/a) A - 1/a = -4 kq,
+    // to the latter (as alpha): its colour is (1 - A) c0 + K (c0 - c1), A = exp(-a t), K = (t + 1/a) A - 1/a = -k4,
     // with dA/dt = -a A, dA/da = -t A, dK/dt = -a t A, dK/da = -(K / a + t^2 A).  Hence, with
-    // h = Tn (D + dF c0 + (t/4) p1), dL/dt = a h, dL/da = t h - p1 T kq / a, and the weights of the entry and exit
-    // colours are those of the composite (sub_segments_F): sum T (1 - A), and sum T ((1 - A) s/4 + kq).
+    // h = Tn (D + dF c0 + t p1), dL/dt = a h, dL/da = t h - p1 T k4 / a, and the weights of the entry and exit
+    // colours are those of the composite (sub_segments_F): sum T (1 - A), and sum T ((1 - A) s + k4) / 4.
     float S0 = 0.f, S1 = 0.f, St = 0.f, Sa = 0.f, Sb = 0.f;
     float D = dF.w;
 #pragma unroll
     for (int s = 3; s >= 0; s--) {
-        const float fb = (float)s * 0.25f, fm = ((float)s + 0.5f) * 0.25f;
+        const float fm = ((float)s + 0.5f) * 0.25f;
         const float a = a_s[s], T = T_s[s];
         const float om = 1.0f - A_s[s];
-        const float sc0 = p0 + fb * p1;
-        const float Tom = T * om, Tk = T * kq_s[s];
+        const float sc0 = s > 0 ? p0 + (float)s * p1 : p0;
+        const float Tom = T * om, Tk = T * k4_s[s];
         float h = Tn * (D + (sc0 + tp));
         h = a < 1e-6f ? 0.0f : h;  // an empty sub-segment
         const float da = tSeg * h - p1 * (ia_s[s] * Tk);
         S0 += Tom;
-        S1 += fb * Tom + Tk;
+        S1 += s > 0 ? (float)s * Tom + Tk : Tk;
         St += a * h;
         Sa += da;
         Sb += fm * da;
-        D = D * A_s[s] - (om * sc0 + kq_s[s] * p1);
+        D = D * A_s[s] - (om * sc0 + k4_s[s] * p1);
         Tn = T;
     }
+    S1 *= 0.25f;
     const float w0 = S0 - S1;
     dcol0[0] = w0 * dF.x;
     dcol0[1] = w0 * dF.y;
