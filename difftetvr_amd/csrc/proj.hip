@@ -510,8 +510,8 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
         }
         // the coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
-        const uint32_t total = build_fragment_list(F.entry, rank_mask, mask, false, lane);
         const uint32_t nmine = (uint32_t)__popc(mask);
+        const uint32_t total = build_fragment_list<kBatch * 64>(F.entry, rank_mask, mask, lane);
         RankCursor cur_e;
         __syncthreads();
         for (uint32_t r0 = 0; r0 < total; r0 += kPtRound) {

@@ -28,16 +28,21 @@ namespace dtv {
 
 constexpr int kRoundDefault = 128;          // fragments shaded per round of the forward (segments per pass)
 constexpr int kRoundAdj = 64;               // fragments per round in the adjoint: one per lane
-constexpr int kMaxFrags = kBatch * 64;      // fragments a batch can produce
 constexpr float kMissMarker = -1.0f;        // transmittance slot of a fragment whose ray missed the tet
 constexpr float kTinyT = 0x1p-100f;         // transmittance below which a fragment's input is not recovered
 
-// The forward's fragment list and round values (kRound fragments shaded per round).
+// The forward's fragment list and round values (kRound fragments shaded per round).  The forward waits on latency (the
+// long dependent chain of one fragment's evaluation) more than on issue slots: with the records, rounds of 128 and less
+// take 10 KB of LDS and 128 registers, so that four waves fit in each SIMD (a CU has 160 KB).  For that a batch of more
+// than kFwdFrags fragments is listed and shaded in several goes, ray directions move between lanes by permute, and the
+// vertex indices stay out of the staged records.  Against three waves (13.4 KB, 140 registers): a render of 5.3M tets
+// at 1920 x 1080 4.80 -> 4.24 ms, a burst of 24 server requests 8.82 -> 7.60 ms, the step of 1.57M tets at 1024 x 1024
+// 6.91 -> 6.62 ms.
+constexpr int kFwdFrags = 1024;
 template <int kRound>
 struct FragListLds {
-    uint16_t entry[kMaxFrags];  // (pixel lane << 5) | record index
+    uint16_t entry[kFwdFrags];  // (pixel lane << 5) | record index
     float4 val[kRound];         // fragment colour F
-    float rd[3][64];            // ray direction of each pixel
 };
 
 // The adjoint's: with the records, 13 KB per wave, so that three waves fit in each SIMD (a CU has 160 KB).  A
@@ -88,12 +93,8 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
     const bool valid = lane < pt.kPixels && x < U.width && y < U.height;
     if (kPart && ballot(valid) == 0ull) return;
     const float3_ ro = f3(U.camPos[0], U.camPos[1], U.camPos[2]);
-    {
-        const float3_ rd = ray_direction(U, x, y);
-        F.rd[0][lane] = rd.x;
-        F.rd[1][lane] = rd.y;
-        F.rd[2][lane] = rd.z;
-    }
+    const float3_ my_rd = ray_direction(U, x, y);
+    const float my_scale = seg_scale(U, my_rd);
     const float att = U.attenuation;
     const uint2 rg = ranges[gtile];
     const int P = U.width * U.height;
@@ -111,8 +112,8 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
     PartFeed<kEdge, false> feed{recs, rec_of, stream.route->masks, rg.x, rg.y, pt.origin, {}};
     uint32_t ahead = 0u;  // this lane's record of the batch after nxt's
     // a part's batch: the stream indices of its records (the entries of a part fill at most half the list)
-    static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kMaxFrags / 2, "no room for a part's indices");
-    uint32_t* const part_idx = reinterpret_cast<uint32_t*>(F.entry + kMaxFrags / 2);
+    static_assert(!kPart || PartOfTile<kEdge>::kPixels * kBatch <= kFwdFrags / 2, "no room for a part's indices");
+    uint32_t* const part_idx = reinterpret_cast<uint32_t*>(F.entry + kFwdFrags / 2);
     uint32_t* const pend = part_idx + kBatch;
     uint32_t cur_idx = 0u, nxt_idx = 0u;
     int ncur = 0, nnxt = 0;
@@ -162,19 +163,22 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
         }
         // the records' coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
-        const uint32_t total = build_fragment_list(F.entry, rank_mask, mask, false, lane);
-        const uint32_t nmine = (uint32_t)__popc(mask);
+        do {  // one list, or several where the batch has more fragments than it holds
+        const uint32_t before = (uint32_t)__popc(mask);
+        const uint32_t total = build_fragment_list<kFwdFrags>(F.entry, rank_mask, mask, lane);
+        const uint32_t nmine = before - (uint32_t)__popc(mask);
         RankCursor cur_e;
         __syncthreads();
         for (uint32_t r0 = 0; r0 < total; r0 += kRound) {
-            for (int i = lane; i < kRound; i += 64) {
-                const uint32_t e = r0 + i;
-                if (e >= total) break;
-                const uint32_t ent = F.entry[e];
+            for (uint32_t i0 = 0; i0 < (uint32_t)kRound && r0 + i0 < total; i0 += 64) {
+                // lanes behind the list's end evaluate the last fragment again
+                const uint32_t i = i0 + lane;
+                const uint32_t ent = F.entry[min(r0 + i, total - 1u)];
                 const int pl = ent >> 5, j = ent & 31;
-                const float3_ rdp = f3(F.rd[0][pl], F.rd[1][pl], F.rd[2][pl]);
+                const float3_ rdp = lane_ray(my_rd, pl);
+                const float tscale = U.linear_depth ? __shfl(my_scale, pl, 64) : 1.0f;
                 FragEval E;
-                eval_fragment<kCell, false>(L, j, ro, rdp, att, seg_scale(U, rdp), E);
+                eval_fragment<kCell, false>(L, j, ro, rdp, att, tscale, E);
                 F.val[i] = E.hit ? E.F : make_float4(0.f, 0.f, 0.f, kMissMarker);
             }
             __syncthreads();
@@ -217,6 +221,7 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
             }
             __syncthreads();
         }
+        } while (ballot(mask != 0u) != 0ull);
         if (ballot(!done) == 0ull) break;
     }
     if (valid) {
@@ -248,7 +253,7 @@ __device__ __forceinline__ uint32_t claim_tile(uint32_t* __restrict__ queue) {
 // kQueue = false: one workgroup per tile of the launch order.  kQueue = true: as many workgroups as the GPU
 // holds at once, each claiming the next tile of the launch order from `queue` until all ntiles are taken.
 template <bool kCell, int kRound, bool kSub, bool kQueue>
-__global__ __launch_bounds__(64) void k_render_forward(const BatchItem* __restrict__ items, int nitems,
+__global__ __launch_bounds__(64, kRound > 128 ? 3 : 4) void k_render_forward(const BatchItem* __restrict__ items, int nitems,
                                                         const uint32_t* __restrict__ order,
                                                         RecordStream stream,
                                                         const uint2* __restrict__ ranges, PixelState ps_all,
@@ -268,7 +273,7 @@ __global__ __launch_bounds__(64) void k_render_forward(const BatchItem* __restri
 
 // (8 / kEdge)^2 workgroups per tile, one per part, in image order.
 template <bool kCell, int kEdge>
-__global__ __launch_bounds__(64) void k_render_forward_parts(const BatchItem* __restrict__ items, int nitems,
+__global__ __launch_bounds__(64, 4) void k_render_forward_parts(const BatchItem* __restrict__ items, int nitems,
                                                               RecordStream stream,
                                                               const uint2* __restrict__ ranges, PixelState ps_all) {
     __shared__ RecordLds L;
@@ -297,7 +302,7 @@ template <bool kRef, bool kCell, bool kSub, int kEdge = kTileEdge>
 __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items,
                                              const AdjointTarget* __restrict__ targets, int nitems,
                                              RecordStream stream, const uint2* __restrict__ ranges,
-                                             const PixelState& ps_all, int use_abs, uint32_t gsub, RecordLds& L,
+                                             const PixelState& ps_all, int use_abs, uint32_t gsub, RecordVidLds& L,
                                              AdjFragLds& A, float4 (&s_seg)[kRef ? 3 : 1][kRoundAdj],
                                              uint32_t part = 0u) {
     constexpr bool kPart = kEdge < kTileEdge;
@@ -747,7 +752,7 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint(const Batch
                                                         const uint2* __restrict__ ranges, PixelState ps_all,
                                                         int use_abs, uint32_t* __restrict__ queue,
                                                         uint32_t ntiles) {
-    __shared__ RecordLds L;
+    __shared__ RecordVidLds L;
     __shared__ AdjFragLds A;
     __shared__ float4 s_seg[kRef ? 3 : 1][kRoundAdj];  // reference mode: sub-segment colours, then their adjoints
     if constexpr (!kQueue) {
@@ -769,7 +774,7 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint_parts(const
                                                                            RecordStream stream,
                                                                            const uint2* __restrict__ ranges,
                                                                            PixelState ps_all, int use_abs) {
-    __shared__ RecordLds L;
+    __shared__ RecordVidLds L;
     __shared__ AdjFragLds A;
     __shared__ float4 s_seg[kRef ? 3 : 1][kRoundAdj];
     constexpr uint32_t kParts = PartOfTile<kEdge>::kParts;

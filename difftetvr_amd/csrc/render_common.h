@@ -1,5 +1,7 @@
 // Record staging and per-fragment maths shared by the tile renderer's forward, adjoint and export kernels.
 #pragma once
+#include <type_traits>
+
 #include "dtv_kernels.h"
 #include "dtv_prims.h"
 #include "raster.h"
@@ -9,13 +11,17 @@ namespace dtv {
 constexpr int kTileEdge = 8;
 constexpr int kBatch = 32;  // records staged per batch (one 32-bit coverage mask per pixel)
 
-struct alignas(16) RecordLds {  // 16-byte aligned: vid[] is also read as int4
+struct alignas(16) RecordLds {
     float p[12][kBatch];      // tet vertex positions, [3*v + c]
     float c[16][kBatch];      // tet vertex colours, [4*v + ch]
     float N[12][kBatch];      // face plane normals cross(p1-p0, p2-p0), [3*f + c]
     float k[4][kBatch];       // dot(N, camPos) - dot(N, p0) per face
     uint32_t mask[2][kBatch]; // coverage of the tile's pixels 0-31 / 32-63 (pixel = ly * 8 + lx = lane)
     uint32_t meta[kBatch];    // bit 3: face normals point outward; bits 4-31: tet index (num_cells <= 2^28)
+};
+
+// With the tets' vertex indices (the adjoint's).
+struct RecordVidLds : RecordLds {
     int32_t vid[4][kBatch];
 };
 
@@ -70,9 +76,9 @@ __device__ __forceinline__ void fetch_record_data(const float* __restrict__ pos,
 
 // kStash (binning tiles larger than 8x8): stash [6][kBatch] int32 receives the record's face as the oriented
 // fixed-point screen triangle of binning (project_face + face_screen arithmetic), for subtile_masks.
-template <bool kStash = false>
+template <bool kStash = false, typename Lds>
 __device__ __forceinline__ void store_record(const ViewUniforms& U, const RecordIn& r, const RecordData& d,
-                                             RecordLds& L, int i, int32_t* stash = nullptr) {
+                                             Lds& L, int i, int32_t* stash = nullptr) {
     const uint4 rec = r.rec;
     const int32_t vid[4] = {(int32_t)r.vid.x, (int32_t)r.vid.y, (int32_t)r.vid.z, (int32_t)r.vid.w};
     const float3_* p = d.p;
@@ -85,7 +91,7 @@ __device__ __forceinline__ void store_record(const ViewUniforms& U, const Record
         L.c[4 * v + 1][i] = d.c[v].y;
         L.c[4 * v + 2][i] = d.c[v].z;
         L.c[4 * v + 3][i] = d.c[v].w;
-        L.vid[v][i] = vid[v];
+        if constexpr (std::is_same_v<Lds, RecordVidLds>) L.vid[v][i] = vid[v];
     }
     L.mask[0][i] = rec.y;
     L.mask[1][i] = rec.z;
@@ -951,26 +957,30 @@ __device__ __forceinline__ void frag_backward_reference(const FragEval& E, const
 }
 
 // Coverage masks -> dense fragment list ordered by (rank, pixel lane): rank r holds the r-th fragment (by record
-// index, ascending, or descending when `reverse`) of every pixel that has more than r, in lane order.  A round of
+// index, ascending) of every pixel that has more than r, in lane order.  A round of
 // the list then holds about one fragment per pixel, so the per-pixel compositing (or its inversion) that walks
 // each pixel's fragments in order takes few serial steps per round.  rank_mask[r] = the lanes with more than r
-// fragments (at most 32 ranks).  Returns the number of fragments.
-__device__ __forceinline__ uint32_t build_fragment_list(uint16_t* entry, uint64_t* rank_mask, uint32_t mask,
-                                                        bool reverse, int lane) {
+// fragments (at most 32 ranks).  Stops before a rank that would exceed kRoom entries (at least 64) and leaves its
+// fragments and the later ones in mask.  Returns the number of fragments listed.
+template <int kRoom>
+__device__ __forceinline__ uint32_t build_fragment_list(uint16_t* entry, uint64_t* rank_mask, uint32_t& mask,
+                                                        int lane) {
     const uint64_t lt = lanemask_lt();
     uint32_t m = mask;
     uint64_t act = ballot(m != 0u);
     uint32_t base = 0;
     for (int r = 0; act != 0ull; r++) {
+        if (kRoom < kBatch * 64 && base + (uint32_t)popc64(act) > (uint32_t)kRoom) break;
         if (m != 0u) {
-            const int j = reverse ? 31 - __clz(m) : __ffs(m) - 1;
+            const int j = __ffs(m) - 1;
             entry[base + (uint32_t)popc64(act & lt)] = (uint16_t)((lane << 5) | j);
-            m &= ~(1u << j);
+            m &= m - 1u;
         }
         if (lane == 0) rank_mask[r] = act;
         base += (uint32_t)popc64(act);
         act = ballot(m != 0u);
     }
+    mask = m;
     return base;
 }
 
