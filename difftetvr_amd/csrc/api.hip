@@ -314,11 +314,12 @@ bool make_uniforms(const dtv_camera& camera, const dtv_render_params& params, Vi
 }
 
 // Pixels per side that a wave of the tile renderer takes, by the number of 8x8 tiles: the GPU's 1,024 SIMDs hold
-// three such waves each, and below that the deepest tile's wave decides the time.  Measured on a step (forward,
-// loss, adjoint) of cube grids with waves of 8x8 / 4x4 / 2x2 pixels, us: 96 tiles 745 / 342 / 247, 256 tiles
-// 1315 / 549 / 379, 625 tiles 2361 / 962 / 842, 1,024 tiles 1193 / 599 / 625, 2,304 tiles 1718 / 1071 / 1367,
-// 4,096 tiles 2264 / 1862 / 2760, 5,000 tiles 3750 / 3054 / 3797, 9,216 tiles 2660 / 3232 / 5478.  (A batch's
-// records cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)
+// four such waves each (three in the adjoint), and below that the deepest tile's wave decides the time.  Measured on a
+// step (forward, loss, adjoint) of cube grids with waves of 8x8 / 4x4 / 2x2 pixels, us: 96 tiles 496 / 235 / 158,
+// 256 tiles 939 / 425 / 296, 625 tiles 880 / 422 / 382, 784 tiles 868 / 433 / 420, 1,024 tiles 857 / 457 / 477,
+// 2,304 tiles 1313 / 884 / 1148, 4,096 tiles 1791 / 1607 / 2360, 5,625 tiles 1822 / 1945 / 3060.  (A batch's records
+// cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)  Waves of 8x4 pixels were never
+// the best of the four.
 //
 // The Projection renderer's waves take 8x8 or 4x4 pixels.  Its adjoint gains the more (a wave's rows then share out
 // the records too) and keeps gaining where its forward no longer does, so each has its own line.  Measured, 8x8 / 4x4:
@@ -618,13 +619,7 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
     ClearList clear;
     // Each distinct gradient target (the items of one mesh share theirs) accumulates its vertex gradients in
     // zeroed interleaved rows (8 floats per vertex), folded into its gradients after the adjoint.
-    struct Fold {
-        float* acc;
-        int64_t V;
-        float* grad_pos;
-        float* grad_col;
-    };
-    std::vector<Fold> folds;
+    std::vector<VertexFold> folds;
     {
         std::unordered_map<const float*, int> first;  // grad_pos -> first item
         std::vector<int64_t> row0((size_t)n, -1);
@@ -650,7 +645,7 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         DTV_HIP(view->vacc.ensure(sizeof(float) * 8 * (size_t)(rows > 0 ? rows : 1)));
         float* base = view->vacc.as<float>();
         int64_t r = 0;
-        for (Fold& fo : folds) {
+        for (VertexFold& fo : folds) {
             fo.acc = base + 8 * r;
             r += fo.V;
         }
@@ -701,7 +696,7 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
                               use_abs_grad ? 1 : 0, adjoint_mode, view->colour_kinds, s, view->sub_tiles,
                               view->queued ? view->tile_queue() : nullptr, view->adjoint_edge);
     }
-    for (const Fold& fo : folds) launch_fold_vertex_grads(fo.acc, fo.V, fo.grad_pos, fo.grad_col, s);
+    launch_fold_vertex_grads(folds.data(), (int)folds.size(), s);
     view->mark(DTV_STAGE_ADJOINT, 1, s);
     DTV_HIP(hipGetLastError());
     return DTV_OK;

@@ -140,7 +140,15 @@ void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets,
                            uint32_t* queue = nullptr, int edge = 8);
 // Adds the tile renderer adjoint's interleaved accumulator rows acc [V][8] into grad_pos [V][3] and, unless
 // NULL, grad_col [V][4].
-void launch_fold_vertex_grads(const float* acc, int64_t V, float* grad_pos, float* grad_col, hipStream_t s);
+// One mesh's interleaved gradient rows (8 floats per vertex: xyz, rgba) and the gradients they are added to (grad_col
+// NULL: positions only).
+struct VertexFold {
+    const float* acc;
+    int64_t V;
+    float* grad_pos;
+    float* grad_col;
+};
+void launch_fold_vertex_grads(const VertexFold* folds, int n, hipStream_t s);
 void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
                              const uint2* ranges, PixelState ps, int max_per_pixel, int32_t* out_ids, hipStream_t s);
 

@@ -981,29 +981,69 @@ void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets,
                                   colour_kinds, queue, s);
 }
 
-// grad_pos[v] += acc[v][0..2], grad_col[v] += acc[v][3..6] (grad_col NULL: positions only).  One thread per
-// vertex, so plain read-modify-writes.
-__global__ __launch_bounds__(256) void k_fold_vertex_grads(const float4* __restrict__ acc, int64_t V,
-                                                           float* __restrict__ grad_pos,
-                                                           float* __restrict__ grad_col) {
-    const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (v >= V) return;
+// Up to kFolds meshes' folds in one launch: each is less work than a launch of its own costs (a batched step of five small
+// Delaunay balls 879 -> 871 us).
+constexpr int kFolds = 8;
+struct FoldList {
+    VertexFold fold[kFolds];
+    uint32_t block0[kFolds];  // first workgroup of each
+    int n;
+};
+
+// grad_pos[v] += acc[v][0..2], grad_col[v] += acc[v][3..6].  One thread per vertex, so plain read-modify-writes.
+__global__ __launch_bounds__(256) void k_fold_vertex_grads(FoldList list) {
+    int k = 0;
+#pragma unroll
+    for (int i = 1; i < kFolds; i++) k = i < list.n && blockIdx.x >= list.block0[i] ? i : k;
+    const VertexFold f = list.fold[k];
+    const int64_t v = (int64_t)(blockIdx.x - list.block0[k]) * 256 + threadIdx.x;
+    if (v >= f.V) return;
+    const float4* __restrict__ acc = reinterpret_cast<const float4*>(f.acc);
     const float4 a = acc[2 * v], b = acc[2 * v + 1];
-    grad_pos[3 * v + 0] += a.x;
-    grad_pos[3 * v + 1] += a.y;
-    grad_pos[3 * v + 2] += a.z;
-    if (grad_col != nullptr) {
-        grad_col[4 * v + 0] += a.w;
-        grad_col[4 * v + 1] += b.x;
-        grad_col[4 * v + 2] += b.y;
-        grad_col[4 * v + 3] += b.z;
+    f.grad_pos[3 * v + 0] += a.x;
+    f.grad_pos[3 * v + 1] += a.y;
+    f.grad_pos[3 * v + 2] += a.z;
+    if (f.grad_col != nullptr) {
+        f.grad_col[4 * v + 0] += a.w;
+        f.grad_col[4 * v + 1] += b.x;
+        f.grad_col[4 * v + 2] += b.y;
+        f.grad_col[4 * v + 3] += b.z;
     }
 }
 
-void launch_fold_vertex_grads(const float* acc, int64_t V, float* grad_pos, float* grad_col, hipStream_t s) {
-    if (V <= 0) return;
-    hipLaunchKernelGGL(k_fold_vertex_grads, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const float4*>(acc), V, grad_pos, grad_col);
+// Whether two folds write to a common float: such folds run one after the other.
+static bool folds_overlap(const VertexFold& a, const VertexFold& b) {
+    const float* at[2] = {a.grad_pos, a.grad_col};
+    const float* bt[2] = {b.grad_pos, b.grad_col};
+    for (int i = 0; i < 2; i++)
+        for (int j = 0; j < 2; j++) {
+            if (at[i] == nullptr || bt[j] == nullptr) continue;
+            const uintptr_t a0 = (uintptr_t)at[i], a1 = a0 + 4u * (uintptr_t)((3 + i) * a.V);
+            const uintptr_t b0 = (uintptr_t)bt[j], b1 = b0 + 4u * (uintptr_t)((3 + j) * b.V);
+            if (a0 < b1 && b0 < a1) return true;
+        }
+    return false;
+}
+
+void launch_fold_vertex_grads(const VertexFold* folds, int n, hipStream_t s) {
+    FoldList list;
+    uint32_t blocks = 0;
+    list.n = 0;
+    auto flush = [&] {
+        if (list.n > 0) hipLaunchKernelGGL(k_fold_vertex_grads, dim3(blocks), dim3(256), 0, s, list);
+        list.n = 0;
+        blocks = 0;
+    };
+    for (int i = 0; i < n; i++) {
+        if (folds[i].V <= 0) continue;
+        bool apart = list.n == kFolds;
+        for (int k = 0; k < list.n && !apart; k++) apart = folds_overlap(list.fold[k], folds[i]);
+        if (apart) flush();
+        list.fold[list.n] = folds[i];
+        list.block0[list.n++] = blocks;
+        blocks += (uint32_t)((folds[i].V + 255) / 256);
+    }
+    flush();
 }
 
 void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
