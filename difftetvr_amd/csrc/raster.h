@@ -10,7 +10,6 @@ namespace dtv {
 struct FaceBins {
     int32_t tx0, tx1, ty0, ty1;  // tile range of the face's pixel-centre bounding box (empty: tx0 > tx1)
     int32_t shift;               // log2 of the tile edge in pixels (3, 4 or 5)
-    ScreenTri S;
 };
 
 // Tile range of screen triangle S (its pixel-centre bounding box, clipped to the view).
@@ -21,21 +20,14 @@ __device__ __forceinline__ FaceBins screen_bins(const ViewUniforms& U, const Scr
     b.ty0 = 0;
     b.ty1 = -1;
     b.shift = U.tile_shift;
-    b.S = S;
     int32_t x0, x1, y0, y1;
-    tri_pixel_bbox(U, b.S, x0, x1, y0, y1);
+    tri_pixel_bbox(U, S, x0, x1, y0, y1);
     if (x0 > x1 || y0 > y1) return b;
     b.tx0 = x0 >> b.shift;
     b.tx1 = x1 >> b.shift;
     b.ty0 = y0 >> b.shift;
     b.ty1 = y1 >> b.shift;
     return b;
-}
-
-__device__ __forceinline__ FaceBins face_bins(const ViewUniforms& U, const ProjectedTet& T, int f) {
-    ScreenTri S;
-    face_screen(U, T, f, S);
-    return screen_bins(U, S);
 }
 
 // Edge e of the oriented screen triangle: E(px, py) = dx (py - Y_a) - dy (px - X_a) in 1/256-pixel units; a
@@ -144,15 +136,4 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
     for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
     return v;
 }
-__device__ __forceinline__ uint32_t wave_and_u32(uint32_t v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v &= __shfl_xor(v, d, 64);
-    return v;
-}
-__device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v |= __shfl_xor(v, d, 64);
-    return v;
-}
-
 }  // namespace dtv

@@ -75,7 +75,7 @@ __device__ __forceinline__ void fetch_record_data(const float* __restrict__ pos,
 }
 
 // kStash (binning tiles larger than 8x8): stash [6][kBatch] int32 receives the record's face as the oriented
-// fixed-point screen triangle of binning (project_face + face_screen arithmetic), for subtile_masks.
+// fixed-point screen triangle of binning (the same arithmetic), for subtile_masks.
 template <bool kStash = false, typename Lds>
 __device__ __forceinline__ void store_record(const ViewUniforms& U, const RecordIn& r, const RecordData& d,
                                              Lds& L, int i, int32_t* stash = nullptr) {

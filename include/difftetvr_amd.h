@@ -76,7 +76,8 @@ typedef struct dtv_render_params {
     int32_t renderer;                  /* DTV_RENDERER_TILE (0) or DTV_RENDERER_PROJECTION (1) */
     int32_t segments_per_pass;         /* ray segments the forward shades per round: 64, 128 (0 = default) or
                                           256 (no reference counterpart) */
-    int32_t tile_launch;               /* DTV_TILE_LAUNCH_GRID (0, default): one workgroup per 8x8 tile;
+    int32_t tile_launch;               /* DTV_TILE_LAUNCH_GRID (0, default): one workgroup per 8x8 tile, or
+                                          several per tile for viewports of few tiles;
                                           DTV_TILE_LAUNCH_QUEUE (1): a persistent grid of the workgroups the GPU
                                           holds at once takes the tiles in launch order from a device work queue
                                           (forward and adjoint; no reference counterpart) */
@@ -106,7 +107,7 @@ typedef struct dtv_render_params {
 
 typedef struct dtv_view_stats {
     int64_t num_triangles;    /* generated front faces (GenerateTrianglesIntersect.glsl:124) */
-    int64_t num_pairs;        /* (tile, face) records after binning */
+    int64_t num_pairs;        /* (tile, face) records after binning, each covering a pixel of its tile */
     int64_t num_tiles;
     int32_t sort_passes;      /* radix passes actually run */
     int32_t width, height;    /* viewport of the first item */
@@ -252,11 +253,11 @@ int dtv_view_records_overflowed(dtv_view* view, int32_t* out_overflowed, int64_t
  * dtv_render_adjoint).  No reference counterpart (the reference only has wall-clock opt_time,
  * pytests/train.py:366,434).  dtv_view_get_timings synchronises on the recorded events and returns the
  * milliseconds of the most recent call of each stage in out_ms[DTV_NUM_STAGES] (negative if not run). */
-#define DTV_STAGE_COUNT_PAIRS 0 /* projection, culling and record counting */
-#define DTV_STAGE_SCAN 1
-#define DTV_STAGE_EMIT 2
+#define DTV_STAGE_COUNT_PAIRS 0 /* the binning pass: projection, culling, exact coverage and the records */
+#define DTV_STAGE_SCAN 1 /* part of the binning pass: takes no time of its own */
+#define DTV_STAGE_EMIT 2 /* as DTV_STAGE_SCAN */
 #define DTV_STAGE_SORT 3
-#define DTV_STAGE_RANGES 4 /* tile ranges and the record gather (exact coverage masks) */
+#define DTV_STAGE_RANGES 4 /* tile ranges, and the coverage masks in sorted order where waves render parts of tiles */
 #define DTV_STAGE_FORWARD 5
 #define DTV_STAGE_ADJOINT 6
 #define DTV_NUM_STAGES 7
