@@ -1,11 +1,11 @@
 // Tile renderer and its adjoint on gfx950.
 //
-// One wave64 per 8x8 screen tile.  The tile's sorted (tile, face) records are consumed in batches of 32: each
-// lane stages one record in LDS (tet vertices, colours, face planes, fixed-point edge functions of the record's
-// face); every lane (pixel) then tests all 32 faces against its pixel centre, giving a 32-bit coverage mask.
-// A wave prefix sum turns the masks into a dense list of (pixel, record) fragments in LDS, and the expensive
+// One wave64 per 8x8 screen tile, or, for viewports of few tiles, several that take 4x4 or 2x2 pixels each.  The
+// tile's sorted (tile, face) records are consumed in batches of 32: each lane stages one record in LDS (tet vertices,
+// colours, face planes); the records' coverage masks, exact from binning, give every lane (pixel) a 32-bit mask of the
+// records that cover it.  The masks become a dense list of (pixel, record) fragments in LDS, and the expensive
 // per-fragment work (ray-tet intersection, barycentric colours, four sub-segment integrals; in the adjoint also
-// their derivatives) runs over that list with every lane busy, in rounds of 128.  Only the cheap per-pixel
+// their derivatives) runs over that list with every lane busy, in rounds.  Only the cheap per-pixel
 // compositing (or, in the adjoint, the inversion of the 'over' operator) walks each pixel's fragments in order.
 //
 // Reference maths (Data/Shaders/...):
@@ -17,8 +17,8 @@
 // The adjoint re-traverses each pixel back to front from the stored final colour, inverting the 'over'
 // operator per tet (the inversion of AdjointIntersectRasterization.glsl:213-228) and resetting to stored
 // checkpoints (every K fragments, and before any fragment that takes the transmittance below 1/8 of the last
-// checkpoint's) to bound inversion drift.  Gradients of the 4 tet vertices are reduced per record in LDS before one global
-// atomic per value.
+// checkpoint's) to bound inversion drift.  Gradients of the 4 tet vertices are reduced per record, then
+// per vertex of a batch, in LDS before one global atomic per value.
 #include <map>
 #include <mutex>
 
@@ -283,13 +283,14 @@ __global__ __launch_bounds__(64, 4) void k_render_forward_parts(const BatchItem*
                                                      blockIdx.x % kParts);
 }
 
-// What bounds it: vector instructions first (1,572,864 tets at 1024 x 1024, 110.0 M fragments: about 980 per round of 64
-// fragments, 85 to 90 % of the issue slots), then the LDS (64 % busy); memory traffic matters little, and three waves
-// per SIMD are all that the registers of a fragment's gradients allow.  So the phases are written for few
+// What bounds it: vector instructions and the LDS together (1,572,864 tets at 1024 x 1024, 110.0 M listed fragments: 1.82e9
+// instructions, about 970 per round of 64 fragments, 82 % of one per SIMD and four cycles; the LDS 67 % busy); memory
+// traffic matters little, and three waves per SIMD are all that the registers of a fragment's gradients allow (four, with
+// rows of a quarter round and 77 spills, made steps 2 to 10 % slower).  So the phases are written for few
 // instructions: A and C without branches, the checkpoint test of B as one comparison, the owners' row masks for both
 // halves of a round from one set of ballots, the flush as LDS additions of doubles (2.19e9 -> 2.02e9 instructions in
 // all, the whole step 7.80 -> 7.62 ms, and 1.02 to 1.04 times faster from 24K tets on), and the sub-segments' adjoint
-// as running sums shared with the composite (frag_backward_exact: a fragment's backward 537 -> 441 instructions; the
+// as running sums shared with the composite (frag_backward_exact: a fragment's backward 537 -> 432 instructions; the
 // step 7.04 -> 6.90 ms).
 //
 // kRef = false: exact derivative of the forward.  kRef = true: the reference's adjoint as written

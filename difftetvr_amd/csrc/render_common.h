@@ -189,8 +189,8 @@ __device__ __forceinline__ uint32_t lane_coverage(const RecordLds& L, int cnt, i
     return m;
 }
 
-// Waves of a part of a tile.  With fewer 8x8 tiles than the GPU has SIMDs, a wave per tile leaves most of the chip
-// idle while the deepest tile's wave runs alone.  A tile is then rendered by (8 / kEdge)^2 waves of kEdge x kEdge
+// Waves of a part of a tile.  With fewer 8x8 tiles than the GPU has room for waves, a wave per tile leaves part of the
+// chip idle while the deepest tile's wave runs alone.  A tile is then rendered by (8 / kEdge)^2 waves of kEdge x kEdge
 // pixels each.  A wave's batches hold only the records that cover its own pixels, picked from the tile's stream
 // by their coverage masks, 128 candidates at a time.
 template <int kEdge>
