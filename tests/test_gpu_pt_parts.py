@@ -16,9 +16,20 @@ pytestmark = pytest.mark.gpu
                                   (640, 512), (648, 512)])
 @pytest.mark.parametrize("kind", ["vertex", "cell", "dense", "abs"])
 def test_parts_equal_whole_tiles(gpu, size, kind):
+    _compare(size, kind, 14)
+
+
+# faces that cover whole tiles: batches with more fragments than the whole tile's list of 1,024 (listed in several
+# goes), and around its edge; 2,304 tiles (4x4 waves, whose lists always fit)
+@pytest.mark.parametrize("n", [2, 3, 5, 9])
+def test_lists_in_several_goes(gpu, n):
+    _compare((384, 384), "vertex", n, (0.5, 0.4, 0.9))
+
+
+def _compare(size, kind, n, eye=(0.7, -0.5, 1.6)):
     import difftetvr_amd as d
     W, H = size
-    w = meshgen.grid_workload(14, seed=5)
+    w = meshgen.grid_workload(n, seed=5)
     mesh = d.TetMesh()
     mesh.set_use_gradients(True)
     if kind in ("cell", "abs"):
@@ -32,7 +43,7 @@ def test_parts_equal_whole_tiles(gpu, size, kind):
     r.set_attenuation(200.0 if kind == "dense" else 1.0)
     r.set_viewport_size(W, H)
     r.set_camera_fovy(FOVY)
-    r.set_view_matrix(meshgen.look_at_view_matrix((0.7, -0.5, 1.6)))
+    r.set_view_matrix(meshgen.look_at_view_matrix(eye))
     dimg = torch.from_numpy(np.random.default_rng(1).standard_normal((H, W, 4)).astype(np.float32)).cuda()
     got = []
     for spp in (128, 64):
