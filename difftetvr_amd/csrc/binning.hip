@@ -7,6 +7,7 @@
 // written in (tet, face, tile) order and the stable sort keeps that order for equal depth keys.  The sort moves
 // record indices; the tile renderers read the records through them.
 #include "bin_block.h"
+#include "sort_plan.h"
 
 namespace dtv {
 
@@ -55,9 +56,9 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const SortRoute* __restrict
     const uint32_t shift = route->tile_shift;
     const int64_t n = run_count(n_cap, n_dev);
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t t = keys[i] >> shift;
-        if (i == 0 || keys[i - 1] >> shift != t) ranges[t].x = (uint32_t)i;
-        if (i == n - 1 || keys[i + 1] >> shift != t) ranges[t].y = (uint32_t)(i + 1);
+        const uint32_t t = tile_of_key(keys[i], shift);
+        if (i == 0 || tile_of_key(keys[i - 1], shift) != t) ranges[t].x = (uint32_t)i;
+        if (i == n - 1 || tile_of_key(keys[i + 1], shift) != t) ranges[t].y = (uint32_t)(i + 1);
         if constexpr (kMasks) {
             const uint4 r = recs[rec_len * ((int64_t)vals[i] + 1) - 1];
             masks[i] = make_uint2(r.y, r.z);

@@ -36,7 +36,7 @@ struct BinSlot {
 };
 // Where the sort left its result (written by its histogram kernel).
 struct SortRoute {
-    const uint32_t* keys;  // sorted compact keys; tile = key >> tile_shift
+    const uint32_t* keys;  // sorted compact keys; tile_of_key(key, tile_shift)
     const uint32_t* vals;  // sorted record indices
     uint2* masks;          // room for one coverage mask per sorted record
     uint32_t tile_shift;

@@ -6,6 +6,7 @@
 // (:682-696).  Stability makes equal keys keep their input order.
 #include "dtv_kernels.h"
 #include "dtv_prims.h"
+#include "sort_plan.h"
 
 namespace dtv {
 
@@ -64,26 +65,7 @@ void launch_clear(const ClearList& regions, const BatchItem* item, BatchItem* it
 // 32-bit keys; a compact key of more bits stays 64 bits wide until the digits sorted so far, which no later pass
 // reads, can be dropped.  Record indices are not read by pass 0 either: they are the positions.
 //   measured (1.57M tets at 1024 x 1024): histogram and 5 passes of 64-bit keys 468 us, and 4 passes 345 us
-struct SortPlan {
-    uint32_t dmin;
-    int dbits, total;  // bits of the depth difference and of the compact key
-    int passes;
-    int drop;          // low bits the 32-bit keys leave out
-    __device__ __forceinline__ int last_wide() const { return drop > 0 ? drop / 8 - 1 : 0; }  // last pass that reads 64 bits
-};
-
-__host__ __device__ inline int bits_of(uint32_t x) { return x == 0u ? 0 : 32 - __builtin_clz(x); }
 int sort_bits(uint32_t range) { return bits_of(range); }
-
-__host__ __device__ inline SortPlan plan_sort(uint32_t dmin, int dbits, int tbits) {
-    SortPlan p;
-    p.dmin = dmin;
-    p.dbits = tbits > 24 ? 32 : dbits;  // the dropped digits then never reach the tile bits
-    p.total = p.dbits + tbits;
-    p.passes = p.total <= 8 ? 1 : (p.total + 7) / 8;
-    p.drop = p.total > 32 ? 8 * ((p.total - 32 + 7) / 8) : 0;
-    return p;
-}
 
 int sort_max_passes(int tbits) { return plan_sort(0u, 32, tbits).passes; }
 
@@ -94,10 +76,6 @@ __device__ __forceinline__ SortPlan make_plan(const SortInput& in) {
     const BinSlot s = in.slots[lane_id()];
     const uint32_t lo = ~wave_max_u32(s.not_min), hi = wave_max_u32(s.max);
     return plan_sort(lo, hi > lo ? bits_of(hi - lo) : 0, in.tbits);
-}
-
-__device__ __forceinline__ uint64_t compact_key(uint64_t k, const SortPlan& p) {
-    return ((k >> 32) << p.dbits) | (uint64_t)((uint32_t)k - p.dmin);
 }
 
 constexpr int kSortBlock = 256, kSortWaves = kSortBlock / 64;
@@ -130,7 +108,7 @@ __global__ __launch_bounds__(256) void k_sort_histogram(SortInput in, uint32_t* 
         route->keys = reinterpret_cast<const uint32_t*>(odd ? in.keys2 : in.keys);
         route->vals = odd ? in.vals2 : in.vals;
         route->masks = reinterpret_cast<uint2*>(odd ? in.keys : in.keys2);
-        route->tile_shift = (uint32_t)(plan.dbits - plan.drop);
+        route->tile_shift = plan.tile_shift();
     }
     __syncthreads();
     const int w = threadIdx.x / 64;
@@ -371,7 +349,7 @@ int sort_records(const SortInput& in, uint32_t* hist, uint32_t* counters, uint32
     if (in.cap <= 0) return 0;
     const bool planned = in.slots != nullptr;
     const SortPlan plan = plan_sort(in.dmin, planned ? 32 : in.dbits, in.tbits);  // planned: the most passes
-    const int last_wide = plan.drop > 0 ? plan.drop / 8 - 1 : 0;
+    const int last_wide = plan.last_wide();
     const int64_t parts = sort_parts(in.cap);
     const int items = sort_items(in.cap);
     const int64_t words = 256 * parts;
