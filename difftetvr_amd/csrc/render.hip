@@ -23,6 +23,7 @@
 #include <mutex>
 
 #include "render_common.h"
+#include "vertex_table.h"
 
 namespace dtv {
 
@@ -639,7 +640,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
         // the kernel's.)
         {
             const int j = lane & 31, half = lane >> 5;
-            constexpr int kTab = 96;
+            constexpr int kTab = kFlushTab;
             // over entry and w, free after the rounds: sums[kTab][7], keys[kTab]
             double* sums = reinterpret_cast<double*>(&A.entry[0]);
             int32_t* keys = reinterpret_cast<int32_t*>(sums + 7 * kTab);
@@ -675,16 +676,8 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             for (int k = 0; k < 2; k++) {
                 if (!slot_live) continue;
                 const int32_t v = k == 0 ? v0 : v1;
-                int e = (int)(((uint32_t)v * 2654435761u) >> 24) * kTab >> 8;  // multiplicative hash -> [0, kTab)
-                for (int probe = 0; probe < kTab; probe++) {
-                    const int32_t old = atomicCAS(&keys[e], -1, v);
-                    if (old == -1 || old == v) {
-                        ent[k] = e;
-                        owner[k] = old == -1;
-                        break;
-                    }
-                    e = e + 1 == kTab ? 0 : e + 1;
-                }
+                ent[k] = vertex_entry<kTab, kFlushProbes>(
+                    v, owner[k], [&](int e, int32_t id) { return atomicCAS(&keys[e], -1, id); });
             }
 #pragma unroll
             for (int k = 0; k < 2; k++) {
@@ -721,7 +714,7 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
             }
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                    // a slot that found no entry (more than kTab distinct vertices) issues its own values
+                // a slot that found no entry issues its own values
                 if (!slot_live || ent[k] >= 0) continue;
                 const int64_t g = k == 0 ? v0 : v1;
 #pragma unroll
