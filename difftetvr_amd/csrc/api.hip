@@ -1185,8 +1185,8 @@ int dtv_tet_regularizer_grad(const dtv_mesh* mesh, float lambda, float beta, flo
     if (mesh->num_cells < 0 || (mesh->num_cells > 0 && (!mesh->cells || !mesh->positions)))
         return fail(DTV_ERR_INVALID_ARGUMENT, "dtv_tet_regularizer_grad: invalid mesh");
     if (!aligned16(mesh->cells)) return fail(DTV_ERR_INVALID_ARGUMENT, "dtv_tet_regularizer_grad: cells must be 16-byte aligned");
-    launch_tet_regularizer(mesh->cells, mesh->positions, mesh->num_cells, lambda, beta, grad_positions,
-                           reinterpret_cast<hipStream_t>(stream));
+    launch_tet_regularizer(mesh->cells, mesh->positions, mesh->num_cells, mesh->num_vertices, lambda, beta,
+                           grad_positions, reinterpret_cast<hipStream_t>(stream));
     DTV_HIP(hipGetLastError());
     return DTV_OK;
 }

@@ -191,7 +191,8 @@ void launch_mse(const float* img, const float* tgt, int64_t n, int64_t denom, fl
                 hipStream_t s);
 
 // regularizer.hip
-void launch_tet_regularizer(const int32_t* cells, const float* pos, int64_t T, float lambda, float beta,
+// V: the mesh's vertices (a rule of the launch looks at how many tets share one).
+void launch_tet_regularizer(const int32_t* cells, const float* pos, int64_t T, int64_t V, float lambda, float beta,
                             float* grad_pos, hipStream_t s);
 
 // api.hip: sets the message dtv_last_error() returns and passes the status code through.

@@ -9,37 +9,19 @@
 // and, as in the reference, S^{5/2} is clamped below at 1e-5 (this damps the gradient of small tets).
 // Gradients are accumulated (+=) into grad_positions.
 //
-// What bounds it: the float atomics.  One per value (12 a tet) go to the memory side at about 25 G/s, whatever
-// their addresses: 746 us for 1.57M tets, against about 20 us for the mesh's bytes.  Neighbouring tets of a mesh
+// What bounds it: the float atomics.  One per value (12 a tet), its wave's lanes at scattered addresses, go to the
+// memory side at about 25 G/s: 742 us for 1.57M tets, against about 20 us for the mesh's bytes.  Neighbouring tets of a mesh
 // file share most vertices, so a workgroup sums the tets of its range per vertex in LDS first (a hash table of
-// vertex ids) and issues one atomic per value of each distinct vertex.  The sums are doubles: on gfx950 an LDS
-// addition of doubles takes about half a cycle per lane, one of floats about four (146 us with float sums).
-// 25 us for the 1.57M tets of a 64^3 grid; 275 -> 35 us for a Delaunay ball of 401K tets; with the grid's tets
-// shuffled, 929 -> 772 us.
+// vertex ids) and issues one atomic per value of each distinct vertex, consecutive lanes to consecutive addresses (about
+// 180 G/s where every tet has its own vertices).  The sums are doubles: on gfx950 an LDS addition of doubles takes about
+// half a cycle per lane, one of floats about four (146 us with float sums).
+// 24 us for the 1.57M tets of a 64^3 grid; 272 -> 32 us for a Delaunay ball of 400K tets; with the grid's tets
+// shuffled, 930 -> 773 us, and with vertices of their own, 714 -> 105 us.
 #include "dtv_kernels.h"
 #include "dtv_prims.h"
+#include "vertex_table.h"
 
 namespace dtv {
-
-// Tets per thread.  A thread takes consecutive tets, so that the lanes of a wave, kRegPer tets apart, seldom add
-// to one vertex at once (LDS atomics on one address serialise).
-constexpr int kRegPer = 4;
-constexpr int kRegProbes = 8;
-
-// Entry of vertex v in the table keys[kTab] (-1 = free; created when absent), or -1 when the probed entries
-// belong to other vertices.  Sixteen consecutive ids lie in consecutive entries, so that the flush's lanes add to
-// consecutive addresses; the probes step from group to group.
-template <int kTab>
-__device__ __forceinline__ int reg_entry(int32_t* keys, int32_t v) {
-    const uint32_t h = ((uint32_t)v >> 4) * 2654435761u;
-    int e = (int)((h >> 16) & (uint32_t)(kTab / 16 - 1)) * 16 + (v & 15);
-    for (int p = 0; p < kRegProbes; p++) {
-        const int32_t old = atomicCAS(&keys[e], -1, v);
-        if (old == -1 || old == v) return e;
-        e = (e + 16) & (kTab - 1);
-    }
-    return -1;
-}
 
 __device__ __forceinline__ void reg_tet(const int32_t* __restrict__ cells, const float* __restrict__ pos, int64_t t,
                                         float lambda, float beta, int32_t vid[4], float3_ g[4]) {
@@ -80,13 +62,14 @@ __device__ __forceinline__ void reg_tet(const int32_t* __restrict__ cells, const
     }
 }
 
-// One workgroup sums kThreads * kRegPer consecutive tets.  A vertex that finds no entry (a mesh without locality
-// fills the table) adds its values to the gradient directly.
-template <int kThreads>
+// One workgroup sums kThreads * kPer consecutive tets.  A thread takes consecutive ones, so that the lanes of a wave, kPer
+// tets apart, seldom add to one vertex at once (LDS atomics on one address serialise).  A vertex that finds no
+// entry (a mesh without locality fills the table) adds its values to the gradient directly.
+template <int kThreads, int kPer>
 __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __restrict__ cells,
                                                               const float* __restrict__ pos, int64_t T, float lambda,
                                                               float beta, float* __restrict__ grad_pos) {
-    constexpr int kTab = kThreads * kRegPer;
+    constexpr int kTab = 4 * kThreads;
     __shared__ int32_t keys[kTab];
     __shared__ double sums[3 * kTab];
     for (int e = threadIdx.x; e < kTab; e += kThreads) {
@@ -94,15 +77,16 @@ __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __r
         sums[3 * e] = sums[3 * e + 1] = sums[3 * e + 2] = 0.0;
     }
     __syncthreads();
-    const int64_t t0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * kRegPer;
-    for (int i = 0; i < kRegPer; i++) {
+    const int64_t t0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * kPer;
+    for (int i = 0; i < kPer; i++) {
         if (t0 + i >= T) break;
         int32_t vid[4];
         float3_ g[4];
         reg_tet(cells, pos, t0 + i, lambda, beta, vid, g);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const int e = reg_entry<kTab>(keys, vid[k]);
+            const int e = grouped_entry<kTab, kRegProbes>(
+                vid[k], [&](int at, int32_t v) { return atomicCAS(&keys[at], -1, v); });
             if (e >= 0) {
                 lds_add_f64(&sums[3 * e + 0], g[k].x);
                 lds_add_f64(&sums[3 * e + 1], g[k].y);
@@ -124,18 +108,22 @@ __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __r
     }
 }
 
-// Ranges of 2,048 tets hold 0.40 distinct vertices a tet on a 64^3 cube grid (1,024 tets: 0.47), so the larger
-// workgroup issues fewer atomics; it is taken when its ranges still give every CU one.
-void launch_tet_regularizer(const int32_t* cells, const float* pos, int64_t T, float lambda, float beta,
+template <int kThreads, int kPer>
+static void launch_range(const int32_t* cells, const float* pos, int64_t T, float lambda, float beta, float* grad_pos,
+                         hipStream_t s) {
+    constexpr int64_t kRange = (int64_t)kThreads * kPer;
+    hipLaunchKernelGGL((k_tet_regularizer<kThreads, kPer>), dim3((unsigned)((T + kRange - 1) / kRange)), dim3(kThreads),
+                       0, s, cells, pos, T, lambda, beta, grad_pos);
+}
+
+void launch_tet_regularizer(const int32_t* cells, const float* pos, int64_t T, int64_t V, float lambda, float beta,
                             float* grad_pos, hipStream_t s) {
     if (T <= 0) return;
-    constexpr int64_t kLarge = 512 * kRegPer, kSmall = 256 * kRegPer;
-    if (T >= 256 * kLarge)
-        hipLaunchKernelGGL(k_tet_regularizer<512>, dim3((unsigned)((T + kLarge - 1) / kLarge)), dim3(512), 0, s,
-                           cells, pos, T, lambda, beta, grad_pos);
-    else
-        hipLaunchKernelGGL(k_tet_regularizer<256>, dim3((unsigned)((T + kSmall - 1) / kSmall)), dim3(256), 0, s,
-                           cells, pos, T, lambda, beta, grad_pos);
+    switch (regularizer_range(T, V).per) {
+        case 1: return launch_range<128, 1>(cells, pos, T, lambda, beta, grad_pos, s);
+        case 2: return launch_range<256, 2>(cells, pos, T, lambda, beta, grad_pos, s);
+        default: return launch_range<512, 4>(cells, pos, T, lambda, beta, grad_pos, s);
+    }
 }
 
 }  // namespace dtv
