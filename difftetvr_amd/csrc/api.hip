@@ -1048,7 +1048,7 @@ int dtv_view_export_fragments(dtv_view* view, const dtv_mesh* mesh, int32_t max_
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     DTV_HIP(hipSetDevice(view->ctx->device));
     launch_export_fragments(view->dItems.as<BatchItem>(), view->nitems(), view->total_subtiles, view->stream(),
-                            view->ranges.as<uint2>(), view->pixel_state(), max_per_pixel, out_ids, s);
+                            view->ranges.as<uint2>(), view->pixel_state(), view->sub_tiles, max_per_pixel, out_ids, s);
     DTV_HIP(hipGetLastError());
     return DTV_OK;
 }

@@ -150,7 +150,8 @@ struct VertexFold {
 };
 void launch_fold_vertex_grads(const VertexFold* folds, int n, hipStream_t s);
 void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
-                             const uint2* ranges, PixelState ps, int max_per_pixel, int32_t* out_ids, hipStream_t s);
+                             const uint2* ranges, PixelState ps, bool sub, int max_per_pixel, int32_t* out_ids,
+                             hipStream_t s);
 
 // proj.hip: the Projection renderer.  Per-tet buffers are indexed by the tet's slot in the batch's block grid
 // (block0 * 256 + tet): pt_info [slots], pt_vert / pt_col [5 * slots] (the five vertices' NDC xyz + thickness,

@@ -776,17 +776,19 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint_parts(const
                                             blockIdx.x / kParts, L, A, s_seg, blockIdx.x % kParts);
 }
 
-// Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.
+// Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.  It needs the records' ids and
+// coverage only (kSub: and their faces' vertices, to test the coverage of the 8x8 sub-tile); a batch's record words are
+// loaded a batch ahead, their indices two.
+template <bool kSub>
 __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __restrict__ items, int nitems,
                                                           RecordStream stream,
                                                           const uint2* __restrict__ ranges, PixelState ps_all,
                                                           int max_per_pixel, int32_t* __restrict__ out_ids_all) {
     __shared__ RecordLds L;
-    __shared__ int32_t s_stash[6 * kBatch];
+    __shared__ int32_t s_stash[kSub ? 6 * kBatch : 1];
     const uint32_t gsub = global_tile_of_block(nullptr);
     const BatchItem& B = items[item_of_sub(items, nitems, gsub)];
     const ViewUniforms& U = B.U;
-    const float* __restrict__ pos = B.pos;
     const uint4* __restrict__ recs = stream.recs;
     const uint32_t* __restrict__ rec_of = stream.route->vals;
     const PixelState ps = item_pixel_state(ps_all, B);
@@ -796,25 +798,32 @@ __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __rest
     const int lx = lane & 7, ly = lane >> 3;
     const int x = st.x0 + lx, y = st.y0 + ly;
     const bool valid = x < U.width && y < U.height;
-    int32_t* stash = U.tile_shift != 3 ? s_stash : nullptr;
     const uint2 rg = ranges[st.gtile];
     const int pix = valid ? pixel_index(U, x, y) : 0;
     const uint32_t last = valid ? ps.last_rec[pix] : 0u;
     int k = 0;
+    RecordIn cur;
+    uint32_t ahead = 0u;
+    if (lane < kBatch && rg.x + lane < rg.y) cur = load_record(recs, rec_of[rg.x + lane]);
+    if (lane < kBatch && rg.x + kBatch + lane < rg.y) ahead = rec_of[rg.x + kBatch + lane];
     for (uint32_t base = rg.x; base < rg.y; base += kBatch) {
         const int cnt = (int)min((uint32_t)kBatch, rg.y - base);
         if (lane < cnt) {
-            RecordData d;
-            const RecordIn r = load_record(recs, rec_of[base + lane]);
-            fetch_record_data(pos, nullptr, r, d);
-            if (stash != nullptr)
-                store_record<true>(U, r, d, L, lane, stash);
-            else
-                store_record<false>(U, r, d, L, lane, nullptr);
+            if constexpr (kSub) {
+                RecordData d;
+                fetch_record_data(B.pos, nullptr, cur, d);
+                store_record<true>(U, cur, d, L, lane, s_stash);
+            } else {
+                L.mask[0][lane] = cur.rec.y;
+                L.mask[1][lane] = cur.rec.z;
+            }
+            L.meta[lane] = cur.rec.x;
         }
+        if (lane < kBatch && base + kBatch + lane < rg.y) cur = load_record(recs, ahead);
+        if (lane < kBatch && base + 2 * kBatch + lane < rg.y) ahead = rec_of[base + 2 * kBatch + lane];
         __syncthreads();
-        if (stash != nullptr) {
-            subtile_masks(L, stash, cnt, x, y, valid, lane);
+        if constexpr (kSub) {
+            subtile_masks(L, s_stash, cnt, x, y, valid, lane);
             __syncthreads();
         }
         uint32_t m = valid ? lane_coverage(L, cnt, lane) : 0u;
@@ -822,8 +831,7 @@ __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __rest
             const int j = __ffs(m) - 1;
             m &= m - 1u;
             if (base + j >= last) break;
-            if (k < max_per_pixel)
-                out_ids[(int64_t)pix * max_per_pixel + k] = (int32_t)recs[2 * (int64_t)rec_of[base + j] + 1].x;
+            if (k < max_per_pixel) out_ids[(int64_t)pix * max_per_pixel + k] = (int32_t)L.meta[j];
             k++;
         }
         __syncthreads();
@@ -1041,10 +1049,11 @@ void launch_fold_vertex_grads(const VertexFold* folds, int n, hipStream_t s) {
 }
 
 void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
-                             const uint2* ranges, PixelState ps, int max_per_pixel, int32_t* out_ids, hipStream_t s) {
+                             const uint2* ranges, PixelState ps, bool sub, int max_per_pixel, int32_t* out_ids,
+                             hipStream_t s) {
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(k_export_fragments, dim3((unsigned)ntiles), dim3(64), 0, s, items, nitems, recs, ranges,
-                       ps, max_per_pixel, out_ids);
+    hipLaunchKernelGGL(sub ? k_export_fragments<true> : k_export_fragments<false>, dim3((unsigned)ntiles), dim3(64), 0, s,
+                       items, nitems, recs, ranges, ps, max_per_pixel, out_ids);
 }
 
 }  // namespace dtv
