@@ -217,7 +217,7 @@ struct dtv_view {
     bool projection = false;        // the last render ran the Projection renderer
     bool sub_tiles = false;         // the last render binned tiles larger than 8x8
     bool queued = false;            // the last render took its tiles from a work queue (the adjoint does too)
-    bool cost_ordered = true;       // the last render launched its tiles heaviest first
+    bool heaviest_first = true;     // the last render's parameters: whole tiles launch heaviest first
     // Pixels per side that a wave of the last render took (8: a tile, less: a part of one), and one of its adjoint takes.
     int edge = 8, adjoint_edge = 8;
     int64_t sorted_room = 0;        // the last render's records, or in planned mode the room for them
@@ -325,6 +325,11 @@ bool make_uniforms(const dtv_camera& camera, const dtv_render_params& params, Vi
 // the records too) and keeps gaining where its forward no longer does, so each has its own line.  Measured, 8x8 / 4x4:
 // render 96 tiles 158 / 114, 1,344 tiles 376 / 275, 2,304 tiles 360 / 316, 4,096 tiles 513 / 538; step 96 tiles
 // 451 / 222, 1,344 tiles 1098 / 562, 2,304 tiles 905 / 597, 4,096 tiles 1251 / 1113, 5,625 tiles 1196 / 1274.
+//
+// The reference adjoint, two waves per SIMD, has a line of its own for 4x4 pixels.  Its time with waves of 8x8 / 4x4, us, at
+// 3,136, 3,600 and 4,096 tiles: cube grid of 82,944 tets 1696 / 1708, 1787 / 1915, 1813 / 2156; of 384,000 tets 2917 / 2893,
+// 3024 / 3222, 2983 / 3591; ball of 8,000 points 1632 / 1450, 1675 / 1614, 1697 / 1824.
+constexpr int64_t kRefPartTiles = 3200;
 int wave_edge(const dtv_render_params& prm, int64_t tiles, bool adjoint = false) {
     if (prm.tile_launch != DTV_TILE_LAUNCH_GRID || (prm.tile_size != 0 && prm.tile_size != 8) ||
         (prm.segments_per_pass != 0 && prm.segments_per_pass != 128))
@@ -518,9 +523,9 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
     DTV_HIP(view->tile_frags.ensure(sizeof(uint32_t) * subtiles));
     DTV_HIP(view->tile_order.ensure(2 * sizeof(uint32_t) * subtiles));
     const int edge = wave_edge(*params, tiles);
-    view->cost_ordered = params->tile_order == 0 && edge == 8;
+    view->heaviest_first = params->tile_order == 0;
     // forward launch order: tiles by record count, heaviest first
-    const uint32_t* fwd_order = view->cost_ordered ? view->tile_order.as<uint32_t>() : nullptr;
+    const uint32_t* fwd_order = view->heaviest_first && edge == 8 ? view->tile_order.as<uint32_t>() : nullptr;
     view->mark(DTV_STAGE_RANGES, 0, s);
     launch_tile_ranges(&scratch->route, K, n_dev, view->ranges.as<uint2>(), edge < 8 ? view->recs.as<uint4>() : nullptr,
                        proj ? 1 : 2, s);
@@ -671,14 +676,19 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
     }
     launch_clear(clear, nullptr, nullptr, targets.data(), staged ? 0 : n,
                  staged ? nullptr : view->dTargets.as<AdjointTarget>(), s);
-    // adjoint launch order: tiles by the forward's composited fragments, heaviest first
-    const uint32_t* adj_order = nullptr;
-    if (view->adjoint_edge < view->edge)  // the coverage masks that a part's wave picks its records by
+    const bool ref_whole = adjoint_mode == DTV_ADJOINT_REFERENCE && view->total_tiles > kRefPartTiles;
+    const int edge = ref_whole ? 8 : view->adjoint_edge;
+    if (edge < view->edge)  // the coverage masks that a part's wave picks its records by
         launch_tile_ranges(&view->scratch()->route, view->sorted_room,
                            view->sorted_planned ? &view->scratch()->total : nullptr, view->ranges.as<uint2>(),
                            view->recs.as<uint4>(), view->projection ? 1 : 2, s);
-    if (view->cost_ordered && view->adjoint_edge == 8) {
+    // launch order of whole tiles: by the forward's composited fragments, heaviest first (a forward that took parts of
+    // tiles left them per pixel only)
+    const uint32_t* adj_order = nullptr;
+    if (view->heaviest_first && edge == 8) {
         uint32_t* o = view->tile_order.as<uint32_t>() + view->total_subtiles;
+        if (view->edge < 8)
+            launch_tile_frags(view->dItems.as<BatchItem>(), view->nitems(), view->total_subtiles, ps, s);
         launch_tile_order(nullptr, view->tile_frags.as<uint32_t>(), view->total_subtiles, o, s);
         adj_order = o;
     }
@@ -689,12 +699,12 @@ int adjoint_batch(dtv_view* view, const AdjointTarget* tg, int n, int32_t use_ab
         launch_pt_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n, view->total_tiles,
                           view->total_blocks, adj_order, view->pt_info.as<uint32_t>(), view->pt_vert.as<float4>(),
                           view->pt_col.as<float4>(), view->stream(), view->ranges.as<uint2>(), ps,
-                          view->tri_grad.as<float>(), tg_floats, use_abs_grad ? 1 : 0, view->adjoint_edge, s);
+                          view->tri_grad.as<float>(), tg_floats, use_abs_grad ? 1 : 0, edge, s);
     } else {
         launch_render_adjoint(view->dItems.as<BatchItem>(), view->dTargets.as<AdjointTarget>(), n,
                               view->total_subtiles, adj_order, view->stream(), view->ranges.as<uint2>(), ps,
                               use_abs_grad ? 1 : 0, adjoint_mode, view->colour_kinds, s, view->sub_tiles,
-                              view->queued ? view->tile_queue() : nullptr, view->adjoint_edge);
+                              view->queued ? view->tile_queue() : nullptr, edge);
     }
     launch_fold_vertex_grads(folds.data(), (int)folds.size(), s);
     view->mark(DTV_STAGE_ADJOINT, 1, s);

@@ -170,6 +170,24 @@ __global__ __launch_bounds__(256) void k_subtile_cost(const BatchItem* __restric
     cost[g] = r.y - r.x;
 }
 
+// tile_frags[g] = fragments composited in 8x8 sub-tile g, from the pixels' counts.  One wave per sub-tile.
+__global__ __launch_bounds__(64) void k_tile_frags(const BatchItem* __restrict__ items, int nitems,
+                                                   const uint32_t* __restrict__ frag_count,
+                                                   uint32_t* __restrict__ tile_frags) {
+    const BatchItem& B = items[item_of_sub(items, nitems, blockIdx.x)];
+    const ViewUniforms& U = B.U;
+    const int sub = (int)(blockIdx.x - B.sub0), lane = threadIdx.x;
+    const int x = 8 * (sub % U.sub_x) + (lane & 7), y = 8 * (sub / U.sub_x) + (lane >> 3);
+    const uint32_t n = x < U.width && y < U.height ? frag_count[B.pixel0 + (int64_t)y * U.width + x] : 0u;
+    const uint32_t all = wave_sum_u32(n);
+    if (lane == 0) tile_frags[blockIdx.x] = all;
+}
+
+void launch_tile_frags(const BatchItem* items, int nitems, int64_t nsub, PixelState ps, hipStream_t s) {
+    if (nsub <= 0) return;
+    hipLaunchKernelGGL(k_tile_frags, dim3((unsigned)nsub), dim3(64), 0, s, items, nitems, ps.frag_count, ps.tile_frags);
+}
+
 void launch_subtile_cost(const BatchItem* items, int nitems, int64_t nsub, const uint2* ranges, uint32_t* cost,
                          hipStream_t s) {
     if (nsub <= 0) return;

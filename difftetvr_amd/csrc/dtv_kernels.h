@@ -118,6 +118,8 @@ struct PixelState {
     unsigned long long* counters;  // optional (NULL): [0] += gradient float atomics issued by the adjoint
     uint32_t* tile_frags;   // [tiles of the batch] fragments composited per tile (written by the forward)
 };
+// ps.tile_frags from ps.frag_count (which a forward of parts of tiles does not write), for the batch's nsub sub-tiles.
+void launch_tile_frags(const BatchItem* items, int nitems, int64_t nsub, PixelState ps, hipStream_t s);
 // order (may be NULL = tile t in workgroup t): the tile each workgroup renders, from launch_tile_order.
 // colour_kinds: which colour storages the batch's items use (kColoursPerVertex | kColoursPerCell); one launch
 // per kind present, each rendering the tiles of its items.
