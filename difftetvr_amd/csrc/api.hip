@@ -463,6 +463,7 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
         clear.add(scratch, (int64_t)(offsetof(ViewScratch, cleared) / 4));
         clear.add(hist, 8 * 256 + 8);
         clear.add(view->ranges.p, 2 * tiles);
+        view->mark(DTV_STAGE_COUNT_PAIRS, 0, s);
         launch_clear(clear, n == 1 ? &items[0] : nullptr, n == 1 ? view->dItems.as<BatchItem>() : nullptr, nullptr, 0,
                      nullptr, s);
         const BinOut out{view->bin_status.as<uint64_t>(), scratch, view->keys.as<uint64_t>(), view->recs.as<uint4>(),
@@ -472,8 +473,8 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
                           view->pt_col.as<float4>(), small, out, s);
         else
             launch_bin(dI, n, blocks, small, out, s);
+        view->mark(DTV_STAGE_COUNT_PAIRS, 1, s);  // (of two passes the second, which made the records)
     };
-    view->mark(DTV_STAGE_COUNT_PAIRS, 0, s);
     int64_t K = planned ? view->planned_cap : view->record_room(rec_bytes);
     bin(K);
     uint32_t dmin = 0;
@@ -503,7 +504,6 @@ int render_batch(dtv_view* view, const dtv_render_item* in, int n, const dtv_ren
         view->num_pairs = -1;
         view->num_tris = -1;
     }
-    view->mark(DTV_STAGE_COUNT_PAIRS, 1, s);
     for (int stage : {DTV_STAGE_SCAN, DTV_STAGE_EMIT}) {  // part of the binning pass
         view->mark(stage, 0, s);
         view->mark(stage, 1, s);

@@ -253,7 +253,8 @@ int dtv_view_records_overflowed(dtv_view* view, int32_t* out_overflowed, int64_t
  * dtv_render_adjoint).  No reference counterpart (the reference only has wall-clock opt_time,
  * pytests/train.py:366,434).  dtv_view_get_timings synchronises on the recorded events and returns the
  * milliseconds of the most recent call of each stage in out_ms[DTV_NUM_STAGES] (negative if not run). */
-#define DTV_STAGE_COUNT_PAIRS 0 /* the binning pass: projection, culling, exact coverage and the records */
+#define DTV_STAGE_COUNT_PAIRS 0 /* the binning pass: projection, culling, exact coverage and the records (a render whose
+                                   records outgrow its buffers makes two and reports the second) */
 #define DTV_STAGE_SCAN 1 /* part of the binning pass: takes no time of its own */
 #define DTV_STAGE_EMIT 2 /* as DTV_STAGE_SCAN */
 #define DTV_STAGE_SORT 3
