@@ -315,20 +315,20 @@ bool make_uniforms(const dtv_camera& camera, const dtv_render_params& params, Vi
 
 // Pixels per side that a wave of the tile renderer takes, by the number of 8x8 tiles: the GPU's 1,024 SIMDs hold
 // four such waves each (three in the adjoint), and below that the deepest tile's wave decides the time.  Measured on a
-// step (forward, loss, adjoint) of cube grids with waves of 8x8 / 4x4 / 2x2 pixels, us: 96 tiles 496 / 235 / 158,
-// 256 tiles 939 / 425 / 296, 625 tiles 880 / 422 / 382, 784 tiles 868 / 433 / 420, 1,024 tiles 857 / 457 / 477,
-// 2,304 tiles 1313 / 884 / 1148, 4,096 tiles 1791 / 1607 / 2360, 5,625 tiles 1822 / 1945 / 3060.  (A batch's records
-// cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)  Waves of 8x4 pixels were never
-// the best of the four.
+// step (forward, loss, adjoint) of cube grids that fill the view, with waves of 8x8 / 4x4 / 2x2 pixels, us: 96 tiles
+// 496 / 235 / 158, 256 tiles 939 / 425 / 296, 625 tiles 880 / 422 / 382, 784 tiles 868 / 433 / 420, 1,024 tiles 857 /
+// 457 / 477, 2,304 tiles 1313 / 884 / 1148, 4,096 tiles 1791 / 1607 / 2360, 5,625 tiles 1822 / 1945 / 3060.  (A batch's
+// records cover fewer of a part's pixels, so parts stage each record about 1.8 and 4 times.)  Waves of 8x4 pixels were
+// never the best of the four.
 //
 // The Projection renderer's waves take 8x8 or 4x4 pixels.  Its adjoint gains the more (a wave's rows then share out
 // the records too) and keeps gaining where its forward no longer does, so each has its own line.  Measured, 8x8 / 4x4:
 // render 96 tiles 158 / 114, 1,344 tiles 376 / 275, 2,304 tiles 360 / 316, 4,096 tiles 513 / 538; step 96 tiles
 // 451 / 222, 1,344 tiles 1098 / 562, 2,304 tiles 905 / 597, 4,096 tiles 1251 / 1113, 5,625 tiles 1196 / 1274.
 //
-// The reference adjoint, two waves per SIMD, has a line of its own for 4x4 pixels.  Its time with waves of 8x8 / 4x4, us, at
-// 3,136, 3,600 and 4,096 tiles: cube grid of 82,944 tets 1696 / 1708, 1787 / 1915, 1813 / 2156; of 384,000 tets 2917 / 2893,
-// 3024 / 3222, 2983 / 3591; ball of 8,000 points 1632 / 1450, 1675 / 1614, 1697 / 1824.
+// The reference adjoint, two waves per SIMD, has a line of its own for 4x4 pixels.  Its time with waves of 8x8 / 4x4,
+// us, at 3,136, 3,600 and 4,096 tiles: cube grid of 82,944 tets 1696 / 1708, 1787 / 1915, 1813 / 2156; of 384,000 tets
+// 2917 / 2893, 3024 / 3222, 2983 / 3591; ball of 8,000 points 1632 / 1450, 1675 / 1614, 1697 / 1824.
 constexpr int64_t kRefPartTiles = 3200;
 int wave_edge(const dtv_render_params& prm, int64_t tiles, bool adjoint = false) {
     if (prm.tile_launch != DTV_TILE_LAUNCH_GRID || (prm.tile_size != 0 && prm.tile_size != 8) ||

@@ -140,8 +140,6 @@ void launch_render_adjoint(const BatchItem* items, const AdjointTarget* targets,
                            const uint32_t* order, RecordStream recs, const uint2* ranges, PixelState ps, int use_abs,
                            int mode, uint32_t colour_kinds, hipStream_t s, bool sub = false,
                            uint32_t* queue = nullptr, int edge = 8);
-// Adds the tile renderer adjoint's interleaved accumulator rows acc [V][8] into grad_pos [V][3] and, unless
-// NULL, grad_col [V][4].
 // One mesh's interleaved gradient rows (8 floats per vertex: xyz, rgba) and the gradients they are added to (grad_col
 // NULL: positions only).
 struct VertexFold {
@@ -150,6 +148,8 @@ struct VertexFold {
     float* grad_pos;
     float* grad_col;
 };
+// Adds the tile renderer adjoint's interleaved accumulator rows acc [V][8] of each fold into its grad_pos [V][3] and,
+// unless NULL, grad_col [V][4].
 void launch_fold_vertex_grads(const VertexFold* folds, int n, hipStream_t s);
 void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles, RecordStream recs,
                              const uint2* ranges, PixelState ps, bool sub, int max_per_pixel, int32_t* out_ids,

@@ -3,7 +3,7 @@
 // Each tet in view becomes 3 or 4 screen triangles, Shirley and Tuchman's classes, with the thickness at the
 // thick vertex taken from the crossing of two edges' projections (GenerateTrianglesVTK.glsl:129-403).  The
 // triangles go through the tile renderer's binning, radix sort and per-tile compositing: one (tile, triangle)
-// record per 8x8 tile the triangle may cover, keyed by the NDC z of the triangle's centroid
+// record per 8x8 tile with a pixel centre the triangle covers, keyed by the NDC z of the triangle's centroid
 // (ComputeTriangleDepths.glsl:99-108), composited front to back.  The reference blends the same list back to
 // front with premultiplied alpha, which sums the same terms.  Each fragment contributes (c.rgb alpha, alpha),
 // alpha = 1 - exp(-c.a d), where colour c and thickness d are interpolated linearly in screen space
@@ -514,55 +514,55 @@ __global__ __launch_bounds__(64) void k_pt_forward(const BatchItem* __restrict__
         // the coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
         do {  // one list, or several where the batch has more fragments than it holds
-        const uint32_t before = (uint32_t)__popc(mask);
-        const uint32_t total = build_fragment_list<kPart ? kBatch * 64 : kPtFrags>(F.entry, rank_mask, mask, lane);
-        const uint32_t nmine = before - (uint32_t)__popc(mask);
-        RankCursor cur_e;
-        __syncthreads();
-        for (uint32_t r0 = 0; r0 < total; r0 += kPtRound) {
-            for (int i = lane; i < kPtRound; i += 64) {
-                const uint32_t e = r0 + (uint32_t)i;
-                if (e >= total) break;
-                const uint32_t ent = F.entry[e];
-                const uint32_t pl = ent >> 5;
-                const int j = (int)(ent & 31u);
-                const float px = 2.0f * (((float)(x0 + (int)(pl % kEdge)) + 0.5f) / (float)U.width) - 1.0f;
-                const float py = 2.0f * (((float)(y0 + (int)(pl / kEdge)) + 0.5f) / (float)U.height) - 1.0f;
-                PtFrag f;
-                pt_eval(L, j, px, py, f);
-                const float a = 1.0f - f.A;
-                F.val[i] = make_float4(a * f.c[0], a * f.c[1], a * f.c[2], f.A);
-            }
+            const uint32_t before = (uint32_t)__popc(mask);
+            const uint32_t total = build_fragment_list<kPart ? kBatch * 64 : kPtFrags>(F.entry, rank_mask, mask, lane);
+            const uint32_t nmine = before - (uint32_t)__popc(mask);
+            RankCursor cur_e;
             __syncthreads();
-            uint32_t e;
-            while (cur_e.next(rank_mask, nmine, lt, r0 + kPtRound, e)) {
-                const float4 f = F.val[e - r0];
-                const float Tout = C.w * f.w;
-                // checkpoint rules of the tet renderer: before an underflow, and periodically
-                if (C.w >= kPtTinyT && Tout < kPtTinyT && nlast != n && (int)nck < U.max_ckpt) {
-                    ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
-                    ps.ckpt_n[(int64_t)nck * P + pix] = n;
-                    nck++;
-                    nlast = n;
+            for (uint32_t r0 = 0; r0 < total; r0 += kPtRound) {
+                for (int i = lane; i < kPtRound; i += 64) {
+                    const uint32_t e = r0 + (uint32_t)i;
+                    if (e >= total) break;
+                    const uint32_t ent = F.entry[e];
+                    const uint32_t pl = ent >> 5;
+                    const int j = (int)(ent & 31u);
+                    const float px = 2.0f * (((float)(x0 + (int)(pl % kEdge)) + 0.5f) / (float)U.width) - 1.0f;
+                    const float py = 2.0f * (((float)(y0 + (int)(pl / kEdge)) + 0.5f) / (float)U.height) - 1.0f;
+                    PtFrag f;
+                    pt_eval(L, j, px, py, f);
+                    const float a = 1.0f - f.A;
+                    F.val[i] = make_float4(a * f.c[0], a * f.c[1], a * f.c[2], f.A);
                 }
-                {
+                __syncthreads();
+                uint32_t e;
+                while (cur_e.next(rank_mask, nmine, lt, r0 + kPtRound, e)) {
+                    const float4 f = F.val[e - r0];
+                    const float Tout = C.w * f.w;
+                    // checkpoint rules of the tet renderer: before an underflow, and periodically
+                    if (C.w >= kPtTinyT && Tout < kPtTinyT && nlast != n && (int)nck < U.max_ckpt) {
+                        ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
+                        ps.ckpt_n[(int64_t)nck * P + pix] = n;
+                        nck++;
+                        nlast = n;
+                    }
+                    {
 #pragma clang fp contract(fast)
-                    C.x = C.x + C.w * f.x;
-                    C.y = C.y + C.w * f.y;
-                    C.z = C.z + C.w * f.z;
+                        C.x = C.x + C.w * f.x;
+                        C.y = C.y + C.w * f.y;
+                        C.z = C.z + C.w * f.z;
+                    }
+                    C.w = Tout;
+                    n++;
+                    last = (kPart ? part_idx[F.entry[e] & 31u] : base + (F.entry[e] & 31u)) + 1;
+                    if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kPtTinyT && (int)nck < U.max_ckpt - 1) {
+                        ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
+                        ps.ckpt_n[(int64_t)nck * P + pix] = n;
+                        nck++;
+                        nlast = n;
+                    }
                 }
-                C.w = Tout;
-                n++;
-                last = (kPart ? part_idx[F.entry[e] & 31u] : base + (F.entry[e] & 31u)) + 1;
-                if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kPtTinyT && (int)nck < U.max_ckpt - 1) {
-                    ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
-                    ps.ckpt_n[(int64_t)nck * P + pix] = n;
-                    nck++;
-                    nlast = n;
-                }
+                __syncthreads();
             }
-            __syncthreads();
-        }
         } while (!kPart && ballot(mask != 0u) != 0ull);
     }
     if (valid) {

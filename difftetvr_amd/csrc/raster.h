@@ -79,7 +79,8 @@ __device__ __forceinline__ bool pixel_inside(const int32_t X[3], const int32_t Y
     return in;
 }
 
-// Faces whose bounding box spans more tiles than this keep every tile of it (bounded per-thread work).
+// Binning tiles larger than 8x8: a face whose bounding box spans more tiles than this keeps every tile of it, untested;
+// the renderers test the coverage per pixel, so the records beyond the face cover nothing.
 constexpr int kMaxTestedTiles = 64;
 
 // Exact coverage of 8x8 tile (tx, ty): bit ly * 8 + lx is set when the centre of pixel (8 tx + lx, 8 ty + ly) is

@@ -10,13 +10,13 @@
 // Gradients are accumulated (+=) into grad_positions.
 //
 // What bounds it: the float atomics.  One per value (12 a tet), its wave's lanes at scattered addresses, go to the
-// memory side at about 25 G/s: 742 us for 1.57M tets, against about 20 us for the mesh's bytes.  Neighbouring tets of a mesh
-// file share most vertices, so a workgroup sums the tets of its range per vertex in LDS first (a hash table of
-// vertex ids) and issues one atomic per value of each distinct vertex, consecutive lanes to consecutive addresses (about
-// 180 G/s where every tet has its own vertices).  The sums are doubles: on gfx950 an LDS addition of doubles takes about
-// half a cycle per lane, one of floats about four (146 us with float sums).
-// 24 us for the 1.57M tets of a 64^3 grid; 272 -> 32 us for a Delaunay ball of 400K tets; with the grid's tets
-// shuffled, 930 -> 773 us, and with vertices of their own, 714 -> 105 us.
+// memory side at about 25 G/s: 742 us for 1.57M tets, against about 20 us for the mesh's bytes.  Neighbouring tets of a
+// mesh file share most vertices, so a workgroup sums the tets of its range per vertex in LDS first (a hash table of
+// vertex ids) and issues one atomic per value of each distinct vertex, consecutive lanes to consecutive addresses
+// (about 180 G/s where every tet has its own vertices).  The sums are doubles: on gfx950 an LDS addition of doubles
+// takes about half a cycle per lane, one of floats about four (146 us with float sums). 24 us for the 1.57M tets of a
+// 64^3 grid; 272 -> 32 us for a Delaunay ball of 400K tets; with the grid's tets shuffled, 930 -> 773 us, and with
+// vertices of their own, 714 -> 105 us.
 #include "dtv_kernels.h"
 #include "dtv_prims.h"
 #include "vertex_table.h"
@@ -62,8 +62,8 @@ __device__ __forceinline__ void reg_tet(const int32_t* __restrict__ cells, const
     }
 }
 
-// One workgroup sums kThreads * kPer consecutive tets.  A thread takes consecutive ones, so that the lanes of a wave, kPer
-// tets apart, seldom add to one vertex at once (LDS atomics on one address serialise).  A vertex that finds no
+// One workgroup sums kThreads * kPer consecutive tets.  A thread takes consecutive ones, so that the lanes of a wave,
+// kPer tets apart, seldom add to one vertex at once (LDS atomics on one address serialise).  A vertex that finds no
 // entry (a mesh without locality fills the table) adds its values to the gradient directly.
 template <int kThreads, int kPer>
 __global__ __launch_bounds__(kThreads) void k_tet_regularizer(const int32_t* __restrict__ cells,

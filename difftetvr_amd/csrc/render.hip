@@ -16,8 +16,8 @@
 //   early ray termination              PPLL/Forward.glsl:168-173
 // The adjoint re-traverses each pixel back to front from the stored final colour, inverting the 'over'
 // operator per tet (the inversion of AdjointIntersectRasterization.glsl:213-228) and resetting to stored
-// checkpoints (every K fragments, and before any fragment that takes the transmittance below 1/8 of the last
-// checkpoint's) to bound inversion drift.  Gradients of the 4 tet vertices are reduced per record, then
+// checkpoints (every K fragments, to bound inversion drift, and before a fragment that takes the transmittance below
+// kTinyT, whose input could not be recovered).  Gradients of the 4 tet vertices are reduced per record, then
 // per vertex of a batch, in LDS before one global atomic per value.
 #include <map>
 #include <mutex>
@@ -46,10 +46,11 @@ struct FragListLds {
     float4 val[kRound];         // fragment colour F
 };
 
-// The adjoint's: with the records, 13 KB per wave, so that three waves fit in each SIMD (a CU has 160 KB).  A
-// batch whose fragments exceed kAdjFrags is processed in two parts of 16 records; the per-fragment gradient rows
-// are reduced half a round (32 fragments) at a time; ray directions stay in registers and move between lanes by
-// permute.  The flush's vertex table spans entry and w, which are free by then.
+// The adjoint's: with the records, 13,312 B per wave.  The LDS is handed out in granules of 1,280 B, so a CU's 160 KB
+// hold 11 such workgroups (12 up to 12,800 B each), where the registers would allow three waves per SIMD.  A batch
+// whose fragments exceed kAdjFrags is processed in two parts of 16 records; the per-fragment gradient rows are reduced
+// half a round (32 fragments) at a time; ray directions stay in registers and move between lanes by permute.  The
+// flush's vertex table spans entry and w, which are free by then.
 constexpr int kAdjFrags = 1024;
 struct AdjFragLds {
     uint16_t entry[kAdjFrags];  // (pixel lane << 5) | record index, one part of a batch
@@ -165,63 +166,63 @@ __device__ __forceinline__ void forward_tile(const BatchItem* __restrict__ items
         // the records' coverage masks are consumed: their slots hold the list's rank masks
         uint64_t* rank_mask = reinterpret_cast<uint64_t*>(&L.mask[0][0]);
         do {  // one list, or several where the batch has more fragments than it holds
-        const uint32_t before = (uint32_t)__popc(mask);
-        const uint32_t total = build_fragment_list<kFwdFrags>(F.entry, rank_mask, mask, lane);
-        const uint32_t nmine = before - (uint32_t)__popc(mask);
-        RankCursor cur_e;
-        __syncthreads();
-        for (uint32_t r0 = 0; r0 < total; r0 += kRound) {
-            for (uint32_t i0 = 0; i0 < (uint32_t)kRound && r0 + i0 < total; i0 += 64) {
-                // lanes behind the list's end evaluate the last fragment again
-                const uint32_t i = i0 + lane;
-                const uint32_t ent = F.entry[min(r0 + i, total - 1u)];
-                const int pl = ent >> 5, j = ent & 31;
-                const float3_ rdp = lane_ray(my_rd, pl);
-                const float tscale = U.linear_depth ? __shfl(my_scale, pl, 64) : 1.0f;
-                FragEval E;
-                eval_fragment<kCell, false>(L, j, ro, rdp, att, tscale, E);
-                F.val[i] = E.hit ? E.F : make_float4(0.f, 0.f, 0.f, kMissMarker);
-            }
+            const uint32_t before = (uint32_t)__popc(mask);
+            const uint32_t total = build_fragment_list<kFwdFrags>(F.entry, rank_mask, mask, lane);
+            const uint32_t nmine = before - (uint32_t)__popc(mask);
+            RankCursor cur_e;
             __syncthreads();
-            uint32_t e;
-            while (!done && cur_e.next(rank_mask, nmine, lt, r0 + kRound, e)) {
-                if (U.use_ert && (1.0f - C.w) > U.ert_alpha) {
-                    done = true;
-                    break;
+            for (uint32_t r0 = 0; r0 < total; r0 += kRound) {
+                for (uint32_t i0 = 0; i0 < (uint32_t)kRound && r0 + i0 < total; i0 += 64) {
+                    // lanes behind the list's end evaluate the last fragment again
+                    const uint32_t i = i0 + lane;
+                    const uint32_t ent = F.entry[min(r0 + i, total - 1u)];
+                    const int pl = ent >> 5, j = ent & 31;
+                    const float3_ rdp = lane_ray(my_rd, pl);
+                    const float tscale = U.linear_depth ? __shfl(my_scale, pl, 64) : 1.0f;
+                    FragEval E;
+                    eval_fragment<kCell, false>(L, j, ro, rdp, att, tscale, E);
+                    F.val[i] = E.hit ? E.F : make_float4(0.f, 0.f, 0.f, kMissMarker);
                 }
-                const float4 f = F.val[e - r0];
-                // C.w is the transmittance T, the product of the fragments' transmittances (relative precision at
-                // any depth), so the adjoint recovers each fragment's input as T_out / T_f.  Only an underflow
-                // (T_out below kTinyT) cannot be inverted: a checkpoint goes before the fragment that causes it.
-                // The state before the first fragment (T = 1) needs no slot.  A missed fragment's value is
-                // (0, 0, 0, kMissMarker): with transmittance 1 it leaves the state as it is, without a branch.
-                const float Tout = C.w * (f.w != kMissMarker ? f.w : 1.0f);
-                if (C.w >= kTinyT && Tout < kTinyT && nlast != n && (int)nck < U.max_ckpt) {
-                    ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
-                    ps.ckpt_n[(int64_t)nck * P + pix] = n;
-                    nck++;
-                    nlast = n;
-                }
-                {
+                __syncthreads();
+                uint32_t e;
+                while (!done && cur_e.next(rank_mask, nmine, lt, r0 + kRound, e)) {
+                    if (U.use_ert && (1.0f - C.w) > U.ert_alpha) {
+                        done = true;
+                        break;
+                    }
+                    const float4 f = F.val[e - r0];
+                    // C.w is the transmittance T, the product of the fragments' transmittances (relative precision at
+                    // any depth), so the adjoint recovers each fragment's input as T_out / T_f.  Only an underflow
+                    // (T_out below kTinyT) cannot be inverted: a checkpoint goes before the fragment that causes it.
+                    // The state before the first fragment (T = 1) needs no slot.  A missed fragment's value is
+                    // (0, 0, 0, kMissMarker): with transmittance 1 it leaves the state as it is, without a branch.
+                    const float Tout = C.w * (f.w != kMissMarker ? f.w : 1.0f);
+                    if (C.w >= kTinyT && Tout < kTinyT && nlast != n && (int)nck < U.max_ckpt) {
+                        ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
+                        ps.ckpt_n[(int64_t)nck * P + pix] = n;
+                        nck++;
+                        nlast = n;
+                    }
+                    {
 #pragma clang fp contract(fast)
-                    C.x = C.x + C.w * f.x;
-                    C.y = C.y + C.w * f.y;
-                    C.z = C.z + C.w * f.z;
+                        C.x = C.x + C.w * f.x;
+                        C.y = C.y + C.w * f.y;
+                        C.z = C.z + C.w * f.z;
+                    }
+                    C.w = Tout;
+                    n++;
+                    last = (kPart ? part_idx[F.entry[e] & 31] : base + (F.entry[e] & 31)) + 1;
+                    // periodic checkpoints bound the rounding the adjoint's chain of divisions accumulates; the last
+                    // slot is kept for the underflow rule above
+                    if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kTinyT && (int)nck < U.max_ckpt - 1) {
+                        ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
+                        ps.ckpt_n[(int64_t)nck * P + pix] = n;
+                        nck++;
+                        nlast = n;
+                    }
                 }
-                C.w = Tout;
-                n++;
-                last = (kPart ? part_idx[F.entry[e] & 31] : base + (F.entry[e] & 31)) + 1;
-                // periodic checkpoints bound the rounding the adjoint's chain of divisions accumulates; the last
-                // slot is kept for the underflow rule above
-                if ((int)(n - nlast) >= U.ckpt_interval && C.w >= kTinyT && (int)nck < U.max_ckpt - 1) {
-                    ps.ckpt_t[(int64_t)nck * P + pix] = C.w;
-                    ps.ckpt_n[(int64_t)nck * P + pix] = n;
-                    nck++;
-                    nlast = n;
-                }
+                __syncthreads();
             }
-            __syncthreads();
-        }
         } while (ballot(mask != 0u) != 0ull);
         if (ballot(!done) == 0ull) break;
     }
@@ -284,15 +285,15 @@ __global__ __launch_bounds__(64, 4) void k_render_forward_parts(const BatchItem*
                                                      blockIdx.x % kParts);
 }
 
-// What bounds it: vector instructions and the LDS together (1,572,864 tets at 1024 x 1024, 110.0 M listed fragments: 1.82e9
-// instructions, about 970 per round of 64 fragments, 82 % of one per SIMD and four cycles; the LDS 67 % busy); memory
-// traffic matters little, and three waves per SIMD are all that the registers of a fragment's gradients allow (four, with
-// rows of a quarter round and 77 spills, made steps 2 to 10 % slower).  So the phases are written for few
-// instructions: A and C without branches, the checkpoint test of B as one comparison, the owners' row masks for both
-// halves of a round from one set of ballots, the flush as LDS additions of doubles (2.19e9 -> 2.02e9 instructions in
-// all, the whole step 7.80 -> 7.62 ms, and 1.02 to 1.04 times faster from 24K tets on), and the sub-segments' adjoint
-// as running sums shared with the composite (frag_backward_exact: a fragment's backward 537 -> 432 instructions; the
-// step 7.04 -> 6.90 ms).
+// What bounds it: vector instructions and the LDS together (1,572,864 tets at 1024 x 1024, 76.1 M listed fragments in
+// 1.32 M rounds: 1.82e9 instructions, about 1,380 a round of up to 64 fragments, 82 % of one per SIMD and four cycles;
+// the LDS 68 % busy); memory traffic matters little, and three waves per SIMD are all that the registers of a
+// fragment's gradients allow (10.7 of the 11 workgroups a CU that fit are resident; four waves, with rows of a quarter
+// round and 77 spills, made steps 2 to 10 % slower).  So the phases are written for few instructions: A and C without
+// branches, the checkpoint test of B as one comparison, the owners' row masks for both halves of a round from one set
+// of ballots, the flush as LDS additions of doubles (2.19e9 -> 2.02e9 instructions in all, the whole step 7.80 -> 7.62
+// ms, and 1.02 to 1.04 times faster from 24K tets on), and the sub-segments' adjoint as running sums shared with the
+// composite (frag_backward_exact: a fragment's backward 537 -> 432 instructions; the step 7.04 -> 6.90 ms).
 //
 // kRef = false: exact derivative of the forward.  kRef = true: the reference's adjoint as written
 // (AdjointIntersectRasterization.glsl:111-362): per pixel from the blended output image, back to front, the
@@ -736,8 +737,9 @@ __device__ __forceinline__ void adjoint_tile(const BatchItem* __restrict__ items
     }
 }
 
-// Waves per SIMD: 3 for the exact adjoint (168 VGPRs of the 512 per lane, 13 KB of LDS), 2 for the reference
-// one, whose sub-segment arrays need more of both.  kQueue as in k_render_forward.
+// Waves per SIMD that the registers allow: 3 for the exact adjoint (168 VGPRs of the 512 per lane; its 13,312 B of LDS
+// fit 11 times, not 12), 2 for the reference one, whose sub-segment arrays need more of both.  kQueue as in
+// k_render_forward.
 template <bool kRef, bool kCell, bool kSub, bool kQueue>
 __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint(const BatchItem* __restrict__ items,
                                                         const AdjointTarget* __restrict__ targets, int nitems,
@@ -776,9 +778,9 @@ __global__ __launch_bounds__(64, kRef ? 2 : 3) void k_render_adjoint_parts(const
                                             blockIdx.x / kParts, L, A, s_seg, blockIdx.x % kParts);
 }
 
-// Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.  It needs the records' ids and
-// coverage only (kSub: and their faces' vertices, to test the coverage of the 8x8 sub-tile); a batch's record words are
-// loaded a batch ahead, their indices two.
+// Ordered fragment export (tet*4 + face per covered record), up to max_per_pixel per pixel.  It needs the records' ids
+// and coverage only (kSub: and their faces' vertices, to test the coverage of the 8x8 sub-tile); a batch's record words
+// are loaded a batch ahead, their indices two.
 template <bool kSub>
 __global__ __launch_bounds__(64) void k_export_fragments(const BatchItem* __restrict__ items, int nitems,
                                                           RecordStream stream,
@@ -1052,7 +1054,8 @@ void launch_export_fragments(const BatchItem* items, int nitems, int64_t ntiles,
                              const uint2* ranges, PixelState ps, bool sub, int max_per_pixel, int32_t* out_ids,
                              hipStream_t s) {
     if (ntiles <= 0) return;
-    hipLaunchKernelGGL(sub ? k_export_fragments<true> : k_export_fragments<false>, dim3((unsigned)ntiles), dim3(64), 0, s,
+    const auto kernel = sub ? k_export_fragments<true> : k_export_fragments<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ntiles), dim3(64), 0, s,
                        items, nitems, recs, ranges, ps, max_per_pixel, out_ids);
 }
 

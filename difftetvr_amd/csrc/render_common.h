@@ -47,7 +47,6 @@ __device__ __forceinline__ void load_record(const uint4* __restrict__ recs, uint
 // As a record of one uint4 (the Projection renderer's).
 __device__ __forceinline__ void load_record(const uint4* __restrict__ recs, uint32_t i, uint4& r) { r = recs[i]; }
 
-// Stages record r in slot i (world-space data only: the coverage was decided at binning).
 // Vertex data of one record, fetched ahead of its staging so that the loads overlap other work.  (On CDNA one
 // counter tracks loads and stores alike: a load issued after the gradient atomics would wait for them too.)
 struct RecordData {
@@ -74,6 +73,7 @@ __device__ __forceinline__ void fetch_record_data(const float* __restrict__ pos,
     }
 }
 
+// Stages record r in slot i (world-space data only: the coverage was decided at binning).
 // kStash (binning tiles larger than 8x8): stash [6][kBatch] int32 receives the record's face as the oriented
 // fixed-point screen triangle of binning (the same arithmetic), for subtile_masks.
 template <bool kStash = false, typename Lds>
@@ -148,7 +148,7 @@ __device__ __forceinline__ void store_record(const ViewUniforms& U, const Record
 }
 
 // Coverage masks of the batch's records for this wave's 8x8 sub-tile (binning tiles larger than 8x8), from the
-// screen triangles store_record stashed: L.mask as the binning's gather writes it for 8x8 tiles.
+// screen triangles store_record stashed: L.mask as binning decides it for 8x8 tiles.
 __device__ __forceinline__ void subtile_masks(RecordLds& L, const int32_t* stash, int cnt, int x, int y,
                                               bool valid, int lane) {
     for (int j = 0; j < cnt; j++) {
@@ -320,13 +320,11 @@ __device__ __forceinline__ float3_ caxpy(float s, float3_ a, float3_ b) {  // s 
     return {s * a.x + b.x, s * a.y + b.y, s * a.z + b.z};
 }
 
-// The hardware's reciprocal, square root and reciprocal square root (about 1 ulp; one instruction each, where
-// x / y and sqrtf expand into correctly rounded sequences of ten or more).  Only for continuous quantities
+// The hardware's reciprocal (about 1 ulp; one instruction, where x / y expands into a correctly rounded sequence of
+// ten or more).  Only for continuous quantities
 // (colours, barycentrics, sub-segment opacity, gradients): no discrete decision may depend on them.
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float fast_div(float x, float y) { return x * __builtin_amdgcn_rcpf(y); }
-__device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 // x / y from the hardware reciprocal and one Newton correction of the quotient (residual by FMA): within about
 // half an ulp, for a chain of divisions whose errors compound.  Still not for discrete decisions.
 __device__ __forceinline__ float div_nr(float x, float y) {

@@ -31,12 +31,12 @@ DTV_HOST_DEVICE inline int vertex_entry(int32_t v, bool& created, Cas cas) {
     return -1;
 }
 
-// The adjoint's flush: up to 128 vertex slots a batch (32 records), about 18 distinct vertices where tets share them.  Where
-// every tet has its own the table overflows, and a slot that finds no entry issues its own atomics; probed to the end
-// the full table cost it 96 dependent compare-and-swaps.  Adjoint, us, with 160 entries that hold every slot / 96 probed
-// to the end / 96 with 4 / 8 / 16 probes, own vertices: 1,296 tets at 64^2 42 / 58 / 39 / 38 / 40, 24,576 at 512^2 561 /
-// 605 / 593 / 530 / 526, 1.57M at 1024^2 6536 / 6450 / 5777 / 5792 / 5911, ball of 2,000 points at 512^2 443 / 492 / 489 /
-// 447 / 438; with shared vertices 4, 8 and 16 differ by less than 3 %, 8 is best.
+// The adjoint's flush: up to 128 vertex slots a batch (32 records), about 18 distinct vertices where tets share them.
+// Where every tet has its own the table overflows, and a slot that finds no entry issues its own atomics; probed to the
+// end the full table cost it 96 dependent compare-and-swaps.  Adjoint, us, with 160 entries that hold every slot / 96
+// probed to the end / 96 with 4 / 8 / 16 probes, own vertices: 1,296 tets at 64^2 42 / 58 / 39 / 38 / 40, 24,576 at
+// 512^2 561 / 605 / 593 / 530 / 526, 1.57M at 1024^2 6536 / 6450 / 5777 / 5792 / 5911, ball of 2,000 points at 512^2
+// 443 / 492 / 489 / 447 / 438; with shared vertices 4, 8 and 16 differ by less than 3 %, 8 is best.
 constexpr int kFlushTab = 96, kFlushProbes = 8;
 
 // As vertex_entry, for the regulariser's larger tables: sixteen consecutive ids lie in consecutive entries, so that the
@@ -59,14 +59,14 @@ struct RegRange {
 };
 
 // A range of more tets has fewer distinct vertices a tet (of a 64^3 cube grid 2,048 tets have 0.40, 1,024 0.47), so it
-// issues fewer atomics, while a thread with more tets has a longer chain of table searches, and a table that the vertices
-// of its tets overfill merges nothing (it holds 4 a thread).  So: a tet a thread for small meshes and for those
-// whose tets share few vertices (two a tet on average, or more), else two, and four in larger workgroups where those
-// still give every CU one.
-// Measured, us, one atomic per value / 128 x 1 / 256 x 2 / 512 x 4 threads x tets: cube grids of 10,368 tets 12 / 4.0 / 5.7 /
-// 8.6, 82,944 43 / 5.2 / 5.7 / 8.7, 384,000 179 / 14 / 8.6 / 11, 1.57M 742 / 48 / 25 / 24; Delaunay balls of 12,666 tets 18 /
-// 5.0 / 7.9 / 12, 400,374 272 / 29 / 32 / 42; tets with vertices of their own, 1,536 of them 3.7 / 4.5 / 7.4 / 12, 41,472
-// 6.8 / 4.7 / 8.6 / 21, 6.3M 714 / 105 / 519 / 722; 24,576 tets of a grid in random order 20 / 10 / 14 / 20.
+// issues fewer atomics, while a thread with more tets has a longer chain of table searches, and a table that the
+// vertices of its tets overfill merges nothing (it holds 4 a thread).  So: a tet a thread for small meshes and for
+// those whose tets share few vertices (two a tet on average, or more), else two, and four in larger workgroups where
+// those still give every CU one.
+// Measured, us, one atomic per value / 128 x 1 / 256 x 2 / 512 x 4 threads x tets: cube grids of 10,368 tets 12 / 4.0 /
+// 5.7 / 8.6, 82,944 43 / 5.2 / 5.7 / 8.7, 384,000 179 / 14 / 8.6 / 11, 1.57M 742 / 48 / 25 / 24; Delaunay balls of
+// 12,666 tets 18 / 5.0 / 7.9 / 12, 400,374 272 / 29 / 32 / 42; 24,576 tets of a grid in random order 20 / 10 / 14 / 20;
+// tets with vertices of their own, 384 3.7 / 4.5 / 7.4 / 12, 10,368 6.8 / 4.7 / 8.6 / 21, 1.57M 714 / 105 / 519 / 722.
 inline RegRange regularizer_range(int64_t T, int64_t V) {
     if (T < (1 << 17) || V >= 2 * T) return {128, 1};
     return T < (1 << 19) ? RegRange{256, 2} : RegRange{512, 4};

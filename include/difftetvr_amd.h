@@ -70,14 +70,19 @@ typedef struct dtv_render_params {
     int32_t checkpoint_interval;       /* fragments between adjoint checkpoints; 0 = 64 */
     int32_t tile_order;                /* launch order of screen tiles (no reference counterpart: the reference
                                           rasterises): 0 = heaviest first (default; forward by record count,
-                                          adjoint by the forward's fragment count), 1 = row-major */
+                                          adjoint by the forward's fragment count), 1 = row-major.  Without effect
+                                          where waves render parts of tiles (tile_launch) */
     int32_t segment_length;            /* DTV_SEGMENT_EUCLIDEAN (INTERSECTION renderer) or
                                           DTV_SEGMENT_LINEAR_DEPTH (PPLL renderer) */
     int32_t renderer;                  /* DTV_RENDERER_TILE (0) or DTV_RENDERER_PROJECTION (1) */
     int32_t segments_per_pass;         /* ray segments the forward shades per round: 64, 128 (0 = default) or
                                           256 (no reference counterpart) */
     int32_t tile_launch;               /* DTV_TILE_LAUNCH_GRID (0, default): one workgroup per 8x8 tile, or
-                                          several per tile for viewports of few tiles;
+                                          several per tile, each rendering a part of it, for viewports of few
+                                          tiles (up to 5,120 in the batch; Projection forward 3,072, reference
+                                          adjoint 3,200).  Parts are taken with the default tile_size and
+                                          segments_per_pass only: other settings render whole tiles and are up
+                                          to three times slower there;
                                           DTV_TILE_LAUNCH_QUEUE (1): a persistent grid of the workgroups the GPU
                                           holds at once takes the tiles in launch order from a device work queue
                                           (forward and adjoint; no reference counterpart) */
