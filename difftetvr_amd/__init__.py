@@ -527,9 +527,10 @@ class Renderer:
         self._segments_per_pass = int(segments)
 
     def set_tile_launch(self, launch):
-        """How the tile kernels are launched: 'grid' (default: one workgroup per 8x8 tile) or 'queue' (a
-        persistent grid of the workgroups the GPU holds at once, taking the tiles in launch order from a device
-        work queue; the adjoint follows its render).  Images are identical either way.  No reference counterpart."""
+        """How the tile kernels are launched: 'grid' (default: one workgroup per 8x8 tile, or several for viewports
+        of few tiles, with the default tile size and segments per pass) or 'queue' (a persistent grid of the
+        workgroups the GPU holds at once, taking the tiles in launch order from a device work queue; the adjoint
+        follows its render).  Images are identical either way.  No reference counterpart."""
         o = {"grid": _lib.DTV_TILE_LAUNCH_GRID, "queue": _lib.DTV_TILE_LAUNCH_QUEUE}.get(str(launch).lower())
         if o is None:
             raise RuntimeError(f"set_tile_launch: unknown launch '{launch}' ('grid' or 'queue').")
